@@ -7,7 +7,7 @@ Steps: (1) the device headers under csrc/kernels/ are embedded as string
 constants (csrc/rx_embedded.inc) so that hiprtc can include them at run time;
 (2) every csrc/*.cpp is compiled (rx_api.cpp as HIP: it holds the AOT copy
 kernel); (3) the GEMM skeletons are compiled once ahead of time with a plain
-epilogue (csrc/kernels/rx_gemm_check.hip) as a device-code build check; (4) link.
+epilogue (csrc/kernels/rx_gemm_check.hip) as a device-code build check; (4) link the library and the compiler's process (rx_rtc_worker.so).
 
     python reactant.jl_amd/build.py --sanitize   # host-only program of the importer / planner under ASan + UBSan
 """
@@ -19,7 +19,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libreactant_mi355x.so")
+WORKER = os.path.join(HERE, "rx_rtc_worker.so")   # a program: named so that it travels wherever the library does
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+ROCM_LIB = "/opt/rocm/lib"
 ARCH = "gfx950"
 PACKED = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON = ["-std=c++17", "-O2", "-fPIC", "-fvisibility=hidden", "-Wall", "-Wno-unused-function",
@@ -65,7 +67,7 @@ def build_library(force=False, verbose=True):
     headers.append(os.path.join(HERE, "..", "include", "reactant_mi355x.h"))
     objs = []
     for f in sorted(os.listdir(CSRC)):
-        if not f.endswith(".cpp") or f == "rx_hostcheck.cpp":   # the sanitizer driver is a program of its own
+        if not f.endswith(".cpp") or f in ("rx_hostcheck.cpp", "rx_rtc_worker.cpp"):   # programs of their own
             continue
         src = os.path.join(CSRC, f)
         obj = os.path.join(OBJ, f[:-4] + ".o")
@@ -75,7 +77,7 @@ def build_library(force=False, verbose=True):
             if f == "rx_api.cpp":
                 cmd += ["-x", "hip", "--offload-arch=" + ARCH] + PACKED
             else:
-                cmd += ["-x", "c++", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include"]   # host code only: no device pass
+                cmd += ["-x", "c++", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", '-DRX_ROCM_LIB="%s"' % ROCM_LIB]   # host code only: no device pass
             _run(cmd + ["-c", src, "-o", obj])
     chk_src = os.path.join(CSRC, "kernels", "rx_gemm_check.hip")
     if os.path.exists(chk_src):
@@ -85,7 +87,12 @@ def build_library(force=False, verbose=True):
                  ["-Wno-unused-command-line-argument", "-c", chk_src, "-o", chk_obj])
     if force or _stale(LIB, objs):
         _run([HIPCC, "-shared", "-fPIC", "--offload-arch=" + ARCH, "-o", LIB] + objs +
-             ["-L/opt/rocm/lib", "-lhiprtc", "-Wl,-rpath,/opt/rocm/lib"])
+             ["-L" + ROCM_LIB, "-lhiprtc", "-ldl", "-Wl,-rpath," + ROCM_LIB])
+    # the compiler's process (csrc/rx_rtc_worker.cpp): its hiprtc comes from ROCM_LIB whatever the environment's library path says
+    src = os.path.join(CSRC, "rx_rtc_worker.cpp")
+    if force or _stale(WORKER, [src] + headers):
+        _run([os.environ.get("CXX", "/opt/rocm/lib/llvm/bin/clang++"), "-std=c++17", "-O2", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", src,
+              "-o", WORKER, "-L" + ROCM_LIB, "-lhiprtc", "-Wl,--disable-new-dtags,-rpath," + ROCM_LIB])
     return LIB
 
 

@@ -2,7 +2,6 @@
 // in include/reactant_mi355x.h.
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
-#include <hip/hiprtc.h>
 
 #include <atomic>
 #include <cstdio>
@@ -16,10 +15,10 @@
 #include <vector>
 
 #include "../../include/reactant_mi355x.h"
-#include "rx_embedded.inc"
 #include "rx_ir.h"
 #include "rx_plan.h"
 #include "rx_gemm.h"
+#include "rx_rtc.h"
 
 #define RX_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -221,39 +220,6 @@ struct RxExecutable {
 };
 
 namespace {
-
-// ---------------------------------------------------------------------------
-// hiprtc
-// ---------------------------------------------------------------------------
-std::string rtc_compile(const std::string& source, const std::string& arch) {
-  hiprtcProgram prog;
-  const char* hdr_src[] = {kRxPreambleSrc, kRxGemmKernelsSrc};
-  const char* hdr_name[] = {"rx_preamble.h", "rx_gemm_kernels.h"};
-  hiprtcResult r = hiprtcCreateProgram(&prog, source.c_str(), "rx_module.hip", 2, hdr_src, hdr_name);
-  if (r != HIPRTC_SUCCESS) throw Error(std::string("hiprtcCreateProgram: ") + hiprtcGetErrorString(r));
-  std::string archopt = "--offload-arch=" + arch;
-  std::vector<const char*> opts = {archopt.c_str(), "-O3", "-std=c++17", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang",
-                                   "-packed-fp32-ops", "-Wno-unused-value"};
-  r = hiprtcCompileProgram(prog, (int)opts.size(), opts.data());
-  size_t ls = 0;
-  hiprtcGetProgramLogSize(prog, &ls);
-  std::string log(ls, '\0');
-  if (ls) hiprtcGetProgramLog(prog, &log[0]);
-  if (r != HIPRTC_SUCCESS) {
-    hiprtcDestroyProgram(&prog);
-    if (getenv("RX_DUMP_FAILED_SOURCE")) {
-      FILE* f = fopen(getenv("RX_DUMP_FAILED_SOURCE"), "w");
-      if (f) { fputs(source.c_str(), f); fclose(f); }
-    }
-    throw Error(std::string("kernel compilation failed (") + hiprtcGetErrorString(r) + "):\n" + log);
-  }
-  size_t cs = 0;
-  hiprtcGetCodeSize(prog, &cs);
-  std::string code(cs, '\0');
-  hiprtcGetCode(prog, &code[0]);
-  hiprtcDestroyProgram(&prog);
-  return code;
-}
 
 rx::PlanOptions plan_options() {
   rx::PlanOptions o;
@@ -883,7 +849,7 @@ RX_EXPORT int RxCompileOffline(const char* text, size_t len, int with_source, ch
   try {
     rx::Graph g = rx::parse_module(text, len);
     rx::Plan p = rx::make_plan(g, plan_options());
-    std::string code = rtc_compile(p.source, "gfx950");
+    std::string code = rx::rtc_compile(p.source, "gfx950");
     if (report) {
       std::string r = p.report() + "code object: " + std::to_string(code.size()) + " bytes\n";
       if (with_source) r += "----- source -----\n" + p.source;
@@ -898,7 +864,7 @@ RX_EXPORT int RxCompileOffline(const char* text, size_t len, int with_source, ch
 }
 
 namespace {
-// Parse, plan and load the module text of an executable: kernels through hiprtc, constants to the device.
+// Parse, plan and load the module text of an executable: kernels compiled (rx_rtc.cpp), constants to the device.
 void load_plan(RxExecutable* ex, rx::PlanOptions opt) {
   RxDevice* d = ex->device;
   if (d->waits_failed) opt.single_pass_scan = false;   // a wait between workgroups has expired on this device before
@@ -915,7 +881,7 @@ void load_plan(RxExecutable* ex, rx::PlanOptions opt) {
   HIP_CHECK(hipSetDevice(d->ordinal));
   ex->fns.clear();
   if (!ex->plan.launches.empty()) {
-    std::string code = rtc_compile(ex->plan.source, d->arch);
+    std::string code = rx::rtc_compile(ex->plan.source, d->arch);
     HIP_CHECK(hipModuleLoadData(&ex->module, code.data()));
     for (auto& L : ex->plan.launches) {
       hipFunction_t f;

@@ -1,0 +1,145 @@
+// Kernel text -> code object, with the compiler of the ROCm that the library was built with.
+//
+// hiprtc and the compiler behind it (comgr) are found by soname, so a process that has already loaded another
+// ROCm's copies (PyTorch ships its own) would compile the kernels with those.  What that costs is not small: the
+// waits of the MFMA skeletons are placed by hand, and a compiler that does not see that a direct-to-LDS load and an
+// LDS read touch different stages adds a full `s_waitcnt vmcnt(0)` in front of the reads (44 instead of 7 in the bf16
+// 256 x 256 kernel) and spills (46 registers in the fp8 one).  MLP of 412 GFLOP in a process with PyTorch's ROCm 7.0
+// libraries: 0.872 ms compiled in the process, 0.33 ms compiled by ROCm 7.2; fp8 8192^3 layer 1.73 against 0.47 ms.
+// Where another copy is loaded, the text goes to a child process (rx_rtc_worker.cpp, a program without any other
+// library) instead; where none is, hiprtc is called here, which saves the child's start (about 0.1 s).
+#include "rx_rtc.h"
+
+#include <fcntl.h>
+#include <limits.h>
+#include <link.h>
+#include <spawn.h>
+#include <sys/mman.h>
+#include <sys/stat.h>
+#include <sys/wait.h>
+#include <unistd.h>
+
+#include <dlfcn.h>
+
+#include <cerrno>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <mutex>
+
+#include "rx_ir.h"
+#include "rx_rtc_hiprtc.h"
+
+#ifndef RX_ROCM_LIB
+#define RX_ROCM_LIB "/opt/rocm/lib"
+#endif
+
+extern char** environ;
+
+namespace rx {
+namespace {
+
+std::string real_dir(const char* path) {
+  char buf[PATH_MAX];
+  const std::string p = realpath(path, buf) ? buf : path;
+  const size_t s = p.rfind('/');
+  return s == std::string::npos ? std::string(".") : p.substr(0, s);
+}
+
+// Has a hiprtc or a comgr from elsewhere than RX_ROCM_LIB been loaded into this process?
+bool foreign_compiler_loaded() {
+  static const std::string own = real_dir(RX_ROCM_LIB "/libhiprtc.so");
+  bool foreign = false;
+  dl_iterate_phdr(
+      [](struct dl_phdr_info* i, size_t, void* f) {
+        const char* base = i->dlpi_name ? strrchr(i->dlpi_name, '/') : nullptr;
+        if (base && (!strncmp(base, "/libhiprtc.so", 13) || !strncmp(base, "/libamd_comgr.so", 16)) && real_dir(i->dlpi_name) != own) *(bool*)f = true;
+        return 0;
+      },
+      &foreign);
+  return foreign;
+}
+
+// The worker lies beside this library.
+const std::string& worker_path() {
+  static const std::string path = [] {
+    Dl_info i;
+    if (!dladdr((const void*)&rtc_compile, &i) || !i.dli_fname) return std::string();
+    return real_dir(i.dli_fname) + "/rx_rtc_worker.so";
+  }();
+  return path;
+}
+
+struct Fd {
+  int fd = -1;
+  ~Fd() { if (fd >= 0) close(fd); }
+};
+
+// Source and result pass through anonymous files, so neither side waits for the other while it writes.
+// True: the worker ran and *code / *error is its answer.  False: it could not be started or did not finish.
+bool worker_compile(const std::string& source, const std::string& arch, std::string* code, std::string* error) {
+  Fd in, out;
+  in.fd = memfd_create("rx_source", MFD_CLOEXEC);
+  out.fd = memfd_create("rx_code", MFD_CLOEXEC);
+  if (in.fd < 0 || out.fd < 0) return false;
+  for (size_t at = 0; at < source.size();) {
+    const ssize_t n = write(in.fd, source.data() + at, source.size() - at);
+    if (n < 0 && errno == EINTR) continue;
+    if (n <= 0) return false;
+    at += (size_t)n;
+  }
+  if (lseek(in.fd, 0, SEEK_SET) < 0) return false;
+  posix_spawn_file_actions_t fa;
+  if (posix_spawn_file_actions_init(&fa) != 0) return false;
+  posix_spawn_file_actions_adddup2(&fa, in.fd, 0);
+  posix_spawn_file_actions_adddup2(&fa, out.fd, 1);
+  posix_spawn_file_actions_addclosefrom_np(&fa, 3);
+  const char* argv[] = {worker_path().c_str(), arch.c_str(), nullptr};
+  pid_t pid = -1;
+  const int rc = posix_spawn(&pid, argv[0], &fa, nullptr, const_cast<char**>(argv), environ);
+  posix_spawn_file_actions_destroy(&fa);
+  if (rc != 0) return false;
+  int status = 0;
+  while (waitpid(pid, &status, 0) < 0)
+    if (errno != EINTR) return false;
+  if (!WIFEXITED(status) || WEXITSTATUS(status) > 1) return false;   // 0: a code object, 1: an error text
+  struct stat st;
+  if (fstat(out.fd, &st) != 0 || st.st_size <= 0) return false;
+  std::string got((size_t)st.st_size, '\0');
+  for (size_t at = 0; at < got.size();) {
+    const ssize_t n = pread(out.fd, &got[at], got.size() - at, (off_t)at);
+    if (n < 0 && errno == EINTR) continue;
+    if (n <= 0) return false;
+    at += (size_t)n;
+  }
+  (WEXITSTATUS(status) == 0 ? *code : *error) = std::move(got);
+  return true;
+}
+
+}  // namespace
+
+std::string rtc_compile(const std::string& source, const std::string& arch) {
+  std::string code, error;
+  bool done = false;
+  if (foreign_compiler_loaded()) {
+    done = worker_compile(source, arch, &code, &error);
+    if (!done) {
+      static std::once_flag told;
+      std::call_once(told, [] {
+        fprintf(stderr, "reactant_mi355x: %s could not be run; kernels are compiled by the hiprtc that this process has loaded, "
+                        "which may make them slower\n", worker_path().c_str());
+      });
+    }
+  }
+  if (!done && hiprtc_compile(source, arch, &code) != 0) { error.swap(code); }
+  if (!error.empty()) {
+    if (getenv("RX_DUMP_FAILED_SOURCE")) {
+      FILE* f = fopen(getenv("RX_DUMP_FAILED_SOURCE"), "w");
+      if (f) { fputs(source.c_str(), f); fclose(f); }
+    }
+    throw Error(error);
+  }
+  return code;
+}
+
+}  // namespace rx

@@ -1,0 +1,28 @@
+// Compiles one kernel text in a process of its own: source on standard input, architecture as the argument, the code
+// object (exit status 0) or the error text (1) on standard output.  Started by rx_rtc.cpp; touches no GPU.
+#include <unistd.h>
+
+#include <cerrno>
+
+#include "rx_rtc_hiprtc.h"
+
+int main(int argc, char** argv) {
+  if (argc != 2) return 2;
+  std::string source, out;
+  char buf[1 << 16];
+  for (;;) {
+    const ssize_t n = read(0, buf, sizeof(buf));
+    if (n < 0 && errno == EINTR) continue;
+    if (n < 0) return 2;
+    if (n == 0) break;
+    source.append(buf, (size_t)n);
+  }
+  const int rc = rx::hiprtc_compile(source, argv[1], &out);
+  for (size_t at = 0; at < out.size();) {
+    const ssize_t n = write(1, out.data() + at, out.size() - at);
+    if (n < 0 && errno == EINTR) continue;
+    if (n <= 0) return 2;
+    at += (size_t)n;
+  }
+  return rc;
+}
