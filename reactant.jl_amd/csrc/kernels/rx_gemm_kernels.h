@@ -387,9 +387,10 @@ RX_DEV int rx_swz_tr(int row, int c) {
 //   TR tiles of 16-bit elements read by the 16 x 16 x 32 MFMA's fragments: the four 16-lane blocks of a transpose read
 //   take rows k, k+8, k+16, k+24, so one 32-lane phase reads rows k..k+3 and k+8..k+11, 32 bytes of each; every
 //   one of those eight rows gets its own 32-byte group of the 256 bytes that the 64 banks hold
+// (CPR & -CPR: rows of a whole number of such blocks of chunks, where CPR is no power of two, swizzle inside the blocks)
 template <int CPR>
 RX_DEV int rx_swz_tr16(int row, int c) {
-  return c ^ ((((row & 3) | (((row >> 3) & 1) << 2)) << 1) & (CPR - 1));
+  return c ^ ((((row & 3) | (((row >> 3) & 1) << 2)) << 1) & ((CPR & -CPR) - 1));
 }
 
 template <class MMA> struct rx_frag_sw;
@@ -780,7 +781,7 @@ RX_DEV void rx_static_for(F&& f) {
 //   its own group of the 256 bytes that the 64 banks hold.
 template <int ESZ, int CPR>
 RX_DEV int rx_swz_tr_s(int row, int c) {
-  if constexpr (ESZ == 1) return c ^ (((row & 7) | (((row >> 4) & 1) << 3)) & (CPR - 1));
+  if constexpr (ESZ == 1) return c ^ (((row & 7) | (((row >> 4) & 1) << 3)) & ((CPR & -CPR) - 1));
   else return rx_swz_tr16<CPR>(row, c);
 }
 
@@ -1480,6 +1481,274 @@ RX_DEV void rx_gemm_body_f64(const double* __restrict__ A, const double* __restr
         const double v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
         if constexpr (BATCHED) epi(v, (int)batch, m, n); else epi(v, m, n);
       }
+    }
+  }
+}
+
+// ===========================================================================
+// Products of few tiles: K in groups inside the workgroup.
+// A product whose tiles do not give every SIMD several wavefronts is bound by latency: a K tile is 16 MFMAs or fewer
+// per wavefront, and nothing runs while its loads and LDS reads are under way.  Here a workgroup is KG groups of WM x
+// WN wavefronts; group g contracts K tiles g, g + KG, ... of the same BM x BN tile of the result through an LDS ring
+// of its own, and the groups' sums are added through LDS at the end (in group order, so the result does not depend on
+// timing): KG times the wavefronts in flight and a chain of K tiles KG times shorter, for one launch and one
+// epilogue.  Skinny products (a few rows against a weight matrix) take 16-row tiles and groups of one wavefront, which
+// stream the weights with KG * (S - 1) K tiles in flight per workgroup and need no barrier until the end.
+// Tiles are 16 x 16 MFMA blocks over K tiles of 128 bytes (as in rx_gemm_body_s), loaded global -> LDS as 16-byte buffer
+// loads.  A load needs dword alignment only and is range-checked dword by dword: rows, columns and K may be any number
+// as long as an operand row is whole dwords.  Positions past the end of an operand read as zero; a [row][k] operand's
+// positions past K inside the matrix are sent past its end (whole 16-byte chunks) or zeroed in registers (the rest of
+// the last one).  SPLIT > 1: workgroup (x, y) contracts K tiles y, y + SPLIT, ... and hands the epilogue (y, m, n).
+// Measured (kernel time, against the skeletons above and the launches they needed): f32 777 x 1001 x 1531 32 us = 74 TFLOP/s
+// (the MFMAs of one 64 x 64 tile alone are 20 us; 9 + 89 + 4 us through padded copies and the register-staged body); bf16
+// 16 x 4096 x 4096 10 (7.4 + 4.1 + 4.1 cut along K), 926 x 1024 x 2048 9 (24.7 + 4.7 + 4.1), 1024 x 2048 x 784 8 (21); e4m3
+// 200 x 6144 x 4096 11.6 (17), 6 x 4096 x 4096 4.2 (130 as a reduction), 3000 x 4096 x 4096 51 (59); f64 4096^3 1.90 ms = 72 of
+// 78.6 TFLOP/s (2.20), 1000^3 44 us (65).
+// ===========================================================================
+struct rx_el_f32 {
+  typedef float elem;
+  static constexpr int NMF = 8;
+  RX_DEV void mma(rx_f32x4v& c, const rx_i32x8& rowop, const rx_i32x8& colop) {
+    struct F8 { float f[8]; };
+    const F8 r = __builtin_bit_cast(F8, rowop), q = __builtin_bit_cast(F8, colop);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(r.f[j], q.f[j], c, 0, 0, 0);
+  }
+};
+struct rx_el_f64 {
+  typedef double elem;
+  static constexpr int NMF = 4;
+  RX_DEV void mma(rx_f64x4& c, const rx_i32x8& rowop, const rx_i32x8& colop) {
+    struct D4 { double d[4]; };
+    const D4 r = __builtin_bit_cast(D4, rowop), q = __builtin_bit_cast(D4, colop);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f64_16x16x4f64(r.d[j], q.d[j], c, 0, 0, 0);
+  }
+};
+template <class EL> struct rx_acc_of { typedef rx_f32x4v type; typedef float scalar; };
+template <> struct rx_acc_of<rx_el_f64> { typedef rx_f64x4 type; typedef double scalar; };
+
+// The [k][o] swizzles: 8- and 16-bit elements as in rx_swz_tr_s; 32-bit: the two 16-lane blocks of one read phase take
+// rows k and k + 4, 64 bytes of each; 64-bit: rows k and k + 2, 128 bytes of each.
+template <int ESZ, int CPR>
+RX_DEV int rx_swz_tr_g(int row, int c) {
+  if constexpr (ESZ == 4) return c ^ ((((row >> 2) & 1) << 2) & ((CPR & -CPR) - 1));
+  else if constexpr (ESZ == 8) return c ^ ((((row >> 1) & 1) << 3) & ((CPR & -CPR) - 1));
+  else return rx_swz_tr_s<ESZ, CPR>(row, c);
+}
+
+// Fragments of 16 rows x 128 bytes of k; which k a lane holds is that of rx_frag_s for every element size (16 bytes at
+// 16 g and 16 bytes at 64 + 16 g, g = lane / 16).  `idx`: the operand row that the lane supplies (lane % 16, except the
+// row operand of the f64 MFMA, see rx_gemm_body_f64).
+template <class EL> struct rx_frag_g {
+  static constexpr int ESZ = sizeof(typename EL::elem);
+  template <int LD> RX_DEV rx_i32x8 kc(const RX_LDS rx_u8* t, int row0, int idx, int lane) {
+    const int r = row0 + idx, c = lane >> 4;
+    struct { rx_i32x4 a, b; } both = {*(const RX_LDS rx_i32x4*)(t + r * LD + rx_swz_kc<LD / 16>(r, c) * 16),
+                                      *(const RX_LDS rx_i32x4*)(t + r * LD + rx_swz_kc<LD / 16>(r, c + 4) * 16)};
+    return __builtin_bit_cast(rx_i32x8, both);
+  }
+  template <int LD> RX_DEV rx_i32x8 tr(const RX_LDS rx_u8* t, int col0, int idx, int lane) {
+    if constexpr (ESZ <= 2) {
+      return rx_frag_s<EL>::template tr<LD>(t, col0, lane);
+    } else {
+      const int colb = (col0 + idx) * ESZ;
+      constexpr int PER = 16 / ESZ;   // elements of one 16-byte half
+      struct { typename EL::elem e[2 * PER]; } all;
+#pragma unroll
+      for (int j = 0; j < 2 * PER; ++j) {
+        const int k = (j / PER) * (64 / ESZ) + PER * (lane >> 4) + j % PER;
+        all.e[j] = *(const RX_LDS typename EL::elem*)(t + k * LD + rx_swz_tr_g<ESZ, LD / 16>(k, colb >> 4) * 16 + (colb & 15));
+      }
+      return __builtin_bit_cast(rx_i32x8, all);
+    }
+  }
+};
+
+// this wavefront's LDS operations are complete and at most N of its vector-memory operations are outstanding
+template <int N>
+RX_DEV void rx_wait_vmcnt_lgkm0() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
+}
+
+template <class EL, int BM, int BN, int WM, int WN, int KG, int S, bool A_KC, bool B_KC, int M, int N, int K, int RB, int CB, bool BATCHED, class Epi, int SPLIT = 1>
+RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typename EL::elem* __restrict__ B, const Epi& epi) {
+  typedef typename rx_acc_of<EL>::type acc_t;
+  typedef typename rx_acc_of<EL>::scalar acc_s;
+  constexpr int ESZ = sizeof(typename EL::elem);
+  constexpr int BKB = 128, BK = BKB / ESZ;
+  constexpr int NW = WM * WN, NA = BM / WM / 16, NB = BN / WN / 16;
+  constexpr int A_COLS = A_KC ? BKB : BM * ESZ, B_COLS = B_KC ? BKB : BN * ESZ;   // bytes of an LDS row
+  constexpr int STAGE = (BM + BN) * BKB;
+  constexpr int NLA = BM / 8 / NW, NLB = BN / 8 / NW, NL = NLA + NLB;             // 1 KB loads per wavefront and K tile
+  static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0 && (BM / 8) % NW == 0 && (BN / 8) % NW == 0, "tile shape");
+  static_assert((long long)M * K * ESZ < (1ll << 31) && (long long)N * K * ESZ < (1ll << 31), "32-bit operand offsets");
+  static_assert((A_KC ? K : M) * ESZ % 4 == 0 && (B_KC ? K : N) * ESZ % 4 == 0, "operand rows are whole dwords");
+  static_assert(!(BATCHED && SPLIT > 1), "slices of K take the place of the batch index");
+  static_assert((A_KC || (long long)(K + 2 * BK * KG * SPLIT) * M * ESZ < (1ll << 32)) && (B_KC || (long long)(K + 2 * BK * KG * SPLIT) * N * ESZ < (1ll << 32)),
+                "offsets of the last groups' K tiles");
+  constexpr unsigned KBYTES = (unsigned)K * ESZ, A_LDB = (A_KC ? K : M) * ESZ, B_LDB = (B_KC ? K : N) * ESZ;
+  constexpr int KT = (K + BK - 1) / BK, STEP = KG * SPLIT, KTG = (KT + STEP - 1) / STEP;   // K tiles, and per group
+  constexpr int SD = KTG < S ? KTG : S;
+  constexpr bool SEL = KBYTES % (BKB * STEP) != 0;   // some group's last K tile reaches past K
+  extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave / NW, w = wave % NW, wm = w / WN, wn = w % WN;
+  RX_LDS rx_u8* const lds = (RX_LDS rx_u8*)rx_smem + grp * (SD * STAGE);
+  constexpr int GM = (M + BM - 1) / BM, GN = (N + BN - 1) / BN;
+  int bm, bn;
+  if (!rx_gemm_tile<GM, GN, RB, CB>(blockIdx.x, &bm, &bn)) return;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const long long batch = BATCHED ? blockIdx.y : 0;
+  const unsigned first = grp * SPLIT + (SPLIT > 1 ? blockIdx.y : 0);   // this group's first K tile
+
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)(A + batch * (long long)M * K), 0, (unsigned)M * KBYTES, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)(B + batch * (long long)N * K), 0, (unsigned)N * KBYTES, 0x00020000);
+  // per-thread byte offset of every load (the K tile's included), and for [row][k] operands the byte of k it starts at
+  unsigned off[NL], kpos[NL];
+#pragma unroll
+  for (int i = 0; i < NL; ++i) {
+    const bool isa = i < NLA;
+    const int s = ((isa ? i : i - NLA) * NW + w) * 64 + lane;      // 16-byte slot of the LDS tile
+    const int cpr = (isa ? A_COLS : B_COLS) / 16, row = s / cpr, pos = s % cpr;
+    const bool kc = isa ? A_KC : B_KC;
+    const unsigned ldb = isa ? A_LDB : B_LDB;
+    const int o0 = isa ? m0 : n0;
+    if (kc) {
+      kpos[i] = first * BKB + rx_swz_kc<8>(row, pos) * 16;
+      off[i] = (unsigned)(o0 + row) * ldb + kpos[i];
+    } else {
+      const int c = isa ? rx_swz_tr_g<ESZ, A_COLS / 16>(row, pos) : rx_swz_tr_g<ESZ, B_COLS / 16>(row, pos);
+      kpos[i] = 0;
+      off[i] = (first * BK + (unsigned)row) * ldb + o0 * ESZ + c * 16;
+    }
+  }
+  auto issue = [&](int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) {
+      const bool isa = i < NLA, kc = isa ? A_KC : B_KC;
+      unsigned o = off[i];
+      if (SEL && kc) {
+        o = kpos[i] < KBYTES ? o : 0xfffffff0u;
+        kpos[i] += BKB * STEP;
+      }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(isa ? ra : rb, (RX_LDS void*)(lds + st * STAGE + (isa ? i * NW + w : BM / 8 + (i - NLA) * NW + w) * 1024), 16, o, 0, 0, 0);
+      off[i] += kc ? BKB * STEP : BK * STEP * (isa ? A_LDB : B_LDB);
+    }
+  };
+
+  acc_t acc[NA][NB];
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  const int idx_a = lane & 15, idx_b = ESZ == 8 ? 4 * (lane & 3) + ((lane & 15) >> 2) : idx_a;
+  // dwords of a [row][k] fragment at or past K: only where K is not a whole number of 16-byte chunks
+  auto cut = [&](rx_i32x8& f, unsigned kt) {
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      const unsigned kb = kt * BKB + (d / 4) * 64 + 16 * (lane >> 4) + 4 * (d % 4);
+      f[d] = kb < KBYTES ? f[d] : 0;
+    }
+  };
+  auto compute = [&](int st, unsigned kt) __attribute__((always_inline)) {
+    const RX_LDS rx_u8* sa = lds + st * STAGE;
+    const RX_LDS rx_u8* sb = sa + BM * BKB;
+    rx_i32x8 fb[NB], fa[NA];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      const int o = wn * (BN / WN) + 16 * j;
+      if constexpr (B_KC) fb[j] = rx_frag_g<EL>::template kc<B_COLS>(sb, o, idx_b, lane);
+      else fb[j] = rx_frag_g<EL>::template tr<B_COLS>(sb, o, idx_b, lane);
+    }
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+      const int o = wm * (BM / WM) + 16 * i;
+      if constexpr (A_KC) fa[i] = rx_frag_g<EL>::template kc<A_COLS>(sa, o, idx_a, lane);
+      else fa[i] = rx_frag_g<EL>::template tr<A_COLS>(sa, o, idx_a, lane);
+    }
+    if constexpr (KBYTES % 16 != 0 && (A_KC || B_KC)) {
+      if (kt == KT - 1) {
+        if constexpr (B_KC) {
+#pragma unroll
+          for (int j = 0; j < NB; ++j) cut(fb[j], kt);
+        }
+        if constexpr (A_KC) {
+#pragma unroll
+          for (int i = 0; i < NA; ++i) cut(fa[i], kt);
+        }
+      }
+    }
+    // the B fragment is the row operand: a lane ends with four consecutive n of one m
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) EL::mma(acc[i][j], fb[j], fa[i]);
+  };
+  // Tile t of the group lies in stage t % SD.  By the time a wavefront passes the barrier of tile t, every wavefront of
+  // its group has read tile t - 1, whose stage then takes tile t + SD - 1.  A group of one wavefront has no one to wait for.
+  auto publish = [&]() {
+    asm volatile("" ::: "memory");
+    if constexpr (NW > 1) __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  rx_static_for<0, (SD > 1 ? SD - 1 : 1)>([&](auto I) { issue(decltype(I)::value); });
+  constexpr int MAIN = SD > 1 ? KTG - (SD - 1) : 0;   // tiles with a successor to request
+  int st = 0;
+  for (int t = 0; t < MAIN; ++t) {
+    rx_wait_vmcnt_lgkm0<(SD > 1 ? SD - 2 : 0) * NL>();
+    publish();
+    issue(st == 0 ? SD - 1 : st - 1);
+    compute(st, first + (unsigned)t * STEP);
+    st = st + 1 == SD ? 0 : st + 1;
+  }
+  rx_static_for<MAIN, KTG>([&](auto T) {
+    constexpr int t = decltype(T)::value;
+    rx_wait_vmcnt_lgkm0<(KTG - 1 - t) * NL>();
+    publish();
+    compute(t % SD, first + (unsigned)t * STEP);
+  });
+
+  // result vectors as wide as the rows allow (an odd N: one element at a time)
+  constexpr int NV = N % 4 == 0 ? 4 : (N % 2 == 0 ? 2 : 1);
+  auto finish = [&](const acc_t& c, int unit) {
+    const int uw = unit / (NA * NB), b = unit % (NA * NB);
+    const int m = m0 + (uw / WN) * (BM / WM) + 16 * (b / NB) + (lane & 15);
+    const int nb = n0 + (uw % WN) * (BN / WN) + 16 * (b % NB) + 4 * (lane >> 4);
+#pragma unroll
+    for (int q = 0; q < 4; q += NV) {
+      const int n = nb + q;
+      if (m < M && n < N) {
+        acc_s v[NV];
+#pragma unroll
+        for (int l = 0; l < NV; ++l) v[l] = c[q + l];
+        if constexpr (BATCHED) epi(v, (int)batch, m, n);
+        else if constexpr (SPLIT > 1) epi(v, (int)blockIdx.y, m, n);
+        else epi(v, m, n);
+      }
+    }
+  };
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) finish(acc[i][j], w * (NA * NB) + i * NB + j);
+  } else {
+    // every group leaves its 16 x 16 blocks in LDS; the wavefronts of the workgroup share the blocks out, add the
+    // groups' sums in order and run the epilogue
+    rx_wait_vmcnt_lgkm0<0>();
+    __syncthreads();
+    RX_LDS acc_t* part = (RX_LDS acc_t*)rx_smem;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) part[((w * (NA * NB) + i * NB + j) * KG + grp) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    for (int u = wave; u < NW * NA * NB; u += KG * NW) {
+      acc_t c = part[(u * KG) * 64 + lane];
+#pragma unroll
+      for (int g = 1; g < KG; ++g) c += part[(u * KG + g) * 64 + lane];
+      finish(c, u);
     }
   }
 }

@@ -1,6 +1,7 @@
 #include "rx_gemm.h"
 
 #include <cstdlib>
+#include <cstring>
 #include <algorithm>
 #include <sstream>
 #include <stdexcept>
@@ -50,9 +51,140 @@ static GemmChoice choose_gemm_f64(int64_t batch, int64_t M, int64_t N, int64_t K
   return c;
 }
 
-GemmChoice choose_gemm(DT a, DT b, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, bool staged_only, int split) {
+// ---------------------------------------------------------------------------
+// rx_gemm_body_g (K in groups inside the workgroup): tile, wavefronts, groups and stages
+// ---------------------------------------------------------------------------
+struct GroupTile { int BM, BN, WM, WN, KG, S; };
+
+static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t, int64_t* lds) {
+  const int es = info(dt).size;
+  const int64_t bk = 128 / es, KT = (K + bk - 1) / bk, step = (int64_t)t.KG * split, KTG = (KT + step - 1) / step;
+  const int NW = t.WM * t.WN;
+  if (t.BM % (16 * t.WM) || t.BN % (16 * t.WN) || t.BM / 8 % NW || t.BN / 8 % NW || NW * t.KG > 16) return false;
+  if ((a_kc ? K : M) * es % 4 || (b_kc ? K : N) * es % 4) return false;   // operand rows are whole dwords
+  const int64_t lim = (int64_t)1 << 31;                                    // 32-bit operand offsets, the last groups' K tiles included
+  if (M * K * es >= lim || N * K * es >= lim) return false;
+  if ((!a_kc && (K + 2 * bk * step) * M * es >= 2 * lim) || (!b_kc && (K + 2 * bk * step) * N * es >= 2 * lim)) return false;
+  if (batch > 65535) return false;                                         // blockIdx.y
+  // accumulators and fragments of a wavefront within its share of the register file
+  const int na = t.BM / t.WM / 16, nb = t.BN / t.WN / 16;
+  if (na * nb * (es == 8 ? 8 : 4) + 8 * (na + nb) + 48 > 512 / std::max(1, (NW * t.KG + 3) / 4)) return false;
+  const int64_t nl = (t.BM + t.BN) / 8 / NW, sd = std::min<int64_t>(t.S, KTG);
+  if (nl * (sd - 1) > 63) return false;                                    // outstanding loads that a wait can count
+  const int64_t ring = (int64_t)t.KG * sd * (t.BM + t.BN) * 128, sums = t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * (es == 8 ? 8 : 4) : 0;
+  *lds = std::max(ring, sums);
+  return *lds <= 160 * 1024;
+}
+
+// Time of a launch in microseconds, for comparing tiles: rounds of workgroups over the 256 compute units; per K tile
+// the largest of the MFMAs, the operand loads and the LDS fragment reads of the workgroups that share a compute unit
+// (with little to overlap them where few wavefronts share a SIMD), or the latency of the loads over the stages in flight;
+// the prologue, the epilogue and the groups' sums; bounded below by the operands' traffic from L2 and from memory.
+// Constants fitted to 1600 timings of 54 shapes (f32, f64, bf16, e4m3; 1 to 8192 rows; all operand orders): the tile
+// with the smallest estimate takes 1.03 times the time of the fastest one (geometric mean).
+static double group_estimate(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t, int64_t lds) {
+  const int es = info(dt).size, NW = t.WM * t.WN, waves = NW * t.KG;
+  const int64_t bk = 128 / es, KT = (K + bk - 1) / bk, step_k = (int64_t)t.KG * split;
+  const double KTG = (double)((KT + step_k - 1) / step_k), sd = std::min<double>(t.S, KTG);
+  const int64_t T = ((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * batch * split;
+  const int64_t R = std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(160 * 1024 / lds, 16 / waves), 8));
+  const int64_t per = (T + 255) / 256, cc = std::min(per, R);          // workgroups of a compute unit in all, and at a time
+  const double rounds = per <= cc ? 1.0 : (double)(per / cc) + (double)(per % cc) / (double)cc;
+  const double w = (double)waves * (double)cc / 4.0;                   // wavefronts per SIMD
+  // flops per clock and compute unit, times what these loops sustain of them
+  const double fl = es == 8 ? 128 * 0.93 : es == 4 ? 256.0 : es == 2 ? 4096 * 0.68 : 8192 * 0.64;
+  const double mf = (double)t.BM * t.BN * (double)bk * t.KG * 2.0 / fl * (double)cc / std::min(1.0, w);
+  const double ld = (double)t.KG * (t.BM + t.BN) * 128.0 / 102.0 * (double)cc;
+  const double rd = (double)waves * ((double)t.BM / t.WM + (double)t.BN / t.WN) * 128.0 / 179.0 * (double)cc;
+  const double big = std::max(mf, std::max(ld, rd));
+  const double step = std::max(1625.0 / std::max(sd - 1.0, 0.5), (big + 0.1 * (mf + ld + rd - big)) * (1.0 + 0.33 / std::max(w, 1.0)) + 170.0);
+  double cycles = 4100.0 + rounds * KTG * step + (double)per * (double)t.BM * t.BN * (0.36 + (t.KG > 1 ? 0.15 * t.KG : 0.0)) + (rounds - 1.0) * 5600.0;
+  cycles += 0.02 * cycles;
+  cycles = std::max(cycles, 4100.0 + (double)(T / split) * (t.BM + t.BN) * (double)K * es / 6000.0);
+  const double bytes = (double)batch * (double)(M + N) * (double)K * es;
+  cycles = std::max(cycles, 4100.0 + bytes / 1700.0);
+  // A compute unit has some 250 lines of 128 bytes under way at a time, whole or not: a line, or the part of one that a
+  // narrow tile reads of a [k][n] row, costs it 7.5 cycles from memory, 4.5 from the memory-side cache, 2 from L2
+  // (16 x 4096 x 25088 bf16: tiles of 16, 32 and 64 columns 84, 98 and 108 us as [k][n], 40, 52 and 77 as [n][k])
+  const double line = bytes < 16e6 ? 2.0 : bytes < 128e6 ? 4.5 : 7.5;
+  auto lines = [&](bool kc, int64_t rows, int tile) {
+    const double tiles = (double)((rows + tile - 1) / tile);
+    return kc ? (double)rows * (double)K * es / 128.0 : tiles * (double)K * (double)((tile * es + 127) / 128);
+  };
+  cycles = std::max(cycles, 4100.0 + (double)batch * (lines(a_kc, M, t.BM) + lines(b_kc, N, t.BN)) * line / (double)std::min<int64_t>(T, 256));
+  return cycles / 2400.0;
+}
+
+static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t) {
   GemmChoice c;
-  if (a != b) return c;
+  int64_t lds = 0;
+  if (!group_fits(dt, batch, M, N, K, a_kc, b_kc, split, t, &lds)) return c;
+  const int64_t gm = (M + t.BM - 1) / t.BM, gn = (N + t.BN - 1) / t.BN;
+  int rb = 4, cb = 8;
+  if (gm * gn < 8) rb = cb = 0;
+  // up to two rounds of tiles over the chip: every XCD takes a band of adjacent columns (rows) of tiles, so that narrow
+  // tiles that share lines of an operand share an L2
+  else if (gm * gn <= 512 && gn >= gm) { rb = (int)gm; cb = (int)((gn + 7) / 8); }
+  else if (gm * gn <= 512) { rb = (int)((gm + 7) / 8); cb = (int)gn; }
+  else if (gm < rb) { cb = (int)(rb * cb / gm); rb = (int)gm; }
+  else if (gn < cb) { rb = (int)(rb * cb / gn); cb = (int)gn; }
+  if (const char* e = getenv("RX_GEMM_BLOCK")) { int v[2]; if (sscanf(e, "%d,%d", &v[0], &v[1]) == 2) { rb = v[0]; cb = v[1]; } }
+  c.lds_bytes = (unsigned)lds;
+  c.block = (unsigned)(t.WM * t.WN * t.KG * 64);
+  c.grid[0] = (unsigned)gemm_grid(gm, gn, rb, cb);
+  c.grid[1] = (unsigned)(split > 1 ? split : batch);
+  c.split = split;
+  c.est_us = group_estimate(dt, batch, M, N, K, a_kc, b_kc, split, t, lds);
+  const std::string el = dt == DT::F64 ? "rx_el_f64" : dt == DT::F32 ? "rx_el_f32" : dt == DT::BF16 ? "rx_el_bf16" : dt == DT::F16 ? "rx_el_f16" : "rx_el_f8";
+  std::ostringstream o;
+  o << el << ", " << t.BM << ", " << t.BN << ", " << t.WM << ", " << t.WN << ", " << t.KG << ", " << t.S << ", " << (a_kc ? "true" : "false") << ", "
+    << (b_kc ? "true" : "false") << ", " << M << ", " << N << ", " << K << ", " << rb << ", " << cb;
+  c.targs = o.str();
+  c.skeleton = "rx_gemm_body_g";
+  c.kind = dt == DT::F64 ? "gemm_f64" : dt == DT::F32 ? "gemm_f32" : dt == DT::BF16 ? "gemm_bf16" : dt == DT::F16 ? "gemm_f16" : "gemm_f8";
+  c.stype_a = el + "::elem";
+  c.ok = true;
+  return c;
+}
+
+// The tile with the smallest estimate.  RX_GEMM_G=BM,BN,WM,WN,KG,S asks for one (products it does not fit keep the
+// estimate's), RX_GEMM_G=0 leaves this skeleton out.
+static GemmChoice choose_group(DT dt, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split) {
+  GemmChoice best;
+  const bool types = (dt == DT::F64 && out == DT::F64) || (dt == DT::F32 && out == DT::F32) || ((dt == DT::BF16 || dt == DT::F16) && (out == dt || out == DT::F32)) ||
+                     (dt == DT::F8E4M3FN && (out == DT::F32 || out == DT::BF16 || out == DT::F16));
+  if (!types || M < 1 || N < 1 || batch < 1) return best;
+  // a few thousand multiplications: the scalar loop is as good
+  if (K < 64 || (double)batch * (double)M * (double)N * (double)K < (double)(1 << 19)) return best;
+  if (const char* e = getenv("RX_GEMM_G")) {
+    GroupTile t;
+    if (!strcmp(e, "0")) return best;
+    if (sscanf(e, "%d,%d,%d,%d,%d,%d", &t.BM, &t.BN, &t.WM, &t.WN, &t.KG, &t.S) != 6 || t.BM < 16 || t.BN < 16 || t.WM < 1 || t.WN < 1 || t.KG < 1 || t.S < 1)
+      throw std::runtime_error("RX_GEMM_G wants BM,BN,WM,WN,KG,S");
+    best = group_gemm(dt, batch, M, N, K, a_kc, b_kc, split, t);
+    if (best.ok) return best;
+  }
+  static const int tiles[][4] = {{16, 16, 1, 1}, {16, 32, 1, 1}, {32, 16, 1, 1}, {16, 64, 1, 2}, {64, 16, 2, 1}, {32, 32, 1, 1}, {32, 64, 1, 2}, {64, 32, 2, 1},
+                                 {32, 64, 2, 2}, {64, 32, 2, 2}, {64, 64, 2, 2}, {64, 96, 2, 2}, {96, 64, 2, 2}, {96, 96, 2, 2}, {64, 128, 2, 2}, {128, 64, 2, 2},
+                                 {64, 128, 2, 4}, {128, 64, 4, 2}, {96, 128, 2, 2}, {128, 96, 2, 2}, {128, 128, 2, 2}, {128, 128, 2, 4}, {128, 128, 4, 2},
+                                 {160, 128, 2, 2}, {128, 160, 2, 2}, {192, 128, 4, 2}, {128, 192, 2, 4}, {256, 128, 4, 2}, {128, 256, 2, 4}};
+  GroupTile pick{};
+  double cost = 0;
+  for (auto& q : tiles)
+    for (int kg = 1; kg <= 16; kg *= 2)
+      for (int s = 2; s <= 5; ++s) {
+        const GroupTile t{q[0], q[1], q[2], q[3], kg, s};
+        int64_t lds = 0;
+        if (!group_fits(dt, batch, M, N, K, a_kc, b_kc, split, t, &lds)) continue;
+        const double c = group_estimate(dt, batch, M, N, K, a_kc, b_kc, split, t, lds);
+        if (cost == 0 || c < cost) { cost = c; pick = t; }
+      }
+  return cost > 0 ? group_gemm(dt, batch, M, N, K, a_kc, b_kc, split, pick) : best;
+}
+
+// The skeletons for tiles that fill the chip (streaming and ping-pong bodies, ring skeleton) and the register-staged one.
+static GemmChoice choose_tiled(DT a, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, bool staged_only, int split) {
+  GemmChoice c;
   if (split > 1 && (staged_only || batch != 1 || a == DT::F64)) return c;
   if (a == DT::F64 && out == DT::F64) return staged_only ? c : choose_gemm_f64(batch, M, N, K, a_kc, b_kc);
   std::string mma;
@@ -220,6 +352,39 @@ GemmChoice choose_gemm(DT a, DT b, DT out, int64_t batch, int64_t M, int64_t N, 
   c.stype_a = mma + "::elem";
   c.ok = true;
   return c;
+}
+
+GemmChoice choose_gemm(DT a, DT b, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, bool staged_only, int split, bool groups) {
+  if (a != b) return GemmChoice();
+  // a request for one of the other skeletons or for their tiles
+  bool asked = false;
+  for (const char* e : {"RX_GEMM_TILE", "RX_GEMM_BK", "RX_GEMM_STAGES", "RX_GEMM_DIRECT", "RX_GEMM_STREAM", "RX_GEMM_MFMA32", "RX_GEMM_TILE_F64"}) asked = asked || getenv(e);
+  if (staged_only || !groups || asked) return choose_tiled(a, out, batch, M, N, K, a_kc, b_kc, staged_only, split);
+  GemmChoice g = choose_group(a, out, batch, M, N, K, a_kc, b_kc, split);
+  if (!g.ok || split > 1) return g.ok ? g : choose_tiled(a, out, batch, M, N, K, a_kc, b_kc, staged_only, split);
+  const char* req = getenv("RX_GEMM_G");
+  if (req && strcmp(req, "0") && g.ok) return g;
+  GemmChoice c = choose_tiled(a, out, batch, M, N, K, a_kc, b_kc, staged_only, split);
+  if (!c.ok) return g;
+  auto rounds = [&](int64_t bm, int64_t bn) { return (double)((((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch + 255) / 256); };
+  // Eight-wavefront tiles that fill the chip.  The streaming and ping-pong bodies keep the MFMA pipes busier than this
+  // skeleton's loop where every round of tiles is full (bf16 4000 x 4096 x 1024 33 against 40 us, e4m3 8192 x 2048 x 5120 72
+  // against 98), but a last round of few tiles costs them a whole one (bf16 2443 x 4096 x 4096, 320 tiles: 124 against 102
+  // us).  Estimates: 1.33 us per K tile of 128 bytes of a 256 x 256 tile, 0.77 of a 256 x 128 tile, 10.5 and 9.5 us around them.
+  // Contractions of fewer than 16 K tiles stay with them: their rounds overlap.
+  if (c.skeleton == "rx_gemm_body_pp" || c.skeleton == "rx_gemm_body_s") {
+    const double kt = (double)(K * info(a).size / 128);
+    const bool sq = c.targs.find(", 256, 256, ") != std::string::npos;
+    const double us = rounds(256, sq ? 256 : 128) * (sq ? kt * 1.33 + 10.5 : kt * 0.77 + 9.5) + 3.0;
+    return kt >= 16 && g.est_us < us ? g : c;
+  }
+  // f32 on 256 x 256 tiles of the ring skeleton: 0.9 of the MFMA peak on a grid of whole rounds (4096^3 964 against 973 us),
+  // less on others (8192 x 4096 x 1024 538 against 522, 2048^3 157 against 146)
+  if (c.skeleton == "rx_gemm_body_dl" && a == DT::F32 && c.targs.find(", 256, 256, ") != std::string::npos)
+    return rounds(256, 256) * ((double)K * 0.2335 + 8.0) < g.est_us ? c : g;
+  // f32, an operand of at most 64 rows against 512 tiles and more (the features of a convolution and its window matrix)
+  if (c.skeleton == "rx_gemm_body_dl" && a == DT::F32 && (M <= 64 || N <= 64) && ((M + 63) / 64) * ((N + 63) / 64) >= 1024) return c;
+  return g;
 }
 
 std::string gemm_instance(const GemmChoice& c, const std::string& kbase, const std::string& epi_params, const std::string& epi_ctor, bool batched,

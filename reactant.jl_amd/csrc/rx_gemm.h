@@ -19,6 +19,7 @@ struct GemmChoice {
   int depth = 0;            // rx_gemm_body_s: blocks of the streamed operand read ahead (0: the skeleton's default)
   int stream_stages = 0;    // rx_gemm_body_s: LDS stages per operand (0: not that skeleton)
   int bk = 0;               // rx_gemm_body_dl: elements of K per tile
+  double est_us = 0;        // rx_gemm_body_g: estimated time
 };
 
 // Workgroups to launch for a gm x gn grid of tiles: the kernels walk the tiles in blocks of 4 x 8,
@@ -31,9 +32,10 @@ inline int64_t gemm_grid(int64_t gm, int64_t gn, int rb = 4, int cb = 8) {
 }
 
 // Returns ok=false when no skeleton covers the case (the caller then writes a scalar loop).
-// `staged_only`: an operand is a functor, which only the register-staged skeleton can read.
+// `staged_only`: an operand is a functor, which only the register-staged skeleton can read.  `groups`: rx_gemm_body_g may
+// be chosen (not where the caller adds row shifts, which it does not take).
 GemmChoice choose_gemm(DT a, DT b, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_k_contig, bool b_k_contig,
-                       bool staged_only = false, int split = 1);
+                       bool staged_only = false, int split = 1, bool groups = true);
 
 // Text of the `extern "C"` kernel <kbase>_gemm that runs the skeleton with epilogue type <kbase>_epi.
 // `epi_params` is the tail of the parameter list (epilogue operands and out0), `epi_ctor` builds `epi`.

@@ -2009,7 +2009,7 @@ struct Builder {
       // the same test), which this form is not (512 -> 512 features on four 14 x 14 images: 0.026 against 0.061 ms)
       const bool sliced = ((B * HO * WO + 63) / 64) * ((O + 63) / 64) < 256 && KK >= 1024 && !(getenv("RX_SPLIT_K") && atoi(getenv("RX_SPLIT_K")) == 0);
       if (HO >= 1 && WO >= 1 && !sliced && MP * CP * 2 < ((int64_t)1 << 31) && O * KK * 2 < ((int64_t)1 << 31) && KH * KW <= 1024)
-        gc = choose_gemm(xct.dt, xct.dt, xct.dt, 1, MP, O, KK, true, true);
+        gc = choose_gemm(xct.dt, xct.dt, xct.dt, 1, MP, O, KK, true, true, false, 1, false);
       if (gc.ok && (gc.skeleton == "rx_gemm_body_pp" || gc.skeleton == "rx_gemm_body_s" || (gc.skeleton == "rx_gemm_body_dl" && gc.bk * 2 == 128 && gc.split == 1))) {
         std::vector<int64_t> want(r);
         want[cd[2].d0] = B; want[cd[2].d1] = O; want[cd[2].sp[0]] = HO; want[cd[2].sp[1]] = WO;

@@ -998,6 +998,10 @@ struct Planner {
   void split_dots() {
     if (!opt.mfma || !opt.split_k) return;
     std::map<int, int> splits;
+    std::vector<char> followed(g.nodes.size(), 0);   // read by an elementwise op
+    for (const Node& n : g.nodes)
+      for (int i : n.in)
+        if (n.k == OpK::Unary || n.k == OpK::Binary || n.k == OpK::Compare || n.k == OpK::Select || n.k == OpK::Clamp || n.k == OpK::Convert || n.k == OpK::Gelu) followed[i] = 1;
     for (const Node& d : g.nodes) {
       if (d.k != OpK::DotGeneral || d.ty.rank() != 2 || !d.a0.empty()) continue;
       DotForm f = dot_form(d);
@@ -1007,11 +1011,28 @@ struct Planner {
       if (!choose_gemm(a, b, d.ty.dt, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig).ok) continue;
       const int64_t tiles = ((f.M + 63) / 64) * ((f.N + 63) / 64);
       if (tiles >= 256 || f.K < 1024) continue;
-      // enough slices for two workgroups per compute unit, each slice at least 512 long
+      const GemmChoice whole = choose_gemm(a, b, d.ty.dt, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig);
+      // the slices' sums cost a launch and a pass over them, and a result that elementwise ops consume loses its epilogue:
+      // another launch (4 us each between dependent launches)
+      const double extra = followed[d.id] ? 8.0 : 4.0;
       int S = 1;
-      while (S < 256 && tiles * S < 512 && f.K / (2 * S) >= 512) S *= 2;
+      double best = whole.skeleton == "rx_gemm_body_g" ? whole.est_us : 1e30;
+      // Cut whatever the estimates say: products that nothing elementwise follows, of at most 128 whole tiles and K >= 2048 (f32 256 x 256 x
+      // 2048 11.6 against 7.9 us uncut, bf16 128 x 128 x 16384 15.7 against 23.7); and 17 to 32 rows of 16-bit elements against
+      // [k][n] weights with K >= 4096 (32 x 4096 x 25088 57 against 104 us, 32 x 4096 x 4096 15.5 against 11.2).
+      const bool few = !followed[d.id] && tiles <= 128 && f.M % 64 == 0 && f.N % 64 == 0 && f.K >= 2048;
+      const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= 4096;
+      if (few || dense) {   // two workgroups per compute unit, slices of at least 512
+        while (S < 256 && tiles * S < 512 && f.K / (2 * S) >= 512) S *= 2;
+      } else {
+        for (int q = 2; q <= 256 && f.K / q >= 256; q *= 2) {
+          GemmChoice c = choose_gemm(a, b, DT::F32, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig, false, q);
+          if (!c.ok || c.split != q) continue;
+          const double us = c.est_us + extra + (double)q * (double)f.M * (double)f.N * 8.0 / 4e6;
+          if (us < best) { best = us; S = q; }
+        }
+      }
       for (; S > 1; S /= 2) {
-        if (f.K % S) continue;
         GemmChoice c = choose_gemm(a, b, DT::F32, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig, false, S);
         if (c.ok && c.split == S) break;
       }
@@ -1086,6 +1107,19 @@ struct Planner {
     if (kprod < 1 || d.ty.numel() < 1) return r;
     // short contractions: one thread per output element walks them as fast
     if (kprod < 128) return r;
+    // A matrix of 2^18 elements and more against one to eight rows, in matrix form: the MFMA skeleton with K in groups
+    // (16-row tiles, one launch with the epilogue; 4-5 us for 12 MB of f32 or 8 MB of bf16 weights) against the reduction
+    // and its combine and epilogue launches (13-22 us; 142 us for e4m3 6 x 4096 x 4096, whose reduction converts every
+    // weight once per row).  One and four rows of 4-byte and wider elements, which the reduction's vectors fit, stay with it
+    // from 2^24 elements on, where it streams the matrix faster (4 x 4096 x 25088 f32 78 against 102 us), and four rows
+    // below 2^21 elements.
+    const int64_t big = std::max(lt.numel(), rt.numel()), rows = r.big_is_lhs ? nfree : mfree;
+    const bool wide = info(lt.dt).size >= 4;
+    const bool streams = wide && (rows == 1 || rows == 4) && (big >= (1 << 24) || (rows == 4 && big < (1 << 21)));
+    if (opt.mfma && is_float(lt.dt) && lt.dt != DT::F8E5M2 && big >= (1 << 18) && !streams) {
+      const DotForm f = dot_form(d);
+      if (f.ok && d.ty.rank() == 2 && choose_gemm(lt.dt, rt.dt, d.ty.dt, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig).skeleton == "rx_gemm_body_g") return r;
+    }
     r.ok = true;
     return r;
   }
@@ -3621,7 +3655,7 @@ struct Planner {
       // first operand carry the tap's row shift (rx_tap_shift)
       const int64_t xrows = xt.numel() / xt.dims.back(), xcols = xt.dims.back();   // the first operand as a matrix (its leading dimensions are the rows)
       if (rn.ty.dims != cn.ty.dims || cn.ty.dims[0] * cn.a3[3] * cn.a3[4] != xrows) throw Error("internal: shifted product with a result of another shape");
-      const GemmChoice gc = choose_gemm(xt.dt, wt.dt, cn.ty.dt, 1, xrows, wt.dims[0], wt.dims[1], true, true);
+      const GemmChoice gc = choose_gemm(xt.dt, wt.dt, cn.ty.dt, 1, xrows, wt.dims[0], wt.dims[1], true, true, false, 1, false);
       const bool dl = gc.skeleton == "rx_gemm_body_dl";
       if (!gc.ok || (gc.skeleton != "rx_gemm_body_pp" && gc.skeleton != "rx_gemm_body_s" && !(dl && gc.bk * (int)info(xt.dt).size == 128 && gc.split == 1)))
         throw Error("internal: shifted product without a skeleton that loads tiles straight into LDS");
