@@ -85,3 +85,12 @@ RX_CHECK_G(rx_check_g_f64_nn, rx_el_f64, double, 32, 32, 2, 1, 2, 2, true, false
 RX_CHECK_G(rx_check_g_bf16_nn, rx_el_bf16, float, 64, 64, 2, 2, 1, 3, true, false, 512, 512, 784)
 RX_CHECK_G(rx_check_g_f16_tt, rx_el_f16, float, 32, 64, 1, 2, 4, 2, false, true, 64, 64, 128)
 RX_CHECK_G(rx_check_g_f8_nt, rx_el_f8, float, 16, 16, 1, 1, 8, 3, true, true, 16, 512, 4096)
+
+#define RX_CHECK_X(NAME, BM, BN, WM, WN, KG, AKC, BKC, M, N, K)                                                        \
+  extern "C" __global__ __launch_bounds__(WM * WN * KG * 64, 2) void NAME(const float* A, const float* B, float* out) {  \
+    rx_check_epi<float, N> epi{out};                                                                                     \
+    rx_gemm_body_x<BM, BN, WM, WN, KG, AKC, BKC, M, N, K, 0, 0, false, rx_check_epi<float, N>>(A, B, epi);                \
+  }
+RX_CHECK_X(rx_check_x_nt, 128, 256, 2, 4, 1, true, true, 301, 277, 131)
+RX_CHECK_X(rx_check_x_nn, 128, 128, 2, 2, 2, true, false, 512, 512, 784)
+RX_CHECK_X(rx_check_x_tn, 128, 128, 2, 2, 1, false, false, 300, 200, 100)

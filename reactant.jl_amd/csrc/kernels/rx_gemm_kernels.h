@@ -1571,6 +1571,52 @@ RX_DEV void rx_wait_vmcnt_lgkm0() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
 }
 
+// The end of the bodies below: the groups' sums are added in group order (through LDS, where they share the blocks out)
+// and go to the epilogue functor in vectors as wide as the rows of the result allow (an odd N: one element at a time).
+template <int BM, int BN, int WM, int WN, int KG, int M, int N, bool BATCHED, int SPLIT, typename acc_t, typename acc_s, int NA, int NB, class Epi>
+RX_DEV void rx_group_finish(const acc_t (&acc)[NA][NB], const Epi& epi, int m0, int n0, int w, int grp, int lane, int batch) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
+  constexpr int NW = WM * WN, NV = N % 4 == 0 ? 4 : (N % 2 == 0 ? 2 : 1);
+  auto finish = [&](const acc_t& c, int unit) {
+    const int uw = unit / (NA * NB), b = unit % (NA * NB);
+    const int m = m0 + (uw / WN) * (BM / WM) + 16 * (b / NB) + (lane & 15);
+    const int nb = n0 + (uw % WN) * (BN / WN) + 16 * (b % NB) + 4 * (lane >> 4);
+#pragma unroll
+    for (int q = 0; q < 4; q += NV) {
+      const int n = nb + q;
+      if (m < M && n < N) {
+        acc_s v[NV];
+#pragma unroll
+        for (int l = 0; l < NV; ++l) v[l] = c[q + l];
+        if constexpr (BATCHED) epi(v, batch, m, n);
+        else if constexpr (SPLIT > 1) epi(v, (int)blockIdx.y, m, n);
+        else epi(v, m, n);
+      }
+    }
+  };
+  if constexpr (KG == 1) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) finish(acc[i][j], w * (NA * NB) + i * NB + j);
+  } else {
+    rx_wait_vmcnt_lgkm0<0>();
+    __syncthreads();
+    RX_LDS acc_t* part = (RX_LDS acc_t*)rx_smem;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) part[((w * (NA * NB) + i * NB + j) * KG + grp) * 64 + lane] = acc[i][j];
+    __syncthreads();
+    for (int u = grp * NW + w; u < NW * NA * NB; u += KG * NW) {
+      acc_t c = part[(u * KG) * 64 + lane];
+#pragma unroll
+      for (int g = 1; g < KG; ++g) c += part[(u * KG + g) * 64 + lane];
+      finish(c, u);
+    }
+  }
+}
+
 template <class EL, int BM, int BN, int WM, int WN, int KG, int S, bool A_KC, bool B_KC, int M, int N, int K, int RB, int CB, bool BATCHED, class Epi, int SPLIT = 1>
 RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typename EL::elem* __restrict__ B, const Epi& epi) {
   typedef typename rx_acc_of<EL>::type acc_t;
@@ -1709,48 +1755,288 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
     compute(t % SD, first + (unsigned)t * STEP);
   });
 
-  // result vectors as wide as the rows allow (an odd N: one element at a time)
-  constexpr int NV = N % 4 == 0 ? 4 : (N % 2 == 0 ? 2 : 1);
-  auto finish = [&](const acc_t& c, int unit) {
-    const int uw = unit / (NA * NB), b = unit % (NA * NB);
-    const int m = m0 + (uw / WN) * (BM / WM) + 16 * (b / NB) + (lane & 15);
-    const int nb = n0 + (uw % WN) * (BN / WN) + 16 * (b % NB) + 4 * (lane >> 4);
+  rx_group_finish<BM, BN, WM, WN, KG, M, N, BATCHED, SPLIT, acc_t, acc_s>(acc, epi, m0, n0, w, grp, lane, (int)batch);
+}
+
+// ===========================================================================
+// f32 products on the bf16 matrix cores: every operand as a sum of three bf16 numbers.
+// x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 3 x 8 bits and two signs hold the 24 bits exactly,
+// and so do subnormal parts (neither the conversion nor the bf16 MFMA flushes them).  A product is then six terms,
+// l h + h l + m m + m h + h m + h h; what is left out, m l + l m + l l, is at most 2^-25 of |x||y| and of either sign, below
+// the rounding of the sum.  Per K tile of 32 the five small terms are summed from zero, the smallest first, added to the
+// running sum, and h h goes into that: it is rounded twice per 32 k.  Error against 64 bits (2-norm, N(0,1) operands), this
+// body and the f32 MFMA bodies: 4096^3 4.4e-7 and 1.14e-6, 8192 x 4096 x 1024 2.1e-7 and 5.7e-7, 2048^3 3.1e-7 (two groups
+// 2.2e-7) and 5.7e-7, 2000 x 3000 x 500 1.5e-7 and 4.0e-7.
+// Two kinds of input do not split: an infinity (and a finite number that rounds to one) leaves inf - inf, so its
+// products become NaN; a number below 2^-102 may have bits below 2^-133, the last that bf16 holds.  The first is seen in the
+// result, which is not finite; the second while splitting, x - h - m being subnormal and not zero.  A workgroup that
+// sees either contracts its tile again with f32 MFMAs.
+//
+// Time: six 16 x 16 x 32 bf16 MFMAs take 96 cycles of the matrix pipe where eight 16 x 16 x 4 f32 MFMAs take 256.  What bounds
+// it is the sum of the MFMAs and the vector instructions (per element 5.5 to split it and one to test it, and four per
+// MFMA block and K tile to add the small terms): 786 and 589 thousand cycles per SIMD for 4096^3 on 128 x 128 tiles, of
+// the 1540 that the kernel takes.  They did not overlap in any order that was tried (a wavefront splitting while its partner
+// multiplies, with and without priorities, and instruction by instruction as here: 704, 722, 697 us), so
+// the splitting is done once per workgroup, between the global load into registers and the LDS tile, which holds three
+// bf16 planes of 32 k per operand: on the fragments, once per wavefront that reads them, 4096^3 took 842 us.  128 x 256 tiles
+// split less per product than 128 x 128 (4096^3 668 against 697 us).  4096^3 977 -> 668 us (206 TFLOP/s), 8192 x 4096 x 1024
+// 545 -> 370, 2048^3 128 -> 98, 2000 x 3000 x 500 66 -> 49.
+// One LDS stage; the next K tile waits split in registers, and the one after it is on its way into the registers that the
+// splitting has left.  K in groups (KG), range checks and sizes are those of rx_gemm_body_g.
+// LDS rows are 64 bytes, four chunks of 16.  A [row][k] operand is loaded as 16-byte vectors along k (a row of 32 k is
+// eight lanes) and lies at its row; of a [k][o] operand a thread loads 4 k x 4 o, and o lies at row (o % 4) (R / 4) + o / 4, so
+// that the lanes of a store write consecutive rows.  Chunks are swizzled by row / 2, so that eight rows read by eight
+// lanes, or eight rows' halves of a chunk written by sixteen, are the 128 bytes of one LDS cycle (no conflicts counted).
+// ===========================================================================
+struct rx_split4 { rx_u32 p[3][2]; };   // four elements: [plane][pair]
+// Half step H (of six) of splitting a pair: two or three vector instructions
+template <int H>
+RX_DEV void rx_split_step(float& x, float& y, rx_split4& s, int pair, bool& odd) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  if constexpr (H == 0 || H == 2) {
+    s.p[H / 2][pair] = __builtin_bit_cast(rx_u32, __builtin_convertvector((f2{x, y}), b2));
+    x -= __builtin_bit_cast(float, s.p[H / 2][pair] << 16);
+  } else if constexpr (H == 1 || H == 3) {
+    y -= __builtin_bit_cast(float, s.p[H / 2][pair] & 0xffff0000u);
+  } else if constexpr (H == 4) {
+    odd |= __builtin_amdgcn_classf(x, 0x90) | __builtin_amdgcn_classf(y, 0x90);   // subnormal of either sign
+  } else {
+    s.p[2][pair] = __builtin_bit_cast(rx_u32, __builtin_convertvector((f2{x, y}), b2));
+  }
+}
+
+// One operand of a K tile: R rows (o) of 32 k, loaded by NT threads.  KC: stored [o][k] (ld = K), else [k][o] (ld = O).
+// STEP: K tiles that the groups take at a time, so the last ones of some groups may lie past K.
+template <int R, int NT, bool KC, int O, int K, int STEP>
+struct rx_x_operand {
+  static constexpr int NV = R * 8 / NT;              // 16-byte vectors per thread
+  static constexpr unsigned KBYTES = (unsigned)K * 4, LDB = (KC ? K : O) * 4u;
+  static constexpr int BL = 8;                       // blocks of four o that consecutive lanes take
+  static_assert(R % 32 == 0 && R * 8 % NT == 0 && (KC || R * 2 % NT == 0), "whole vectors (blocks) per thread");
+  RX_DEV int row_of(int o) { return KC ? o : (o & 3) * (R / 4) + (o >> 2); }                                   // LDS row
+  RX_DEV int chunk_of(int o, int c) { return c ^ ((row_of(o) >> 1) & 3) ^ (KC ? 0 : (o & 3)); }              // of the row's four
+  // thread t: vector i (KC), or block u of 4 k x 4 o whose vector j is k0 + j
+  RX_DEV void block(int u, int* o, int* k) { *o = 4 * (u / (BL * 8) * BL + u % BL); *k = 4 * (u / BL % 8); }
+  // vectors first .. first + N - 1 of K tile kt (of whole blocks); positions past K read as zero
+  template <int FIRST, int N>
+  RX_DEV void load(rx_f32x4v (&raw)[NV], const __amdgpu_buffer_rsrc_t& rs, int o0, int t, unsigned kt) {
+    if constexpr (KC) {
+      const unsigned kb = kt * 128 + (t & 7) * 16;
+      const unsigned base = (unsigned)(o0 + (t >> 3)) * LDB + kb;
 #pragma unroll
-    for (int q = 0; q < 4; q += NV) {
-      const int n = nb + q;
-      if (m < M && n < N) {
-        acc_s v[NV];
+      for (int i = FIRST; i < FIRST + N; ++i) {
+        const unsigned o = base + (unsigned)(i * (NT / 8)) * LDB;
+        raw[i] = __builtin_bit_cast(rx_f32x4v, __builtin_amdgcn_raw_buffer_load_b128(rs, KBYTES % (128 * STEP) != 0 ? (kb < KBYTES ? o : 0xfffffff0u) : o, 0, 0));
+      }
+    } else {
 #pragma unroll
-        for (int l = 0; l < NV; ++l) v[l] = c[q + l];
-        if constexpr (BATCHED) epi(v, (int)batch, m, n);
-        else if constexpr (SPLIT > 1) epi(v, (int)blockIdx.y, m, n);
-        else epi(v, m, n);
+      for (int b = FIRST / 4; b < (FIRST + N) / 4; ++b) {
+        int o, k;
+        block(b * NT + t, &o, &k);
+        const unsigned base = (kt * 32 + k) * LDB + (unsigned)(o0 + o) * 4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) raw[4 * b + j] = __builtin_bit_cast(rx_f32x4v, __builtin_amdgcn_raw_buffer_load_b128(rs, base + (unsigned)j * LDB, 0, 0));
       }
     }
-  };
-  if constexpr (KG == 1) {
+  }
+  // the four elements with consecutive k that go to one place of the LDS tile, q of NV: (o, first k, values)
+  RX_DEV rx_f32x4v quad(const rx_f32x4v (&raw)[NV], int q, int t, unsigned kt, int* o, int* k) {
+    rx_f32x4v v;
+    if constexpr (KC) {
+      *o = q * (NT / 8) + (t >> 3);
+      *k = 4 * (t & 7);
+      v = raw[q];
+      if constexpr (KBYTES % 16 != 0) {   // K ends inside a vector
 #pragma unroll
-    for (int i = 0; i < NA; ++i)
+        for (int d = 0; d < 4; ++d) v[d] = kt * 32 + 4 * (t & 7) + d < (unsigned)K ? v[d] : 0.f;
+      }
+    } else {
+      block(q / 4 * NT + t, o, k);
+      *o += q % 4;
 #pragma unroll
-      for (int j = 0; j < NB; ++j) finish(acc[i][j], w * (NA * NB) + i * NB + j);
-  } else {
-    // every group leaves its 16 x 16 blocks in LDS; the wavefronts of the workgroup share the blocks out, add the
-    // groups' sums in order and run the epilogue
-    rx_wait_vmcnt_lgkm0<0>();
-    __syncthreads();
-    RX_LDS acc_t* part = (RX_LDS acc_t*)rx_smem;
+      for (int d = 0; d < 4; ++d) v[d] = raw[q / 4 * 4 + d][q % 4];
+    }
+    return v;
+  }
+  RX_DEV void put(const rx_split4 (&s)[NV], RX_LDS rx_u8* tile, int t) {
+    typedef rx_u32 u2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int i = 0; i < NA; ++i)
+    for (int q = 0; q < NV; ++q) {
+      const rx_f32x4v none[NV] = {};
+      int o, k;
+      (void)quad(none, q, t, 0, &o, &k);
+      RX_LDS rx_u8* at = tile + row_of(o) * 64 + chunk_of(o, k >> 3) * 16 + (k & 4) * 2;
 #pragma unroll
-      for (int j = 0; j < NB; ++j) part[((w * (NA * NB) + i * NB + j) * KG + grp) * 64 + lane] = acc[i][j];
-    __syncthreads();
-    for (int u = wave; u < NW * NA * NB; u += KG * NW) {
-      acc_t c = part[(u * KG) * 64 + lane];
-#pragma unroll
-      for (int g = 1; g < KG; ++g) c += part[(u * KG + g) * 64 + lane];
-      finish(c, u);
+      for (int p = 0; p < 3; ++p) *(RX_LDS u2*)(at + p * (R * 64)) = u2{s[q].p[p][0], s[q].p[p][1]};
     }
   }
+  RX_DEV rx_bf16x8 frag(const RX_LDS rx_u8* tile, int plane, int row0, int lane) {
+    const int o = row0 + (lane & 15);
+    return *(const RX_LDS rx_bf16x8*)(tile + plane * (R * 64) + row_of(o) * 64 + chunk_of(o, lane >> 4) * 16);
+  }
+  // the same tile in f32, rows of 144 bytes
+  RX_DEV void put_f32(const rx_f32x4v (&raw)[NV], RX_LDS rx_u8* tile, int t, unsigned kt) {
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+      int o, k;
+      const rx_f32x4v v = quad(raw, q, t, kt, &o, &k);
+      *(RX_LDS rx_f32x4v*)(tile + o * 144 + k * 4) = v;
+    }
+  }
+  RX_DEV rx_i32x8 frag_f32(const RX_LDS rx_u8* tile, int row0, int lane) {
+    const RX_LDS rx_u8* at = tile + (row0 + (lane & 15)) * 144 + (lane >> 4) * 32;
+    struct { rx_i32x4 a, b; } both = {*(const RX_LDS rx_i32x4*)at, *(const RX_LDS rx_i32x4*)(at + 16)};
+    return __builtin_bit_cast(rx_i32x8, both);
+  }
+};
+
+template <int BM, int BN, int WM, int WN, int KG, bool A_KC, bool B_KC, int M, int N, int K, int RB, int CB, bool BATCHED, class Epi>
+RX_DEV void rx_gemm_body_x(const float* __restrict__ A, const float* __restrict__ B, const Epi& epi) {
+  constexpr int NW = WM * WN, NT = NW * 64, NA = BM / WM / 16, NB = BN / WN / 16;
+  typedef rx_x_operand<BM, NT, A_KC, M, K, KG> OA;
+  typedef rx_x_operand<BN, NT, B_KC, N, K, KG> OB;
+  static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "tile shape");
+  static_assert((long long)M * K * 4 < (1ll << 31) && (long long)N * K * 4 < (1ll << 31), "32-bit operand offsets");
+  constexpr int KT = (K + 31) / 32, STEP = KG, KTG = (KT + STEP - 1) / STEP;   // K tiles, and per group
+  static_assert((A_KC || ((long long)K + 128 * STEP) * M * 4 < (1ll << 32)) && (B_KC || ((long long)K + 128 * STEP) * N * 4 < (1ll << 32)), "offsets of the last groups' K tiles");
+  constexpr int STAGE = (BM + BN) * 192;
+  extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
+  __shared__ int again[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave / NW, w = wave % NW, wm = w / WN, wn = w % WN, t = tid - grp * NT;
+  RX_LDS rx_u8* const lds = (RX_LDS rx_u8*)rx_smem + grp * STAGE;
+  constexpr int GM = (M + BM - 1) / BM, GN = (N + BN - 1) / BN;
+  int bm, bn;
+  if (!rx_gemm_tile<GM, GN, RB, CB>(blockIdx.x, &bm, &bn)) return;
+  const int m0 = bm * BM, n0 = bn * BN;
+  const long long batch = BATCHED ? blockIdx.y : 0;
+  const unsigned first = grp;   // this group's first K tile
+  const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void*)(A + batch * (long long)M * K), 0, (unsigned)M * (unsigned)K * 4u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)(B + batch * (long long)N * K), 0, (unsigned)N * (unsigned)K * 4u, 0x00020000);
+  rx_f32x4v acc[NA][NB];
+  rx_f32x4v va[OA::NV], vb[OB::NV];   // a K tile on its way
+  rx_split4 sa[OA::NV], sb[OB::NV];   // the next one, split
+  float px, py;                       // the pair being split
+  bool odd = false;                   // a number that does not split into three bf16
+  auto kt_of = [&](int i) { return first + (unsigned)i * STEP; };
+  auto load = [&](int i) __attribute__((always_inline)) {
+    OA::template load<0, OA::NV>(va, ra, m0, t, kt_of(i));
+    OB::template load<0, OB::NV>(vb, rb, n0, t, kt_of(i));
+  };
+  // Half step H of splitting K tile i (there are HS); registers that it has finished with take their part of tile i + 1.
+  constexpr int HS = (OA::NV + OB::NV) * 12;
+  auto step = [&](auto HH, int i) __attribute__((always_inline)) {
+    constexpr int h = decltype(HH)::value, q = h / 12, pair = h / 6 % 2;
+    int o, k;
+    if constexpr (q < OA::NV) {
+      if constexpr (h % 6 == 0) { const rx_f32x4v v = OA::quad(va, q, t, kt_of(i), &o, &k); px = v[2 * pair]; py = v[2 * pair + 1]; }
+      rx_split_step<h % 6>(px, py, sa[q], pair, odd);
+      if constexpr (h % 12 == 11 && (A_KC || q % 4 == 3)) OA::template load<A_KC ? q : q - 3, A_KC ? 1 : 4>(va, ra, m0, t, kt_of(i + 1));
+    } else {
+      constexpr int p = q - OA::NV;
+      if constexpr (h % 6 == 0) { const rx_f32x4v v = OB::quad(vb, p, t, kt_of(i), &o, &k); px = v[2 * pair]; py = v[2 * pair + 1]; }
+      rx_split_step<h % 6>(px, py, sb[p], pair, odd);
+      if constexpr (h % 12 == 11 && (B_KC || p % 4 == 3)) OB::template load<B_KC ? p : p - 3, B_KC ? 1 : 4>(vb, rb, n0, t, kt_of(i + 1));
+    }
+  };
+  auto put = [&]() __attribute__((always_inline)) {
+    OA::put(sa, lds, t);
+    OB::put(sb, lds + BM * 192, t);
+  };
+  // LDS operations of this wavefront are complete, loads into registers stay under way
+  auto publish = [&]() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    rx_wait_vmcnt_lgkm0<63>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = rx_f32x4v{0.f, 0.f, 0.f, 0.f};
+  };
+  // The tile in LDS is multiplied; with AHEAD the half steps of splitting K tile i are dealt out between the MFMAs.
+  auto compute = [&](auto AHEAD, int i) __attribute__((always_inline)) {
+    const RX_LDS rx_u8* ta = lds;
+    const RX_LDS rx_u8* tb = ta + BM * 192;
+    rx_bf16x8 fb[3][NB], fa[3];
+    rx_f32x4v small[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) fb[p][j] = OB::frag(tb, p, wn * (BN / WN) + 16 * j, lane);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) fa[p] = OA::frag(ta, p, wm * (BM / WM), lane);
+    constexpr int SLOTS = NA * NB * 6;
+    // the B fragment is the row operand: a lane ends with four consecutive n of one m
+    rx_static_for<0, SLOTS>([&](auto SL) {
+      constexpr int sl = decltype(SL)::value, ia = sl / (6 * NB), q = sl / NB % 6, j = sl % NB;
+      if constexpr (q < 5) {
+        small[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[q == 0 ? 2 : (q == 2 || q == 3 ? 1 : 0)][j], fa[q == 1 ? 2 : (q == 2 || q == 4 ? 1 : 0)],
+                                                           q == 0 ? rx_f32x4v{0.f, 0.f, 0.f, 0.f} : small[j], 0, 0, 0);
+      } else {
+        acc[ia][j] += small[j];
+        acc[ia][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fb[0][j], fa[0], acc[ia][j], 0, 0, 0);
+      }
+      if constexpr (ia + 1 < NA && sl % (6 * NB) == 6 * NB - 1) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) fa[p] = OA::frag(ta, p, wm * (BM / WM) + 16 * (ia + 1), lane);
+      }
+      if constexpr (decltype(AHEAD)::value != 0) {
+        rx_static_for<sl * HS / SLOTS, (sl + 1) * HS / SLOTS>([&](auto H) { step(H, i); });
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    });
+  };
+
+  clear();
+  load(0);
+  rx_static_for<0, HS>([&](auto H) { step(H, 0); });
+  put();
+  publish();
+  for (int i = 0; i + 1 < KTG; ++i) {
+    compute(rx_int<1>{}, i + 1);
+    publish();
+    put();
+    publish();
+  }
+  compute(rx_int<0>{}, 0);
+
+  float fin = 0.f;   // NaN once a sum is not finite
+#pragma unroll
+  for (int i = 0; i < NA; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) fin = __builtin_fmaf(acc[i][j][q], 0.f, fin);
+  const bool mine = __builtin_amdgcn_ballot_w64(odd || fin != fin) != 0;
+  if (lane == 0) again[wave] = mine;
+  __syncthreads();
+  int any = 0;
+#pragma unroll
+  for (int u = 0; u < NW * KG; ++u) any |= again[u];
+  if (__builtin_amdgcn_readfirstlane(any)) {
+    clear();
+    for (int i = 0; i < KTG; ++i) {
+      load(i);
+      __syncthreads();
+      OA::put_f32(va, lds, t, kt_of(i));
+      OB::put_f32(vb, lds + BM * 192, t, kt_of(i));
+      __syncthreads();
+      rx_i32x8 fb[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) fb[j] = OB::frag_f32(lds + BM * 192, wn * (BN / WN) + 16 * j, lane);
+#pragma unroll
+      for (int i2 = 0; i2 < NA; ++i2) {
+        const rx_i32x8 fa = OA::frag_f32(lds, wm * (BM / WM) + 16 * i2, lane);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) rx_el_f32::mma(acc[i2][j], fb[j], fa);
+      }
+    }
+  }
+  rx_group_finish<BM, BN, WM, WN, KG, M, N, BATCHED, 1, rx_f32x4v, float>(acc, epi, m0, n0, w, grp, lane, (int)batch);
 }
 
 // ===========================================================================

@@ -54,7 +54,7 @@ static GemmChoice choose_gemm_f64(int64_t batch, int64_t M, int64_t N, int64_t K
 // ---------------------------------------------------------------------------
 // rx_gemm_body_g (K in groups inside the workgroup): tile, wavefronts, groups and stages
 // ---------------------------------------------------------------------------
-struct GroupTile { int BM, BN, WM, WN, KG, S; };
+struct GroupTile { int BM, BN, WM, WN, KG, S, split3 = 0; };   // split3: f32 operands as three bf16 each (rx_gemm_body_x)
 
 static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t, int64_t* lds) {
   const int es = info(dt).size;
@@ -68,7 +68,15 @@ static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bo
   if (batch > 65535) return false;                                         // blockIdx.y
   // accumulators and fragments of a wavefront within its share of the register file
   const int na = t.BM / t.WM / 16, nb = t.BN / t.WN / 16;
-  if (na * nb * (es == 8 ? 8 : 4) + 8 * (na + nb) + 48 > 512 / std::max(1, (NW * t.KG + 3) / 4)) return false;
+  const int share = 512 / std::max(1, (NW * t.KG + 3) / 4);
+  if (t.split3) {   // rx_gemm_body_x: whole vectors or 4 x 4 blocks per thread, loaded and split registers beside the fragments
+    const int nt = NW * 64, nv = (t.BM + t.BN) * 8 / nt;
+    if (dt != DT::F32 || split > 1 || t.BM % 32 || t.BN % 32 || t.BM * (a_kc ? 8 : 2) % nt || t.BN * (b_kc ? 8 : 2) % nt) return false;
+    if (na * nb * 4 + 10 * nv + 12 * (nb + 1) + 40 > std::min(share, 256)) return false;   // two wavefronts per SIMD
+    *lds = std::max<int64_t>((int64_t)t.KG * (t.BM + t.BN) * 192, t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * 4 : 0);
+    return *lds + 64 <= 160 * 1024;   // (64: the wavefronts' votes)
+  }
+  if (na * nb * (es == 8 ? 8 : 4) + 8 * (na + nb) + 48 > share) return false;
   const int64_t nl = (t.BM + t.BN) / 8 / NW, sd = std::min<int64_t>(t.S, KTG);
   if (nl * (sd - 1) > 63) return false;                                    // outstanding loads that a wait can count
   const int64_t ring = (int64_t)t.KG * sd * (t.BM + t.BN) * 128, sums = t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * (es == 8 ? 8 : 4) : 0;
@@ -115,6 +123,17 @@ static double group_estimate(DT dt, int64_t batch, int64_t M, int64_t N, int64_t
   return cycles / 2400.0;
 }
 
+// rx_gemm_body_x: microseconds per K tile of 32 of a workgroup, alone on its compute unit or beside a second one.
+// Measured: 128 x 128 2048^3 (one workgroup per compute unit) 107 us, 4096^3 (four) 697, 8192 x 4096 x 1024 (eight) 371; two groups
+// 2048^3 98; 128 x 256 4096^3 668, 8192 x 4096 x 1024 370.
+static double split3_estimate(int64_t batch, int64_t M, int64_t N, int64_t K, const GroupTile& t) {
+  const int64_t T = ((M + t.BM - 1) / t.BM) * ((N + t.BN - 1) / t.BN) * batch, n = (T + 255) / 256, kt = ((K + 31) / 32 + t.KG - 1) / t.KG;
+  const double area = (double)t.BM * t.BN / 16384.0;
+  if (t.KG > 1) return 11.0 + (double)(n * kt) * 1.45 * t.KG * area;
+  if (t.WM * t.WN > 4) return 8.0 + (double)(n * kt) * 1.3 * area;
+  return 8.0 + (double)kt * ((double)(n / 2) * 2.75 + (double)(n % 2) * 1.6) * area;
+}
+
 static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t) {
   GemmChoice c;
   int64_t lds = 0;
@@ -134,20 +153,25 @@ static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t
   c.grid[0] = (unsigned)gemm_grid(gm, gn, rb, cb);
   c.grid[1] = (unsigned)(split > 1 ? split : batch);
   c.split = split;
-  c.est_us = group_estimate(dt, batch, M, N, K, a_kc, b_kc, split, t, lds);
+  c.est_us = t.split3 ? split3_estimate(batch, M, N, K, t) : group_estimate(dt, batch, M, N, K, a_kc, b_kc, split, t, lds);
   const std::string el = dt == DT::F64 ? "rx_el_f64" : dt == DT::F32 ? "rx_el_f32" : dt == DT::BF16 ? "rx_el_bf16" : dt == DT::F16 ? "rx_el_f16" : "rx_el_f8";
   std::ostringstream o;
-  o << el << ", " << t.BM << ", " << t.BN << ", " << t.WM << ", " << t.WN << ", " << t.KG << ", " << t.S << ", " << (a_kc ? "true" : "false") << ", "
+  if (!t.split3) o << el << ", ";
+  o << t.BM << ", " << t.BN << ", " << t.WM << ", " << t.WN << ", ";
+  if (!t.split3) o << t.KG << ", " << t.S << ", ";
+  else o << t.KG << ", ";
+  o << (a_kc ? "true" : "false") << ", "
     << (b_kc ? "true" : "false") << ", " << M << ", " << N << ", " << K << ", " << rb << ", " << cb;
   c.targs = o.str();
-  c.skeleton = "rx_gemm_body_g";
+  c.skeleton = t.split3 ? "rx_gemm_body_x" : "rx_gemm_body_g";
   c.kind = dt == DT::F64 ? "gemm_f64" : dt == DT::F32 ? "gemm_f32" : dt == DT::BF16 ? "gemm_bf16" : dt == DT::F16 ? "gemm_f16" : "gemm_f8";
-  c.stype_a = el + "::elem";
+  c.stype_a = t.split3 ? "float" : el + "::elem";
+  c.waves = t.split3 ? 2 : 0;   // two workgroups of four wavefronts share a compute unit
   c.ok = true;
   return c;
 }
 
-// The tile with the smallest estimate.  RX_GEMM_G=BM,BN,WM,WN,KG,S asks for one (products it does not fit keep the
+// The tile with the smallest estimate.  RX_GEMM_G=BM,BN,WM,WN,KG,S asks for one (a seventh number, 1: rx_gemm_body_x, which has no S; products it does not fit keep the
 // estimate's), RX_GEMM_G=0 leaves this skeleton out.
 static GemmChoice choose_group(DT dt, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split) {
   GemmChoice best;
@@ -159,7 +183,7 @@ static GemmChoice choose_group(DT dt, DT out, int64_t batch, int64_t M, int64_t 
   if (const char* e = getenv("RX_GEMM_G")) {
     GroupTile t;
     if (!strcmp(e, "0")) return best;
-    if (sscanf(e, "%d,%d,%d,%d,%d,%d", &t.BM, &t.BN, &t.WM, &t.WN, &t.KG, &t.S) != 6 || t.BM < 16 || t.BN < 16 || t.WM < 1 || t.WN < 1 || t.KG < 1 || t.S < 1)
+    if (sscanf(e, "%d,%d,%d,%d,%d,%d,%d", &t.BM, &t.BN, &t.WM, &t.WN, &t.KG, &t.S, &t.split3) < 6 || t.BM < 16 || t.BN < 16 || t.WM < 1 || t.WN < 1 || t.KG < 1 || t.S < 1 || t.split3 < 0 || t.split3 > 1)
       throw std::runtime_error("RX_GEMM_G wants BM,BN,WM,WN,KG,S");
     best = group_gemm(dt, batch, M, N, K, a_kc, b_kc, split, t);
     if (best.ok) return best;
@@ -179,6 +203,14 @@ static GemmChoice choose_group(DT dt, DT out, int64_t batch, int64_t M, int64_t 
         const double c = group_estimate(dt, batch, M, N, K, a_kc, b_kc, split, t, lds);
         if (cost == 0 || c < cost) { cost = c; pick = t; }
       }
+  // f32 products that fill the chip with 128-wide tiles: operands split into bf16 (rx_gemm_body_x)
+  if (dt == DT::F32)
+    for (const GroupTile& t : {GroupTile{128, 128, 2, 2, 1, 1, 1}, GroupTile{128, 128, 2, 2, 2, 1, 1}, GroupTile{128, 256, 2, 4, 1, 1, 1}, GroupTile{256, 128, 4, 2, 1, 1, 1}}) {
+      int64_t lds = 0;
+      if (!group_fits(dt, batch, M, N, K, a_kc, b_kc, split, t, &lds)) continue;
+      const double c = split3_estimate(batch, M, N, K, t);
+      if (cost == 0 || c < cost) { cost = c; pick = t; }
+    }
   return cost > 0 ? group_gemm(dt, batch, M, N, K, a_kc, b_kc, split, pick) : best;
 }
 
@@ -378,10 +410,6 @@ GemmChoice choose_gemm(DT a, DT b, DT out, int64_t batch, int64_t M, int64_t N, 
     const double us = rounds(256, sq ? 256 : 128) * (sq ? kt * 1.33 + 10.5 : kt * 0.77 + 9.5) + 3.0;
     return kt >= 16 && g.est_us < us ? g : c;
   }
-  // f32 on 256 x 256 tiles of the ring skeleton: 0.9 of the MFMA peak on a grid of whole rounds (4096^3 964 against 973 us),
-  // less on others (8192 x 4096 x 1024 538 against 522, 2048^3 157 against 146)
-  if (c.skeleton == "rx_gemm_body_dl" && a == DT::F32 && c.targs.find(", 256, 256, ") != std::string::npos)
-    return rounds(256, 256) * ((double)K * 0.2335 + 8.0) < g.est_us ? c : g;
   // f32, an operand of at most 64 rows against 512 tiles and more (the features of a convolution and its window matrix)
   if (c.skeleton == "rx_gemm_body_dl" && a == DT::F32 && (M <= 64 || N <= 64) && ((M + 63) / 64) * ((N + 63) / 64) >= 1024) return c;
   return g;
@@ -392,7 +420,7 @@ std::string gemm_instance(const GemmChoice& c, const std::string& kbase, const s
   std::ostringstream o;
   o << "// dot_general on MFMA: " << c.kind << " <" << c.targs << ">\n";
   const bool fn = !fa.type.empty() || !fb.type.empty();
-  o << "extern \"C\" __global__ __launch_bounds__(" << c.block << ") void " << kbase << "_gemm(";
+  o << "extern \"C\" __global__ __launch_bounds__(" << c.block << (c.waves ? ", " + std::to_string(c.waves) : std::string()) << ") void " << kbase << "_gemm(";
   // operands that are read from memory come first, then what the operand functors read, then the epilogue's operands
   std::string params;
   if (fa.type.empty()) params += ", const " + c.stype_a + "* __restrict__ A";

@@ -19,7 +19,8 @@ struct GemmChoice {
   int depth = 0;            // rx_gemm_body_s: blocks of the streamed operand read ahead (0: the skeleton's default)
   int stream_stages = 0;    // rx_gemm_body_s: LDS stages per operand (0: not that skeleton)
   int bk = 0;               // rx_gemm_body_dl: elements of K per tile
-  double est_us = 0;        // rx_gemm_body_g: estimated time
+  int waves = 0;          // wavefronts per SIMD that the registers have to leave room for (0: as many as a workgroup needs)
+  double est_us = 0;        // rx_gemm_body_g and rx_gemm_body_x: estimated time
 };
 
 // Workgroups to launch for a gm x gn grid of tiles: the kernels walk the tiles in blocks of 4 x 8,

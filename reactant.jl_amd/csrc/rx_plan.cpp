@@ -1016,7 +1016,7 @@ struct Planner {
       // another launch (4 us each between dependent launches)
       const double extra = followed[d.id] ? 8.0 : 4.0;
       int S = 1;
-      double best = whole.skeleton == "rx_gemm_body_g" ? whole.est_us : 1e30;
+      double best = whole.est_us > 0 ? whole.est_us : 1e30;   // the skeletons that slices compete with have an estimate
       // Cut whatever the estimates say: products that nothing elementwise follows, of at most 128 whole tiles and K >= 2048 (f32 256 x 256 x
       // 2048 11.6 against 7.9 us uncut, bf16 128 x 128 x 16384 15.7 against 23.7); and 17 to 32 rows of 16-bit elements against
       // [k][n] weights with K >= 4096 (32 x 4096 x 25088 57 against 104 us, 32 x 4096 x 4096 15.5 against 11.2).

@@ -60,3 +60,63 @@ def test_rows_past_an_edge_do_not_leak_into_others(rx, client):
     fin = np.isfinite(got[0].a)
     assert not fin[17].any() and not fin[:, 40].any()
     assert fin[np.arange(70) != 17][:, np.arange(66) != 40].all()
+
+
+X_TILES = ["128,128,2,2,1,1,1", "128,128,2,2,2,1,1", "128,256,2,4,1,1,1", "256,128,4,2,1,1,1", "64,64,2,1,2,1,1"]
+# edges of both dimensions and of K inside a vector, one K tile for each of two groups, whole tiles, batches
+X_SHAPES = [(129, 260, 77, 0), (300, 131, 1030, 0), (128, 256, 64, 0), (70, 515, 96, 0), (130, 66, 131, 3)]
+
+
+def x_fits(tile, order):
+    bm, bn, wm, wn = (int(v) for v in tile.split(",")[:4])
+    return (order[0] or bm * 2 % (wm * wn * 64) == 0) and (order[1] or bn * 2 % (wm * wn * 64) == 0)
+
+
+@pytest.mark.parametrize("tile,shape,order", [(t, s, o) for t in X_TILES for i, s in enumerate(X_SHAPES) for o in (ORDERS[i % 4], ORDERS[(i + 1) % 4]) if x_fits(t, o)])
+def test_f32_operands_split_into_bf16(rx, client, monkeypatch, tile, shape, order):
+    """Componentwise within what two roundings of the sum per 32 k and the terms left out allow, (K / 16 + 2) 2^-24 of |A| . |B|."""
+    M, N, K, batch = shape
+    text, sa, sb = dot_module(M, N, K, "f32", "f32", *order, batch)
+    monkeypatch.setenv("RX_GEMM_G", tile)
+    monkeypatch.setenv("RX_SPLIT_K", "0")
+    assert "rx_gemm_body_x<" in rx.compile_offline(text, with_source=True)
+    a, b = (I.tensor(np.random.default_rng(s).normal(size=z), "f32") for s, z in ((6, sa), (7, sb)))
+    got, exe = gpu_run(rx, client, text, [a, b])
+    ref = oracle_run(text, [a, b], hifi=True)
+    assert contraction_err(got[0].a, ref[0].a, dot_bound(text, [a, b])) <= (K / 16 + 2) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("order", ORDERS)
+def test_numbers_that_do_not_split_into_bf16(rx, client, monkeypatch, order):
+    """Infinities, NaN, numbers that round to infinity in bf16, subnormals: as the f32 MFMAs of the general path have them."""
+    M, N, K = 140, 130, 70
+    text, sa, sb = dot_module(M, N, K, "f32", "f32", *order)
+    rng = np.random.default_rng(8)
+    A, B = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(N, K)).astype(np.float32)
+    A[3, 5], A[4, 6], A[5, 69], A[131, 7], B[129, 0] = np.inf, -np.inf, np.nan, np.float32(3.4e38), np.inf
+    B[:, 7] *= np.float32(1e-3)                       # finite sums with the largest numbers
+    A[20:24] = rng.normal(size=(4, K)) * 1e-36        # bits below what bf16 holds
+    A[24:28] = rng.normal(size=(4, K)) * 1e-40        # subnormal
+    A[28], A[28, 1], B[40, :] = 0, 1e-37, 0           # one tiny product alone
+    B[40, 1] = 1 + 2.0 ** -20
+    a, b = (I.Tensor(np.ascontiguousarray(x if kc else x.T), "f32") for x, kc in ((A, order[0]), (B, order[1])))
+    out = {}
+    for tile in ("0", "128,128,2,2,1,1,1", "128,128,2,2,2,1,1"):
+        monkeypatch.setenv("RX_GEMM_G", tile)
+        assert ("rx_gemm_body_x<" in rx.compile_offline(text, with_source=True)) == (tile != "0")
+        out[tile] = gpu_run(rx, client, text, [a, b])[0][0].a
+    ref = out.pop("0")
+    with np.errstate(all="ignore"):
+        exact = A.astype(np.float64) @ B.astype(np.float64).T
+        bound = np.abs(A).astype(np.float64) @ np.abs(B).astype(np.float64).T
+    for got in out.values():
+        assert np.array_equal(np.isnan(got), np.isnan(ref)) and np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
+        fin = np.isfinite(ref)
+        # a rounding per product and K 2^-149 for sums that are subnormal
+        assert (np.abs(got[fin].astype(np.float64) - exact[fin]) <= bound[fin] * (K + 2) * 2.0 ** -24 + K * 2.0 ** -149).all()
+
+
+def test_large_f32_products_take_the_split(rx):
+    for (m, n, k, order) in ((4096, 4096, 4096, ORDERS[1]), (2048, 2048, 2048, ORDERS[3]), (2000, 3000, 500, ORDERS[0])):
+        assert "rx_gemm_body_x<" in rx.compile_offline(dot_module(m, n, k, "f32", "f32", *order)[0], with_source=True)
+    assert "rx_gemm_body_g<" in rx.compile_offline(dot_module(777, 1001, 1531, "f32", "f32", True, False)[0], with_source=True)
