@@ -1899,7 +1899,9 @@ RX_DEV void rx_gemm_body_x(const float* __restrict__ A, const float* __restrict_
   static_assert(BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "tile shape");
   static_assert((long long)M * K * 4 < (1ll << 31) && (long long)N * K * 4 < (1ll << 31), "32-bit operand offsets");
   constexpr int KT = (K + 31) / 32, STEP = KG, KTG = (KT + STEP - 1) / STEP;   // K tiles, and per group
-  static_assert((A_KC || ((long long)K + 128 * STEP) * M * 4 < (1ll << 32)) && (B_KC || ((long long)K + 128 * STEP) * N * 4 < (1ll << 32)), "offsets of the last groups' K tiles");
+  // The last tile that is requested (never contracted) is KTG of the last group: its rows are below K + 64 STEP.  The same
+  // bound as the host's (group_fits in rx_gemm.cpp).
+  static_assert((A_KC || ((long long)K + 64 * STEP) * M * 4 < (1ll << 32)) && (B_KC || ((long long)K + 64 * STEP) * N * 4 < (1ll << 32)), "offsets of the last groups' K tiles");
   constexpr int STAGE = (BM + BN) * 192;
   extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
   __shared__ int again[16];
