@@ -1571,9 +1571,59 @@ RX_DEV void rx_wait_vmcnt_lgkm0() {
   __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | ((N >> 4) << 14));
 }
 
+// Totals that short sums are added to: one sum in the accumulators' own type, or (wide) sums of a few of them, which are
+// added in f64 (f32) or with the rounding errors of the additions kept apart, as two-sum gives them (f64; an infinite
+// or NaN total has no such error).
+template <class A> struct rx_total_same {
+  A s = {0, 0, 0, 0};
+  __device__ __forceinline__ void add(A v) { s += v; }
+  __device__ __forceinline__ void flush() {}
+  __device__ __forceinline__ A value() { return s; }
+};
+template <class A> struct rx_total_wide;
+template <> struct rx_total_wide<rx_f32x4v> {
+  rx_f32x4v few = {0, 0, 0, 0};
+  rx_f64x4 s = {0, 0, 0, 0};
+  __device__ __forceinline__ void add(rx_f32x4v v) { few += v; }
+  __device__ __forceinline__ void flush() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] += (double)few[i];
+    few = rx_f32x4v{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ rx_f32x4v value() {
+    flush();
+    return rx_f32x4v{(float)s[0], (float)s[1], (float)s[2], (float)s[3]};
+  }
+};
+template <> struct rx_total_wide<rx_f64x4> {
+  rx_f64x4 few = {0, 0, 0, 0}, s = {0, 0, 0, 0}, e = {0, 0, 0, 0};
+  __device__ __forceinline__ void add(rx_f64x4 v) { few += v; }
+  __device__ __forceinline__ void flush() {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double t = s[i] + few[i], b = t - s[i];
+      e[i] += (s[i] - (t - b)) + (few[i] - b);
+      s[i] = t;
+    }
+    few = rx_f64x4{0, 0, 0, 0};
+  }
+  __device__ __forceinline__ rx_f64x4 value() {
+    flush();
+    rx_f64x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double t = s[i] + e[i];
+      r[i] = t == t ? t : s[i];
+    }
+    return r;
+  }
+};
+template <class A, bool WIDE> struct rx_total { typedef rx_total_same<A> type; };
+template <class A> struct rx_total<A, true> { typedef rx_total_wide<A> type; };
+
 // The end of the bodies below: the groups' sums are added in group order (through LDS, where they share the blocks out)
 // and go to the epilogue functor in vectors as wide as the rows of the result allow (an odd N: one element at a time).
-template <int BM, int BN, int WM, int WN, int KG, int M, int N, bool BATCHED, int SPLIT, typename acc_t, typename acc_s, int NA, int NB, class Epi>
+template <int BM, int BN, int WM, int WN, int KG, int M, int N, bool BATCHED, int SPLIT, bool WIDE, typename acc_t, typename acc_s, int NA, int NB, class Epi>
 RX_DEV void rx_group_finish(const acc_t (&acc)[NA][NB], const Epi& epi, int m0, int n0, int w, int grp, int lane, int batch) {
   extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
   constexpr int NW = WM * WN, NV = N % 4 == 0 ? 4 : (N % 2 == 0 ? 2 : 1);
@@ -1609,15 +1659,26 @@ RX_DEV void rx_group_finish(const acc_t (&acc)[NA][NB], const Epi& epi, int m0, 
       for (int j = 0; j < NB; ++j) part[((w * (NA * NB) + i * NB + j) * KG + grp) * 64 + lane] = acc[i][j];
     __syncthreads();
     for (int u = grp * NW + w; u < NW * NA * NB; u += KG * NW) {
-      acc_t c = part[(u * KG) * 64 + lane];
+      if constexpr (WIDE) {
+        rx_total_wide<acc_t> c;
 #pragma unroll
-      for (int g = 1; g < KG; ++g) c += part[(u * KG + g) * 64 + lane];
-      finish(c, u);
+        for (int g = 0; g < KG; ++g) {
+          c.add(part[(u * KG + g) * 64 + lane]);
+          c.flush();
+        }
+        finish(c.value(), u);
+      } else {
+        acc_t c = part[(u * KG) * 64 + lane];
+#pragma unroll
+        for (int g = 1; g < KG; ++g) c += part[(u * KG + g) * 64 + lane];
+        finish(c, u);
+      }
     }
   }
 }
 
-template <class EL, int BM, int BN, int WM, int WN, int KG, int S, bool A_KC, bool B_KC, int M, int N, int K, int RB, int CB, bool BATCHED, class Epi, int SPLIT = 1>
+// FOLD > 0: every FOLD K tiles are summed from zero and added to totals, with WIDE to wide ones, FEW sums at a time.
+template <class EL, int BM, int BN, int WM, int WN, int KG, int S, int FOLD, bool WIDE, bool A_KC, bool B_KC, int M, int N, int K, int RB, int CB, bool BATCHED, class Epi, int SPLIT = 1>
 RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typename EL::elem* __restrict__ B, const Epi& epi) {
   typedef typename rx_acc_of<EL>::type acc_t;
   typedef typename rx_acc_of<EL>::scalar acc_s;
@@ -1688,6 +1749,33 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
   for (int i = 0; i < NA; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  // A running sum of all k of a group is rounded once per MFMA (f32 and f64: once per k), and the error of such a chain
+  // grows with its length; totals of short sums keep it at that of the short ones.  2-norm error against 64 bits,
+  // operands uniform in [0, 1), one running sum -> totals: f32 2 x 1024 x 25088 3.0e-7 -> 3.3e-8, 6 x 4096 x 4096 4.2e-7 ->
+  // 3.9e-8 (16.9 -> 18.4 us), 16 x 4096 x 4096 4.2e-7 -> 1.1e-7 (16.6 -> 16.7 us), bf16 with f32 results 2 x 4096 x 4096
+  // 1.5e-7 -> 4.6e-8 (9.4 -> 9.2 us), f64 6 x 4096 x 4096 7.5e-16 -> 6.8e-17 (34.3 -> 34.2 us).
+  constexpr int FEW = KTG <= 16 ? 1 : 4;   // (f32 3 x 4096 x 784, N(0, 1): 1.08e-7 with 1, 1.17e-7 with 4, 1.13e-7 as a reduction)
+  constexpr bool FOLDS = FOLD > 0 && KTG > 1;
+  typename rx_total<acc_t, WIDE>::type tot[FOLDS ? NA : 1][FOLDS ? NB : 1];
+  auto fold = [&]() __attribute__((always_inline)) {
+    if constexpr (FOLDS) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          tot[i][j].add(acc[i][j]);
+          acc[i][j] = acc_t{0, 0, 0, 0};
+        }
+    }
+  };
+  auto flush = [&]() __attribute__((always_inline)) {
+    if constexpr (FOLDS && WIDE) {
+#pragma unroll
+      for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) tot[i][j].flush();
+    }
+  };
   const int idx_a = lane & 15, idx_b = ESZ == 8 ? 4 * (lane & 3) + ((lane & 15) >> 2) : idx_a;
   // dwords of a [row][k] fragment at or past K: only where K is not a whole number of 16-byte chunks
   auto cut = [&](rx_i32x8& f, unsigned kt) {
@@ -1741,21 +1829,46 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
   rx_static_for<0, (SD > 1 ? SD - 1 : 1)>([&](auto I) { issue(decltype(I)::value); });
   constexpr int MAIN = SD > 1 ? KTG - (SD - 1) : 0;   // tiles with a successor to request
   int st = 0;
-  for (int t = 0; t < MAIN; ++t) {
+  // FIRST: the first tile of the next sum.  The one before is added here, when its MFMAs are long done.
+  auto tile = [&](auto FIRST, int t) __attribute__((always_inline)) {
     rx_wait_vmcnt_lgkm0<(SD > 1 ? SD - 2 : 0) * NL>();
     publish();
     issue(st == 0 ? SD - 1 : st - 1);
+    if constexpr (decltype(FIRST)::value != 0) fold();
     compute(st, first + (unsigned)t * STEP);
     st = st + 1 == SD ? 0 : st + 1;
+  };
+  if constexpr (FOLDS) {
+    for (int t = 0; t < MAIN;) {
+      flush();
+      const int end = MAIN - t < FOLD * FEW ? MAIN : t + FOLD * FEW;
+      while (t < end) {
+        const int e = end - t < FOLD ? end : t + FOLD;
+        tile(rx_int<1>{}, t++);
+        if constexpr (FOLD > 1)
+          for (; t < e; ++t) tile(rx_int<0>{}, t);
+      }
+    }
+  } else {
+    for (int t = 0; t < MAIN; ++t) tile(rx_int<0>{}, t);
   }
   rx_static_for<MAIN, KTG>([&](auto T) {
     constexpr int t = decltype(T)::value;
     rx_wait_vmcnt_lgkm0<(KTG - 1 - t) * NL>();
     publish();
+    if constexpr (FOLDS && t % (FOLDS ? FOLD : 1) == 0) fold();
+    if constexpr (FOLDS && t % ((FOLDS ? FOLD : 1) * FEW) == 0) flush();
     compute(t % SD, first + (unsigned)t * STEP);
   });
+  if constexpr (FOLDS) {
+    fold();
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = tot[i][j].value();
+  }
 
-  rx_group_finish<BM, BN, WM, WN, KG, M, N, BATCHED, SPLIT, acc_t, acc_s>(acc, epi, m0, n0, w, grp, lane, (int)batch);
+  rx_group_finish<BM, BN, WM, WN, KG, M, N, BATCHED, SPLIT, WIDE, acc_t, acc_s>(acc, epi, m0, n0, w, grp, lane, (int)batch);
 }
 
 // ===========================================================================
@@ -2038,7 +2151,7 @@ RX_DEV void rx_gemm_body_x(const float* __restrict__ A, const float* __restrict_
       }
     }
   }
-  rx_group_finish<BM, BN, WM, WN, KG, M, N, BATCHED, 1, rx_f32x4v, float>(acc, epi, m0, n0, w, grp, lane, (int)batch);
+  rx_group_finish<BM, BN, WM, WN, KG, M, N, BATCHED, 1, false, rx_f32x4v, float>(acc, epi, m0, n0, w, grp, lane, (int)batch);
 }
 
 // ===========================================================================

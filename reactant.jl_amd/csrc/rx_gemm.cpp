@@ -56,6 +56,27 @@ static GemmChoice choose_gemm_f64(int64_t batch, int64_t M, int64_t N, int64_t K
 // ---------------------------------------------------------------------------
 struct GroupTile { int BM, BN, WM, WN, KG, S, split3 = 0; };   // split3: f32 operands as three bf16 each (rx_gemm_body_x)
 
+// After how many K tiles rx_gemm_body_g adds its sums to totals (0: one running sum per group), and whether those are wide.
+// What took these products otherwise sums shortly: the reduction of products of up to eight rows in parts of 16 to 400 k,
+// the products cut along K (fewer than 256 64 x 64 tiles, K >= 1024) in slices of 512 k and more.  So for up to eight rows
+// sums of 32 k of f32, 16 of f64 and four MFMAs of 16-bit elements go into wide totals, and for the others sums of 512 k
+// into totals of the accumulators' type; no error is larger than that of those plans (f32 3 x 4096 x 784 is closest).
+struct GroupFold { int tiles = 0; bool wide = false; };
+static GroupFold group_fold(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, int split, const GroupTile& t) {
+  const int es = info(dt).size;
+  const int64_t bk = 128 / es, KT = (K + bk - 1) / bk, step = (int64_t)t.KG * split, KTG = (KT + step - 1) / step;
+  GroupFold f;
+  if (t.split3) return f;
+  if (std::min(M, N) <= 8) {
+    f.wide = true;
+    f.tiles = es >= 4 ? 1 : es == 2 ? 2 : 4;
+  } else if (batch == 1 && es <= 4 && ((M + 63) / 64) * ((N + 63) / 64) < 256 && K >= 1024) {
+    f.tiles = (int)(512 / bk);
+  }
+  if (KTG <= (f.wide ? 1 : f.tiles)) f.tiles = 0;
+  return f;
+}
+
 static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t, int64_t* lds) {
   const int es = info(dt).size;
   const int64_t bk = 128 / es, KT = (K + bk - 1) / bk, step = (int64_t)t.KG * split, KTG = (KT + step - 1) / step;
@@ -76,7 +97,9 @@ static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bo
     *lds = std::max<int64_t>((int64_t)t.KG * (t.BM + t.BN) * 192, t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * 4 : 0);
     return *lds + 64 <= 160 * 1024;   // (64: the wavefronts' votes)
   }
-  if (na * nb * (es == 8 ? 8 : 4) + 8 * (na + nb) + 48 > share) return false;
+  const GroupFold fold = group_fold(dt, batch, M, N, K, split, t);
+  const int words = es == 8 ? 8 : 4;   // of an accumulator block
+  if (na * nb * words * (fold.tiles == 0 ? 1 : fold.wide ? 4 : 2) + 8 * (na + nb) + 48 > share) return false;
   const int64_t nl = (t.BM + t.BN) / 8 / NW, sd = std::min<int64_t>(t.S, KTG);
   if (nl * (sd - 1) > 63) return false;                                    // outstanding loads that a wait can count
   const int64_t ring = (int64_t)t.KG * sd * (t.BM + t.BN) * 128, sums = t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * (es == 8 ? 8 : 4) : 0;
@@ -158,7 +181,8 @@ static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t
   std::ostringstream o;
   if (!t.split3) o << el << ", ";
   o << t.BM << ", " << t.BN << ", " << t.WM << ", " << t.WN << ", ";
-  if (!t.split3) o << t.KG << ", " << t.S << ", ";
+  const GroupFold fold = group_fold(dt, batch, M, N, K, split, t);
+  if (!t.split3) o << t.KG << ", " << t.S << ", " << fold.tiles << ", " << (fold.wide ? "true" : "false") << ", ";
   else o << t.KG << ", ";
   o << (a_kc ? "true" : "false") << ", "
     << (b_kc ? "true" : "false") << ", " << M << ", " << N << ", " << K << ", " << rb << ", " << cb;

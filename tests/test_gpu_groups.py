@@ -120,3 +120,24 @@ def test_large_f32_products_take_the_split(rx):
     for (m, n, k, order) in ((4096, 4096, 4096, ORDERS[1]), (2048, 2048, 2048, ORDERS[3]), (2000, 3000, 500, ORDERS[0])):
         assert "rx_gemm_body_x<" in rx.compile_offline(dot_module(m, n, k, "f32", "f32", *order)[0], with_source=True)
     assert "rx_gemm_body_g<" in rx.compile_offline(dot_module(777, 1001, 1531, "f32", "f32", True, False)[0], with_source=True)
+
+
+# A rounding is at most u, and u / sqrt(3) in the mean square, of the sum that it rounds.  Sums of n positive terms from zero
+# are rounded n times, at a third of their square in the mean, and m such sums in one result average out: sqrt(n / 3 m) of that.
+# Up to eight rows: n = 32 (f64 16, 16-bit operands 4 MFMAs), in totals with more bits, fewer than 24 sums nowhere here, and the
+# rounding of the result; the sums of four before them add a third of u: 0.8 u.  More rows: n = 512, m = 8, in totals
+# of the same type: 2.9 u.
+@pytest.mark.parametrize("dt,M,N,K,units", [("f32", 2, 1024, 25088, 0.8), ("f32", 6, 4096, 4096, 0.8), ("f32", 3, 4096, 784, 0.8), ("f32", 1, 2048, 4096, 0.8),
+                                            ("f64", 3, 512, 4096, 0.8), ("f64", 6, 1024, 784, 0.8), ("bf16", 2, 1024, 4096, 0.8), ("bf16", 6, 1000, 25088, 0.8),
+                                            ("f32", 16, 4096, 4096, 2.9)])
+def test_long_sums_of_one_sign(rx, client, monkeypatch, dt, M, N, K, units):
+    """The error of few rows against a matrix does not grow with K (2-norm, operands uniform in [0, 1))."""
+    out = {"bf16": "f32"}.get(dt, dt)
+    text, sa, sb = dot_module(M, N, K, dt, out, True, False)
+    a, b = (I.tensor(np.random.default_rng(s).random(size=z), dt) for s, z in ((9, sa), (10, sb)))
+    got, exe = gpu_run(rx, client, text, [a, b])
+    assert exe.launches()[0]["kind"].startswith("gemm")
+    wide = np.longdouble if dt == "f64" else np.float64
+    exact = a.a.astype(wide) @ b.a.astype(wide)
+    err = np.sqrt(((got[0].a - exact) ** 2).sum() / (exact ** 2).sum())
+    assert err <= 1.25 * units * 2.0 ** (-53 if dt == "f64" else -24), err
