@@ -84,7 +84,8 @@ RX_CHECK_G(rx_check_g_f32_tn, rx_el_f32, float, 16, 64, 1, 1, 4, 4, 1, true, fal
 RX_CHECK_G(rx_check_g_f64_nn, rx_el_f64, double, 32, 32, 2, 1, 2, 2, 1, true, true, false, 96, 96, 100)
 RX_CHECK_G(rx_check_g_bf16_nn, rx_el_bf16, float, 64, 64, 2, 2, 1, 3, 8, false, true, false, 512, 512, 784)
 RX_CHECK_G(rx_check_g_f16_tt, rx_el_f16, float, 32, 64, 1, 2, 4, 2, 0, false, false, true, 64, 64, 128)
-RX_CHECK_G(rx_check_g_f8_nt, rx_el_f8, float, 16, 16, 1, 1, 8, 3, 4, true, true, true, 16, 512, 4096)
+RX_CHECK_G(rx_check_g_f8_nt, rx_el_f8, float, 16, 16, 1, 1, 8, 3, 4, false, true, true, 16, 512, 4096)
+RX_CHECK_G(rx_check_g_f8b_nn, rx_el_f8b, float, 16, 16, 1, 1, 8, 3, 1, true, true, false, 6, 512, 4096)
 
 #define RX_CHECK_X(NAME, BM, BN, WM, WN, KG, AKC, BKC, M, N, K)                                                        \
   extern "C" __global__ __launch_bounds__(WM * WN * KG * 64, 2) void NAME(const float* A, const float* B, float* out) {  \

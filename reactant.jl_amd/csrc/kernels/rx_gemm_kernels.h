@@ -1525,6 +1525,25 @@ struct rx_el_f64 {
     for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f64_16x16x4f64(r.d[j], q.d[j], c, 0, 0, 0);
   }
 };
+// e4m3 operands on the bf16 MFMA: they convert exactly.  The f8 MFMA adds its 128 products with fewer bits than f32 holds; for
+// up to eight rows, which are bound by reading the other operand, the sums are those of f32 (6 x 4096 x 4096, N(0, 80):
+// 2-norm error 3.4e-8 in 8.2 us, 1.5e-5 in 6.0 us on the f8 MFMA, 5.3e-8 in 226 us as a reduction).
+struct rx_el_f8b {
+  typedef rx_u8 elem;
+  static constexpr int NMF = 4;
+  // the eight codes of two dwords
+  RX_DEV rx_bf16x8 wide(rx_u32 a, rx_u32 b) {
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    struct { b2 p[4]; } w = {{__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 1.0f, false), __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(a, 1.0f, true),
+                              __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 1.0f, false), __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 1.0f, true)}};
+    return __builtin_bit_cast(rx_bf16x8, w);
+  }
+  RX_DEV void mma(rx_f32x4v& c, const rx_i32x8& rowop, const rx_i32x8& colop) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wide(rowop[2 * q], rowop[2 * q + 1]), wide(colop[2 * q], colop[2 * q + 1]), c, 0, 0, 0);
+  }
+};
 template <class EL> struct rx_acc_of { typedef rx_f32x4v type; typedef float scalar; };
 template <> struct rx_acc_of<rx_el_f64> { typedef rx_f64x4 type; typedef double scalar; };
 

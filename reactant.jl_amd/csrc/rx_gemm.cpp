@@ -59,7 +59,7 @@ struct GroupTile { int BM, BN, WM, WN, KG, S, split3 = 0; };   // split3: f32 op
 // After how many K tiles rx_gemm_body_g adds its sums to totals (0: one running sum per group), and whether those are wide.
 // What took these products otherwise sums shortly: the reduction of products of up to eight rows in parts of 16 to 400 k,
 // the products cut along K (fewer than 256 64 x 64 tiles, K >= 1024) in slices of 512 k and more.  So for up to eight rows
-// sums of 32 k of f32, 16 of f64 and four MFMAs of 16-bit elements go into wide totals, and for the others sums of 512 k
+// sums of 32 k of f32, 16 of f64 and four MFMAs of narrower elements go into wide totals, and for the others sums of 512 k
 // into totals of the accumulators' type; no error is larger than that of those plans (f32 3 x 4096 x 784 is closest).
 struct GroupFold { int tiles = 0; bool wide = false; };
 static GroupFold group_fold(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, int split, const GroupTile& t) {
@@ -69,7 +69,7 @@ static GroupFold group_fold(DT dt, int64_t batch, int64_t M, int64_t N, int64_t 
   if (t.split3) return f;
   if (std::min(M, N) <= 8) {
     f.wide = true;
-    f.tiles = es >= 4 ? 1 : es == 2 ? 2 : 4;
+    f.tiles = es == 2 ? 2 : 1;
   } else if (batch == 1 && es <= 4 && ((M + 63) / 64) * ((N + 63) / 64) < 256 && K >= 1024) {
     f.tiles = (int)(512 / bk);
   }
@@ -177,7 +177,7 @@ static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t
   c.grid[1] = (unsigned)(split > 1 ? split : batch);
   c.split = split;
   c.est_us = t.split3 ? split3_estimate(batch, M, N, K, t) : group_estimate(dt, batch, M, N, K, a_kc, b_kc, split, t, lds);
-  const std::string el = dt == DT::F64 ? "rx_el_f64" : dt == DT::F32 ? "rx_el_f32" : dt == DT::BF16 ? "rx_el_bf16" : dt == DT::F16 ? "rx_el_f16" : "rx_el_f8";
+  const std::string el = dt == DT::F64 ? "rx_el_f64" : dt == DT::F32 ? "rx_el_f32" : dt == DT::BF16 ? "rx_el_bf16" : dt == DT::F16 ? "rx_el_f16" : std::min(M, N) <= 8 ? "rx_el_f8b" : "rx_el_f8";
   std::ostringstream o;
   if (!t.split3) o << el << ", ";
   o << t.BM << ", " << t.BN << ", " << t.WM << ", " << t.WN << ", ";

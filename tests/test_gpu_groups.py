@@ -141,3 +141,29 @@ def test_long_sums_of_one_sign(rx, client, monkeypatch, dt, M, N, K, units):
     exact = a.a.astype(wide) @ b.a.astype(wide)
     err = np.sqrt(((got[0].a - exact) ** 2).sum() / (exact ** 2).sum())
     assert err <= 1.25 * units * 2.0 ** (-53 if dt == "f64" else -24), err
+
+
+@pytest.mark.parametrize("M,N,K,order", [(6, 4096, 512, (True, True)), (1, 1024, 4096, (True, False)), (1024, 8, 1000, (False, True))])
+def test_e4m3_products_of_few_rows_sum_as_f32(rx, client, M, N, K, order):
+    """2-norm error against 64 bits: four roundings per 128 k of sums of either sign, at half of their square in the mean, and
+    that of the result, each u / sqrt(3) in the mean square: u (the f8 MFMA's sums: 250 u)."""
+    text, sa, sb = dot_module(M, N, K, "f8E4M3FN", "f32", *order)
+    assert "rx_el_f8b" in rx.compile_offline(text, with_source=True)
+    a, b = (I.tensor(np.clip(np.random.default_rng(s).normal(size=z) * 80, -448, 448), "f8E4M3FN") for s, z in ((11, sa), (12, sb)))
+    got, _ = gpu_run(rx, client, text, [a, b])
+    x, y = a.a.astype(np.float64), b.a.astype(np.float64)
+    exact = (x if order[0] else x.T) @ (y.T if order[1] else y)
+    err = np.sqrt(((got[0].a - exact) ** 2).sum() / (exact ** 2).sum())
+    assert err <= 1.5 * 2.0 ** -24, err
+
+
+def test_every_e4m3_code_of_a_matrix_against_a_row(rx, client):
+    """Row n holds code n mod 256 alone, at k = n: its product with ones is the code's value, NaN where that is."""
+    N, K = 1024, 1024
+    text, sa, sb = dot_module(1, N, K, "f8E4M3FN", "f32", True, True)
+    assert "rx_el_f8b" in rx.compile_offline(text, with_source=True)
+    w = np.zeros((N, K), dtype=np.uint8)
+    w[np.arange(N), np.arange(N)] = np.arange(N) % 256
+    b = I.Tensor.from_bytes(w.tobytes(), "f8E4M3FN", sb)
+    got, _ = gpu_run(rx, client, text, [I.tensor(np.ones(sa), "f8E4M3FN"), b])
+    assert np.array_equal(got[0].a[0], b.a[np.arange(N), np.arange(N)], equal_nan=True)
