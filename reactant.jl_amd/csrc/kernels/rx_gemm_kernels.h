@@ -1901,8 +1901,12 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
 // 2.2e-7) and 5.7e-7, 2000 x 3000 x 500 1.5e-7 and 4.0e-7.
 // Two kinds of input do not split: an infinity (and a finite number that rounds to one) leaves inf - inf, so its
 // products become NaN; a number below 2^-102 may have bits below 2^-133, the last that bf16 holds.  The first is seen in the
-// result, which is not finite; the second while splitting, x - h - m being subnormal and not zero.  A workgroup that
-// sees either contracts its tile again with f32 MFMAs.
+// result, which is not finite; the second while splitting, x - h - m being subnormal and not zero.  A workgroup that sees
+// the first contracts its tile again with f32 MFMAs.  One that sees the second does so only if a sum is so small that the
+// lost bits may show in it (magnitudes from a second look at the operands; a few sums, which cancelled, are contracted one
+// by one): exp(-x) beside ordinary numbers costs that look alone.  4096^3, 8192 x 4096 x 1024 and 2048^3: 634, 331 and 91
+// us, 745, 407 and 120 with such numbers in every tile, 1663, 848 and 225 contracted again in every tile (the f32 MFMA
+// bodies: 955, 545, 139).
 //
 // Time: six 16 x 16 x 32 bf16 MFMAs take 96 cycles of the matrix pipe where eight 16 x 16 x 4 f32 MFMAs take 256.  What bounds
 // it is the sum of the MFMAs and the vector instructions (per element 5.5 to split it and one to test it, and four per
@@ -2036,7 +2040,7 @@ RX_DEV void rx_gemm_body_x(const float* __restrict__ A, const float* __restrict_
   static_assert((A_KC || ((long long)K + 64 * STEP) * M * 4 < (1ll << 32)) && (B_KC || ((long long)K + 64 * STEP) * N * 4 < (1ll << 32)), "offsets of the last groups' K tiles");
   constexpr int STAGE = (BM + BN) * 192;
   extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
-  __shared__ int again[16];
+  __shared__ int again[16], largest[2];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int grp = wave / NW, w = wave % NW, wm = w / WN, wn = w % WN, t = tid - grp * NT;
   RX_LDS rx_u8* const lds = (RX_LDS rx_u8*)rx_smem + grp * STAGE;
@@ -2145,20 +2149,86 @@ RX_DEV void rx_gemm_body_x(const float* __restrict__ A, const float* __restrict_
     for (int j = 0; j < NB; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) fin = __builtin_fmaf(acc[i][j][q], 0.f, fin);
-  const bool mine = __builtin_amdgcn_ballot_w64(odd || fin != fin) != 0;
-  if (lane == 0) again[wave] = mine;
-  __syncthreads();
-  int any = 0;
+  // votes of the workgroup: 2 contracts again, 1 does if that is of consequence
+  auto vote = [&](bool must, bool may) __attribute__((always_inline)) {
+    const int mine = __builtin_amdgcn_ballot_w64(must) != 0 ? 2 : (__builtin_amdgcn_ballot_w64(may) != 0 ? 1 : 0);
+    if (lane == 0) again[wave] = mine;
+    __syncthreads();
+    int any = 0;
 #pragma unroll
-  for (int u = 0; u < NW * KG; ++u) any |= again[u];
-  if (__builtin_amdgcn_readfirstlane(any)) {
-    clear();
+    for (int u = 0; u < NW * KG; ++u) any |= again[u];
+    return __builtin_amdgcn_readfirstlane(any);
+  };
+  if (tid < 2) largest[tid] = 0;
+  int any = vote(fin != fin, odd);
+  if (any == 1) {
+    // An element's three parts are off by 2^-134 at most, a sum by K 2^-134 (max |a| + max |b|).  That is below half a rounding
+    // of a sum whose magnitude is K 2^-109 of these maxima: read the operands once more for them.
+    float la = 0.f, lb = 0.f;
+    load(0);
     for (int i = 0; i < KTG; ++i) {
-      load(i);
+      rx_static_for<0, OA::NV>([&](auto Q) {
+        constexpr int q = decltype(Q)::value;
+        int o, k;
+        const rx_f32x4v v = OA::quad(va, q, t, kt_of(i), &o, &k);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) la = __builtin_fmaxf(la, __builtin_fabsf(v[d]));
+        if constexpr (A_KC || q % 4 == 3) OA::template load<A_KC ? q : q - 3, A_KC ? 1 : 4>(va, ra, m0, t, kt_of(i + 1));
+      });
+      rx_static_for<0, OB::NV>([&](auto Q) {
+        constexpr int q = decltype(Q)::value;
+        int o, k;
+        const rx_f32x4v v = OB::quad(vb, q, t, kt_of(i), &o, &k);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) lb = __builtin_fmaxf(lb, __builtin_fabsf(v[d]));
+        if constexpr (B_KC || q % 4 == 3) OB::template load<B_KC ? q : q - 3, B_KC ? 1 : 4>(vb, rb, n0, t, kt_of(i + 1));
+      });
+    }
+    // (magnitudes are ordered as their bits are)
+    __hip_atomic_fetch_max(&largest[0], __builtin_bit_cast(int, la), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_max(&largest[1], __builtin_bit_cast(int, lb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    const float least = (__builtin_bit_cast(float, largest[0]) + __builtin_bit_cast(float, largest[1])) * ((float)K * 0x1p-109f);
+    static_assert(NA * NB * 4 <= 64, "a bit per sum");
+    unsigned long long low = 0;
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        const int m = m0 + wm * (BM / WM) + 16 * i + (lane & 15), n = n0 + wn * (BN / WN) + 16 * j + 4 * (lane >> 4);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) low |= (unsigned long long)(m < M && n + q < N && !(__builtin_fabsf(acc[i][j][q]) >= least)) << ((i * NB + j) * 4 + q);
+      }
+    // Ordinary terms cancel to as little, or to nothing, here and there: a few sums of a wavefront are contracted one by one.
+    any = vote(__builtin_popcountll(__builtin_amdgcn_ballot_w64(low != 0)) > 4 || (low & (low - 1)) != 0, false);
+    if (any == 0)
+      for (unsigned long long todo = __builtin_amdgcn_ballot_w64(low != 0); todo != 0; todo &= todo - 1) {
+        const int from = __builtin_ctzll(todo);
+        const int e = __builtin_amdgcn_readlane(low ? __builtin_ctzll(low) : 0, from);
+        const int m = m0 + wm * (BM / WM) + 16 * (e / (4 * NB)) + (from & 15), n = n0 + wn * (BN / WN) + 16 * (e / 4 % NB) + 4 * (from >> 4) + e % 4;
+        float s = 0.f;
+        for (int i = lane >> 5; i < KTG; i += 2) {
+          const unsigned k = kt_of(i) * 32 + (lane & 31);
+          const unsigned oa = A_KC ? (unsigned)m * (unsigned)K + k : k * (unsigned)M + (unsigned)m, ob = B_KC ? (unsigned)n * (unsigned)K + k : k * (unsigned)N + (unsigned)n;
+          const unsigned past = 0xfffffff0u;   // of the operand: zero
+          s = __builtin_fmaf(__builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(ra, k < (unsigned)K ? oa * 4 : past, 0, 0)),
+                             __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, k < (unsigned)K ? ob * 4 : past, 0, 0)), s);
+        }
+        s = rx_wave_reduce(s, rx_op_add());
+#pragma unroll
+        for (int u = 0; u < NA * NB * 4; ++u)
+          if (u == e && lane == from) acc[u / (4 * NB)][u / 4 % NB][u % 4] = s;
+      }
+  }
+  if (any & 2) {
+    clear();
+    load(0);
+    for (int i = 0; i < KTG; ++i) {
       __syncthreads();
       OA::put_f32(va, lds, t, kt_of(i));
       OB::put_f32(vb, lds + BM * 192, t, kt_of(i));
       __syncthreads();
+      load(i + 1);
       rx_i32x8 fb[NB];
 #pragma unroll
       for (int j = 0; j < NB; ++j) fb[j] = OB::frag_f32(lds + BM * 192, wn * (BN / WN) + 16 * j, lane);

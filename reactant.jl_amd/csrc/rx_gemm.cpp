@@ -95,7 +95,7 @@ static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bo
     if (dt != DT::F32 || split > 1 || t.BM % 32 || t.BN % 32 || t.BM * (a_kc ? 8 : 2) % nt || t.BN * (b_kc ? 8 : 2) % nt) return false;
     if (na * nb * 4 + 10 * nv + 12 * (nb + 1) + 40 > std::min(share, 256)) return false;   // two wavefronts per SIMD
     *lds = std::max<int64_t>((int64_t)t.KG * (t.BM + t.BN) * 192, t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * 4 : 0);
-    return *lds + 64 <= 160 * 1024;   // (64: the wavefronts' votes)
+    return *lds + 128 <= 160 * 1024;   // (128: the wavefronts' votes and the operands' largest magnitudes)
   }
   const GroupFold fold = group_fold(dt, batch, M, N, K, split, t);
   const int words = es == 8 ? 8 : 4;   // of an accumulator block

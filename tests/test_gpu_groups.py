@@ -167,3 +167,53 @@ def test_every_e4m3_code_of_a_matrix_against_a_row(rx, client):
     b = I.Tensor.from_bytes(w.tobytes(), "f8E4M3FN", sb)
     got, _ = gpu_run(rx, client, text, [I.tensor(np.ones(sa), "f8E4M3FN"), b])
     assert np.array_equal(got[0].a[0], b.a[np.arange(N), np.arange(N)], equal_nan=True)
+
+
+BIG_X_TILES = ["128,128,2,2,1,1,1", "128,128,2,2,2,1,1", "128,256,2,4,1,1,1", "256,128,4,2,1,1,1"]
+
+
+@pytest.mark.parametrize("tile,order,batch", [(t, [o for o in ORDERS if x_fits(t, o)][j], 3 * j) for t in BIG_X_TILES for j in (0, 1)])
+def test_tiny_numbers_where_they_matter_and_where_not(rx, client, monkeypatch, tile, order, batch):
+    """Numbers with bits below what bf16 holds, in a product of several tiles and many K tiles: beside numbers of ordinary size
+    they change nothing and no tile is contracted again (the same bits as with numbers that do split in their place); rows
+    and columns of nothing else come out as exactly as all others."""
+    M, N, K = 300, 290, 1030
+    text, sa, sb = dot_module(M, N, K, "f32", "f32", *order, batch)
+    monkeypatch.setenv("RX_GEMM_G", tile)
+    monkeypatch.setenv("RX_SPLIT_K", "0")
+    assert "rx_gemm_body_x<" in rx.compile_offline(text, with_source=True)
+    rng = np.random.default_rng(13)
+    lead = (batch,) if batch else ()
+    A, B = rng.normal(size=lead + (M, K)).astype(np.float32), rng.normal(size=lead + (N, K)).astype(np.float32)
+
+    def run(a, b):
+        a, b = (np.ascontiguousarray(x if kc else np.swapaxes(x, -1, -2)) for x, kc in ((a, order[0]), (b, order[1])))
+        return gpu_run(rx, client, text, [I.Tensor(a, "f32"), I.Tensor(b, "f32")])[0][0].a.copy()
+
+    a0, a1, b0, b1 = A.copy(), A.copy(), B.copy(), B.copy()
+    for x0, x1 in ((a0, a1), (b0, b1)):
+        x0[..., ::40, 7], x1[..., ::40, 7] = np.float32(1.2345678e-33), np.float32(2.0 ** -109)
+        x0[..., 5, 1029], x1[..., 5, 1029] = np.float32(-1e-41), 0
+    # one sum whose ordinary terms cancel, in the K tiles of either of two groups
+    b0[..., 70, :] = b1[..., 70, :] = 0
+    for x in (a0, a1):
+        x[..., 60, [0, 1, 32, 33]] = 3, -3, 5, -5
+        x[..., 60, 9] = np.float32(1.2345678e-33) if x is a0 else 0
+    for x in (b0, b1):
+        x[..., 70, [0, 1, 9, 32, 33]] = 1
+    one, two = run(a0, b0), run(a1, b1)
+    assert (one[..., 60, 70] == np.float32(1.2345678e-33)).all() and (two[..., 60, 70] == 0).all()
+    two[..., 60, 70] = one[..., 60, 70]
+    assert np.array_equal(one, two)
+    a0[..., 20:24, :] *= np.float32(1e-36)
+    a0[..., 290, :] *= np.float32(1e-40)
+    b0[..., 150, :] *= np.float32(1e-35)
+    b0[..., 40, :] = 0
+    got = run(a0, b0).astype(np.float64)
+    exact = np.matmul(a0.astype(np.float64), np.swapaxes(b0, -1, -2).astype(np.float64))
+    bound = np.matmul(np.abs(a0).astype(np.float64), np.swapaxes(np.abs(b0), -1, -2).astype(np.float64))
+    # one rounding per product where a tile is contracted in f32, and K 2^-149 for sums that are subnormal
+    assert (np.abs(got - exact) <= bound * (K + 2) * 2.0 ** -24 + K * 2.0 ** -149).all()
+    a0[..., 299, 3] = np.inf
+    got = run(a0, b0)
+    assert not np.isfinite(got[..., 299, :]).any() and np.isfinite(got[..., :299, :]).all()
