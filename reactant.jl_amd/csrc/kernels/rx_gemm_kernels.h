@@ -1716,6 +1716,7 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
   constexpr unsigned KBYTES = (unsigned)K * ESZ, A_LDB = (A_KC ? K : M) * ESZ, B_LDB = (B_KC ? K : N) * ESZ;
   constexpr int KT = (K + BK - 1) / BK, STEP = KG * SPLIT, KTG = (KT + STEP - 1) / STEP;   // K tiles, and per group
   constexpr int SD = KTG < S ? KTG : S;
+  static_assert(SD > 1 || KTG == 1, "a stage to read and one to load");
   constexpr bool SEL = KBYTES % (BKB * STEP) != 0;   // some group's last K tile reaches past K
   extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

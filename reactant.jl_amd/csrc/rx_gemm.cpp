@@ -100,6 +100,7 @@ static bool group_fits(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bo
   const GroupFold fold = group_fold(dt, batch, M, N, K, split, t);
   const int words = es == 8 ? 8 : 4;   // of an accumulator block
   if (na * nb * words * (fold.tiles == 0 ? 1 : fold.wide ? 4 : 2) + 8 * (na + nb) + 48 > share) return false;
+  if (t.S < 2 && KTG > 1) return false;                                    // a stage to read and one to load
   const int64_t nl = (t.BM + t.BN) / 8 / NW, sd = std::min<int64_t>(t.S, KTG);
   if (nl * (sd - 1) > 63) return false;                                    // outstanding loads that a wait can count
   const int64_t ring = (int64_t)t.KG * sd * (t.BM + t.BN) * 128, sums = t.KG > 1 ? (int64_t)t.KG * t.BM * t.BN * (es == 8 ? 8 : 4) : 0;

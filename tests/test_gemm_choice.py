@@ -24,3 +24,13 @@ def test_f32_products_of_a_tall_matrix_compile(tall, other, k):
 def test_f32_products_past_the_offset_bound_compile():
     assert skeleton(8_388_608, 128, 64, "f32", "f32", False, True) not in (None, "rx_gemm_body_x", "rx_gemm_body_g")
     assert skeleton(128, 8_388_608, 64, "f32", "f32", True, False) not in (None, "rx_gemm_body_x", "rx_gemm_body_g")
+
+
+def test_one_stage_serves_one_tile(monkeypatch):
+    """A tile asked for with one LDS stage is refused (the planner's own is taken) where a group has more than one K tile."""
+    def text(k, spec):
+        monkeypatch.setenv("RX_GEMM_G", spec)
+        return rx.compile_offline(dot_module(256, 256, k, "f32", "f32", True, True)[0], with_source=True)
+    assert "rx_gemm_body_g<rx_el_f32, 64, 64, 2, 2, 1, 1, " not in text(512, "64,64,2,2,1,1")
+    assert "rx_gemm_body_g<rx_el_f32, 64, 64, 2, 2, 1, 2, " in text(512, "64,64,2,2,1,2")
+    assert "rx_gemm_body_g<rx_el_f32, 64, 64, 2, 2, 2, 1, " in text(64, "64,64,2,2,2,1")
