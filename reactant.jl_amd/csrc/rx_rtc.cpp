@@ -75,12 +75,22 @@ struct Fd {
   ~Fd() { if (fd >= 0) close(fd); }
 };
 
-// Source and result pass through anonymous files, so neither side waits for the other while it writes.
+// An anonymous file, above the descriptors that the worker's process uses.
+int anonymous_file(const char* name) {
+  const int fd = memfd_create(name, MFD_CLOEXEC);
+  if (fd < 0) return -1;
+  const int up = fcntl(fd, F_DUPFD_CLOEXEC, kWorkerResult + 1);
+  close(fd);
+  return up;
+}
+
+// Source and result pass through anonymous files, so neither side waits for the other while it writes.  The result has a
+// descriptor of its own: a library that is preloaded into every process may write to standard output.
 // True: the worker ran and *code / *error is its answer.  False: it could not be started or did not finish.
 bool worker_compile(const std::string& source, const std::string& arch, std::string* code, std::string* error) {
   Fd in, out;
-  in.fd = memfd_create("rx_source", MFD_CLOEXEC);
-  out.fd = memfd_create("rx_code", MFD_CLOEXEC);
+  in.fd = anonymous_file("rx_source");
+  out.fd = anonymous_file("rx_code");
   if (in.fd < 0 || out.fd < 0) return false;
   for (size_t at = 0; at < source.size();) {
     const ssize_t n = write(in.fd, source.data() + at, source.size() - at);
@@ -92,8 +102,9 @@ bool worker_compile(const std::string& source, const std::string& arch, std::str
   posix_spawn_file_actions_t fa;
   if (posix_spawn_file_actions_init(&fa) != 0) return false;
   posix_spawn_file_actions_adddup2(&fa, in.fd, 0);
-  posix_spawn_file_actions_adddup2(&fa, out.fd, 1);
-  posix_spawn_file_actions_addclosefrom_np(&fa, 3);
+  posix_spawn_file_actions_adddup2(&fa, out.fd, kWorkerResult);
+  posix_spawn_file_actions_addopen(&fa, 1, "/dev/null", O_WRONLY, 0);
+  posix_spawn_file_actions_addclosefrom_np(&fa, kWorkerResult + 1);
   const char* argv[] = {worker_path().c_str(), arch.c_str(), nullptr};
   pid_t pid = -1;
   const int rc = posix_spawn(&pid, argv[0], &fa, nullptr, const_cast<char**>(argv), environ);
@@ -138,6 +149,10 @@ std::string rtc_compile(const std::string& source, const std::string& arch) {
       if (f) { fputs(source.c_str(), f); fclose(f); }
     }
     throw Error(error);
+  }
+  if (const char* e = getenv("RX_DUMP_CODE_OBJECT")) {
+    FILE* f = fopen(e, "wb");
+    if (f) { fwrite(code.data(), 1, code.size(), f); fclose(f); }
   }
   return code;
 }

@@ -9,6 +9,8 @@
 
 namespace rx {
 
+constexpr int kWorkerResult = 3;   // the descriptor that the worker writes its answer to
+
 // 0 and the code object, or non-zero and the error text.
 static int hiprtc_compile(const std::string& source, const std::string& arch, std::string* out) {
   hiprtcProgram prog;

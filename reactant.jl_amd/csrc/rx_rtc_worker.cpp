@@ -1,5 +1,5 @@
 // Compiles one kernel text in a process of its own: source on standard input, architecture as the argument, the code
-// object (exit status 0) or the error text (1) on standard output.  Started by rx_rtc.cpp; touches no GPU.
+// object (exit status 0) or the error text (1) on descriptor kWorkerResult.  Started by rx_rtc.cpp; touches no GPU.
 #include <unistd.h>
 
 #include <cerrno>
@@ -19,7 +19,7 @@ int main(int argc, char** argv) {
   }
   const int rc = rx::hiprtc_compile(source, argv[1], &out);
   for (size_t at = 0; at < out.size();) {
-    const ssize_t n = write(1, out.data() + at, out.size() - at);
+    const ssize_t n = write(rx::kWorkerResult, out.data() + at, out.size() - at);
     if (n < 0 && errno == EINTR) continue;
     if (n <= 0) return 2;
     at += (size_t)n;
