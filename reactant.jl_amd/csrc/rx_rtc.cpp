@@ -86,7 +86,8 @@ int anonymous_file(const char* name) {
 
 // Source and result pass through anonymous files, so neither side waits for the other while it writes.  The result has a
 // descriptor of its own: a library that is preloaded into every process may write to standard output.
-// True: the worker ran and *code / *error is its answer.  False: it could not be started or did not finish.
+// True: *code / *error is the worker's answer.  False: it could not be started or did not finish.  That is read off the result's
+// last bytes, not the exit status, which a process that ignores SIGCHLD or waits for any child does not get to see.
 bool worker_compile(const std::string& source, const std::string& arch, std::string* code, std::string* error) {
   Fd in, out;
   in.fd = anonymous_file("rx_source");
@@ -110,12 +111,11 @@ bool worker_compile(const std::string& source, const std::string& arch, std::str
   const int rc = posix_spawn(&pid, argv[0], &fa, nullptr, const_cast<char**>(argv), environ);
   posix_spawn_file_actions_destroy(&fa);
   if (rc != 0) return false;
-  int status = 0;
-  while (waitpid(pid, &status, 0) < 0)
-    if (errno != EINTR) return false;
-  if (!WIFEXITED(status) || WEXITSTATUS(status) > 1) return false;   // 0: a code object, 1: an error text
+  // fails with ECHILD once the worker has ended if its status went elsewhere
+  while (waitpid(pid, nullptr, 0) < 0)
+    if (errno != EINTR) break;
   struct stat st;
-  if (fstat(out.fd, &st) != 0 || st.st_size <= 0) return false;
+  if (fstat(out.fd, &st) != 0 || st.st_size < (off_t)sizeof(WorkerEnd)) return false;
   std::string got((size_t)st.st_size, '\0');
   for (size_t at = 0; at < got.size();) {
     const ssize_t n = pread(out.fd, &got[at], got.size() - at, (off_t)at);
@@ -123,7 +123,11 @@ bool worker_compile(const std::string& source, const std::string& arch, std::str
     if (n <= 0) return false;
     at += (size_t)n;
   }
-  (WEXITSTATUS(status) == 0 ? *code : *error) = std::move(got);
+  WorkerEnd end;
+  got.copy((char*)&end, sizeof(end), got.size() - sizeof(end));
+  got.resize(got.size() - sizeof(end));
+  if (end.magic != kWorkerMagic || end.length != got.size() || end.status > 1) return false;
+  (end.status == 0 ? *code : *error) = std::move(got);
   return true;
 }
 

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hiprtc.h>
 
+#include <cstdint>
 #include <string>
 #include <vector>
 
@@ -10,6 +11,9 @@
 namespace rx {
 
 constexpr int kWorkerResult = 3;   // the descriptor that the worker writes its answer to
+// What follows the answer, a code object (status 0) or an error text (1).
+struct WorkerEnd { uint64_t magic, status, length; };
+constexpr uint64_t kWorkerMagic = 0x5258525443454e44;
 
 // 0 and the code object, or non-zero and the error text.
 static int hiprtc_compile(const std::string& source, const std::string& arch, std::string* out) {

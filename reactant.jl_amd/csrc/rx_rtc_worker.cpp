@@ -1,5 +1,5 @@
 // Compiles one kernel text in a process of its own: source on standard input, architecture as the argument, the code
-// object (exit status 0) or the error text (1) on descriptor kWorkerResult.  Started by rx_rtc.cpp; touches no GPU.
+// object or the error text and a WorkerEnd on descriptor kWorkerResult.  Started by rx_rtc.cpp; touches no GPU.
 #include <unistd.h>
 
 #include <cerrno>
@@ -17,7 +17,9 @@ int main(int argc, char** argv) {
     if (n == 0) break;
     source.append(buf, (size_t)n);
   }
-  const int rc = rx::hiprtc_compile(source, argv[1], &out);
+  const int rc = rx::hiprtc_compile(source, argv[1], &out) == 0 ? 0 : 1;
+  const rx::WorkerEnd end = {rx::kWorkerMagic, (uint64_t)rc, out.size()};
+  out.append((const char*)&end, sizeof(end));
   for (size_t at = 0; at < out.size();) {
     const ssize_t n = write(rx::kWorkerResult, out.data() + at, out.size() - at);
     if (n < 0 && errno == EINTR) continue;

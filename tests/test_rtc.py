@@ -55,3 +55,9 @@ def test_a_preloaded_library_that_prints(tmp_path, want):
     got, err = _code(tmp_path, "import torch", LD_PRELOAD=":".join([str(lib)] + os.environ.get("LD_PRELOAD", "").split()))
     assert "rx_rtc_worker" not in err
     assert got == want
+
+
+def test_a_process_that_ignores_its_children(tmp_path, want):
+    got, err = _code(tmp_path, "import torch, signal; signal.signal(signal.SIGCHLD, signal.SIG_IGN)")
+    assert "rx_rtc_worker" not in err
+    assert got == want
