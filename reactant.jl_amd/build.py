@@ -91,7 +91,8 @@ def build_library(force=False, verbose=True):
     # the compiler's process (csrc/rx_rtc_worker.cpp): its hiprtc comes from ROCM_LIB whatever the environment's library path says
     src = os.path.join(CSRC, "rx_rtc_worker.cpp")
     if force or _stale(WORKER, [src] + headers):
-        _run([os.environ.get("CXX", "/opt/rocm/lib/llvm/bin/clang++"), "-std=c++17", "-O2", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", src,
+        _run([os.environ.get("CXX", "/opt/rocm/lib/llvm/bin/clang++"), "-std=c++17", "-O2", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+              '-DRX_ROCM_LIB="%s"' % ROCM_LIB, src,
               "-o", WORKER, "-L" + ROCM_LIB, "-lhiprtc", "-Wl,--disable-new-dtags,-rpath," + ROCM_LIB])
     return LIB
 

@@ -11,8 +11,6 @@
 #include "rx_rtc.h"
 
 #include <fcntl.h>
-#include <limits.h>
-#include <link.h>
 #include <spawn.h>
 #include <sys/mman.h>
 #include <sys/stat.h>
@@ -21,6 +19,7 @@
 
 #include <dlfcn.h>
 
+#include <algorithm>
 #include <cerrno>
 #include <cstdio>
 #include <cstdlib>
@@ -30,34 +29,32 @@
 #include "rx_ir.h"
 #include "rx_rtc_hiprtc.h"
 
-#ifndef RX_ROCM_LIB
-#define RX_ROCM_LIB "/opt/rocm/lib"
-#endif
-
 extern char** environ;
 
 namespace rx {
 namespace {
 
-std::string real_dir(const char* path) {
-  char buf[PATH_MAX];
-  const std::string p = realpath(path, buf) ? buf : path;
-  const size_t s = p.rfind('/');
-  return s == std::string::npos ? std::string(".") : p.substr(0, s);
-}
-
-// Has a hiprtc or a comgr from elsewhere than RX_ROCM_LIB been loaded into this process?
-bool foreign_compiler_loaded() {
-  static const std::string own = real_dir(RX_ROCM_LIB "/libhiprtc.so");
-  bool foreign = false;
-  dl_iterate_phdr(
-      [](struct dl_phdr_info* i, size_t, void* f) {
-        const char* base = i->dlpi_name ? strrchr(i->dlpi_name, '/') : nullptr;
-        if (base && (!strncmp(base, "/libhiprtc.so", 13) || !strncmp(base, "/libamd_comgr.so", 16)) && real_dir(i->dlpi_name) != own) *(bool*)f = true;
-        return 0;
-      },
-      &foreign);
-  return foreign;
+// The worker's environment: without another ROCm's libraries (LD_LIBRARY_PATH, which goes before the path that hiprtc looks for
+// comgr on; entries of LD_PRELOAD that are one of ROCm's), and without what makes a profiler's library start the GPU.
+std::vector<std::string> worker_environment() {
+  std::vector<std::string> env;
+  auto starts = [](const std::string& s, const char* p) { return s.compare(0, strlen(p), p) == 0; };
+  for (char** e = environ; *e; ++e) {
+    const std::string v = *e;
+    if (starts(v, "LD_LIBRARY_PATH=") || starts(v, "ROCP_") || starts(v, "ROCPROF") || starts(v, "ROCTRACER_") || starts(v, "HSA_TOOLS_")) continue;
+    if (!starts(v, "LD_PRELOAD=")) { env.push_back(v); continue; }
+    std::string kept;
+    for (size_t at = strlen("LD_PRELOAD="); at < v.size();) {
+      const size_t end = std::min(v.find_first_of(": ", at), v.size());
+      const std::string lib = v.substr(at, end - at), base = lib.substr(lib.rfind('/') + 1);
+      bool rocm = lib.empty();
+      for (const char* p : {"libamd_comgr", "libhiprtc", "libamdhip64", "libhsa-runtime64", "librocprof", "libroctracer", "libroctx"}) rocm = rocm || starts(base, p);
+      if (!rocm) kept += (kept.empty() ? "" : ":") + lib;
+      at = end + 1;
+    }
+    if (!kept.empty()) env.push_back("LD_PRELOAD=" + kept);
+  }
+  return env;
 }
 
 // The worker lies beside this library.
@@ -108,7 +105,11 @@ bool worker_compile(const std::string& source, const std::string& arch, std::str
   posix_spawn_file_actions_addclosefrom_np(&fa, kWorkerResult + 1);
   const char* argv[] = {worker_path().c_str(), arch.c_str(), nullptr};
   pid_t pid = -1;
-  const int rc = posix_spawn(&pid, argv[0], &fa, nullptr, const_cast<char**>(argv), environ);
+  std::vector<std::string> env = worker_environment();
+  std::vector<char*> envp;
+  for (std::string& v : env) envp.push_back(&v[0]);
+  envp.push_back(nullptr);
+  const int rc = posix_spawn(&pid, argv[0], &fa, nullptr, const_cast<char**>(argv), envp.data());
   posix_spawn_file_actions_destroy(&fa);
   if (rc != 0) return false;
   // fails with ECHILD once the worker has ended if its status went elsewhere

@@ -1,6 +1,11 @@
 // One compilation with the hiprtc that this program or library is linked to (rx_rtc.cpp and rx_rtc_worker.cpp).
 #pragma once
 #include <hip/hiprtc.h>
+#include <limits.h>
+#include <link.h>
+
+#include <cstdlib>
+#include <cstring>
 
 #include <cstdint>
 #include <string>
@@ -8,7 +13,32 @@
 
 #include "rx_embedded.inc"
 
+#ifndef RX_ROCM_LIB
+#define RX_ROCM_LIB "/opt/rocm/lib"
+#endif
+
 namespace rx {
+
+static std::string real_dir(const char* path) {
+  char buf[PATH_MAX];
+  const std::string p = realpath(path, buf) ? buf : path;
+  const size_t s = p.rfind('/');
+  return s == std::string::npos ? std::string(".") : p.substr(0, s);
+}
+
+// Has a hiprtc or a comgr from elsewhere than RX_ROCM_LIB been loaded into this process?
+static bool foreign_compiler_loaded() {
+  static const std::string own = real_dir(RX_ROCM_LIB "/libhiprtc.so");
+  bool foreign = false;
+  dl_iterate_phdr(
+      [](struct dl_phdr_info* i, size_t, void* f) {
+        const char* base = i->dlpi_name ? strrchr(i->dlpi_name, '/') : nullptr;
+        if (base && (!strncmp(base, "/libhiprtc.so", 13) || !strncmp(base, "/libamd_comgr.so", 16)) && real_dir(i->dlpi_name) != own) *(bool*)f = true;
+        return 0;
+      },
+      &foreign);
+  return foreign;
+}
 
 constexpr int kWorkerResult = 3;   // the descriptor that the worker writes its answer to
 // What follows the answer, a code object (status 0) or an error text (1).

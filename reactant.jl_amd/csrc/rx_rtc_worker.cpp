@@ -1,5 +1,6 @@
 // Compiles one kernel text in a process of its own: source on standard input, architecture as the argument, the code
 // object or the error text and a WorkerEnd on descriptor kWorkerResult.  Started by rx_rtc.cpp; touches no GPU.
+// Ends without an answer where another ROCm's compiler was loaded into it all the same.
 #include <unistd.h>
 
 #include <cerrno>
@@ -18,6 +19,7 @@ int main(int argc, char** argv) {
     source.append(buf, (size_t)n);
   }
   const int rc = rx::hiprtc_compile(source, argv[1], &out) == 0 ? 0 : 1;
+  if (rx::foreign_compiler_loaded()) return 2;
   const rx::WorkerEnd end = {rx::kWorkerMagic, (uint64_t)rc, out.size()};
   out.append((const char*)&end, sizeof(end));
   for (size_t at = 0; at < out.size();) {

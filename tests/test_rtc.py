@@ -61,3 +61,16 @@ def test_a_process_that_ignores_its_children(tmp_path, want):
     got, err = _code(tmp_path, "import torch, signal; signal.signal(signal.SIGCHLD, signal.SIG_IGN)")
     assert "rx_rtc_worker" not in err
     assert got == want
+
+
+@pytest.mark.parametrize("how", ["LD_PRELOAD", "LD_LIBRARY_PATH"])
+def test_another_compiler_in_the_environment(tmp_path, want, how):
+    """The child compiles with neither (with that comgr the code object is another one)."""
+    import torch
+    lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    value = [os.path.join(lib, "libamd_comgr.so")] if how == "LD_PRELOAD" else [lib]
+    if not os.path.exists(os.path.join(lib, "libamd_comgr.so")):
+        pytest.skip("this torch brings no comgr")
+    got, err = _code(tmp_path, "import torch", **{how: ":".join(value + os.environ.get(how, "").split(":")).rstrip(":")})
+    assert "rx_rtc_worker" not in err
+    assert got == want
