@@ -158,6 +158,14 @@ static double split3_estimate(int64_t batch, int64_t M, int64_t N, int64_t K, co
   return 8.0 + (double)kt * ((double)(n / 2) * 2.75 + (double)(n % 2) * 1.6) * area;
 }
 
+// The most tiles that one of the eight XCDs takes of a gm x gn grid walked in blocks of rb x cb (rx_gemm_tile).
+static int64_t xcd_tiles(int64_t gm, int64_t gn, int64_t rb, int64_t cb) {
+  int64_t load[8] = {}, blk = 0;
+  for (int64_t r = 0; r < gm; r += rb)
+    for (int64_t c = 0; c < gn; c += cb) load[blk++ % 8] += std::min(rb, gm - r) * std::min(cb, gn - c);
+  return *std::max_element(load, load + 8);
+}
+
 static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc, int split, const GroupTile& t) {
   GemmChoice c;
   int64_t lds = 0;
@@ -171,6 +179,15 @@ static GemmChoice group_gemm(DT dt, int64_t batch, int64_t M, int64_t N, int64_t
   else if (gm * gn <= 512) { rb = (int)((gm + 7) / 8); cb = (int)gn; }
   else if (gm < rb) { cb = (int)(rb * cb / gm); rb = (int)gm; }
   else if (gn < cb) { rb = (int)(rb * cb / gn); cb = (int)gn; }
+  // Dealt one by one where these blocks give an XCD a tenth more rounds or tiles than that does: a 9 x 27 grid in
+  // bands of four columns is 36 tiles on an XCD of 32 compute units, two rounds (f64 576 x 3456 x 1024 133 against 70 us, f32 69
+  // against 36; f64 704 x 1152 x 2048 135 against 69, 1600 x 2496 x 2944 529 against 363), and a last column of blocks that is
+  // mostly empty may fall to the same XCDs again and again (3904 x 320 x 1216 132 against 89).  Balanced blocks are the better order
+  // (2076 x 2008 x 1544 325 against 372).
+  if (rb > 0) {
+    const int64_t most = xcd_tiles(gm, gn, rb, cb), even = (gm * gn + 7) / 8;
+    if ((most + 31) / 32 * 10 > (even + 31) / 32 * 11 || most * 10 > even * 11) rb = cb = 0;
+  }
   if (const char* e = getenv("RX_GEMM_BLOCK")) { int v[2]; if (sscanf(e, "%d,%d", &v[0], &v[1]) == 2) { rb = v[0]; cb = v[1]; } }
   c.lds_bytes = (unsigned)lds;
   c.block = (unsigned)(t.WM * t.WN * t.KG * 64);

@@ -34,3 +34,24 @@ def test_one_stage_serves_one_tile(monkeypatch):
     assert "rx_gemm_body_g<rx_el_f32, 64, 64, 2, 2, 1, 1, " not in text(512, "64,64,2,2,1,1")
     assert "rx_gemm_body_g<rx_el_f32, 64, 64, 2, 2, 1, 2, " in text(512, "64,64,2,2,1,2")
     assert "rx_gemm_body_g<rx_el_f32, 64, 64, 2, 2, 2, 1, " in text(64, "64,64,2,2,2,1")
+
+
+@pytest.mark.parametrize("dt,m,n,k", [("f64", 576, 3456, 1024), ("f32", 576, 3456, 1024), ("f64", 704, 1152, 2048), ("bf16", 1344, 704, 1024), ("f64", 3904, 320, 1216),
+                                      ("f64", 1600, 2496, 2944), ("f32", 664, 4096, 1024), ("f32", 1001, 777, 1531), ("f64", 2076, 2008, 1544), ("f32", 4096, 4096, 4096)])
+def test_every_xcd_takes_its_share_of_the_tiles(dt, m, n, k):
+    """The order in which workgroups (dealt to eight XCDs of 32 compute units in turn) walk the tiles: no XCD takes a tenth more
+    tiles, or rounds of them, than an even share."""
+    text = rx.compile_offline(dot_module(m, n, k, dt, dt, True, False)[0], with_source=True)
+    args = re.search(r"rx_gemm_body_[gx]<(?:rx_el_\w+, )?([^>]*)>\(A, B, epi", text).group(1)
+    x = re.match(r"(\d+), (\d+), [^a-z]*(?:(?:true|false), )+%d, %d, %d, (\d+), (\d+)," % (m, n, k), args)
+    bm, bn, rb, cb = (int(v) for v in x.groups())
+    gm, gn = -(-m // bm), -(-n // bn)
+    load = [0] * 8
+    if rb == 0:
+        load = [len(range(x, gm * gn, 8)) for x in range(8)]
+    else:
+        for i, (r, c) in enumerate((r, c) for r in range(0, gm, rb) for c in range(0, gn, cb)):
+            load[i % 8] += min(rb, gm - r) * min(cb, gn - c)
+    even = -(-gm * gn // 8)
+    assert sum(load) == gm * gn
+    assert -(-max(load) // 32) <= 1.1 * -(-even // 32) and max(load) <= 1.1 * even, (load, even)
