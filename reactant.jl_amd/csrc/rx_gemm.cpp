@@ -132,6 +132,11 @@ static double group_estimate(DT dt, int64_t batch, int64_t M, int64_t N, int64_t
   const double step = std::max(1625.0 / std::max(sd - 1.0, 0.5), (big + 0.1 * (mf + ld + rd - big)) * (1.0 + 0.33 / std::max(w, 1.0)) + 170.0);
   double cycles = 4100.0 + rounds * KTG * step + (double)per * (double)t.BM * t.BN * (0.36 + (t.KG > 1 ? 0.15 * t.KG : 0.0)) + (rounds - 1.0) * 5600.0;
   cycles += 0.02 * cycles;
+  // Wavefronts that share no fragments, in five rounds of workgroups and more, take 1.35 to 1.9 times what is above (32 x 32 tiles:
+  // f32 276 x 4096 x 2048 88 us for 47, 615 x 2048 x 3000 107 for 70, f64 1408 x 1984 x 3840 548 for 392, 832 x 1408 x 704 60 for
+  // 35; 32 x 64 tiles: f64 2432 x 1472 x 1920 383 for 241).  With it f32 276 x 4096 x 2048 takes 53 us, f64 2232 x 700 x 3136
+  // 203 (320 on 32 x 32 tiles), 1368 x 3524 x 468 90 (105).
+  if (es >= 4 && NW <= 2 && t.BM * t.BN >= 1024 && per >= 5) cycles *= 1.5;
   cycles = std::max(cycles, 4100.0 + (double)(T / split) * (t.BM + t.BN) * (double)K * es / 6000.0);
   const double bytes = (double)batch * (double)(M + N) * (double)K * es;
   cycles = std::max(cycles, 4100.0 + bytes / 1700.0);

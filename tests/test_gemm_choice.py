@@ -55,3 +55,10 @@ def test_every_xcd_takes_its_share_of_the_tiles(dt, m, n, k):
     even = -(-gm * gn // 8)
     assert sum(load) == gm * gn
     assert -(-max(load) // 32) <= 1.1 * -(-even // 32), (load, even)
+
+
+@pytest.mark.parametrize("dt,m,n,k", [("f32", 276, 4096, 2048), ("f32", 615, 2048, 3000), ("f64", 1408, 1984, 3840), ("f64", 2432, 1472, 1920)])
+def test_many_rounds_of_tiles_are_not_those_of_lone_wavefronts(dt, m, n, k):
+    text = rx.compile_offline(dot_module(m, n, k, dt, dt, True, False)[0], with_source=True)
+    wm, wn = re.search(r"rx_gemm_body_g<rx_el_\w+, \d+, \d+, (\d+), (\d+), ", text).groups()
+    assert int(wm) * int(wn) > 2
