@@ -1112,13 +1112,27 @@ struct Planner {
     // and its combine and epilogue launches (13-22 us; 142 us for e4m3 6 x 4096 x 4096, whose reduction converts every
     // weight once per row).  One and four rows of 4-byte and wider elements, which the reduction's vectors fit, stay with it
     // from 2^24 elements on, where it streams the matrix faster (4 x 4096 x 25088 f32 78 against 102 us), and four rows
-    // below 2^21 elements.
-    const int64_t big = std::max(lt.numel(), rt.numel()), rows = r.big_is_lhs ? nfree : mfree;
+    // below 2^21 elements.  So does one row against a matrix whose rows are contracted, which is one launch without a
+    // combine (f32 1 x 1024 x 8192 6.3 against 12.9 us, 1 x 8192 x 1024 6.4 against 9.6, f64 1 x 2048 x 4096 11.1 against 18.1).
+    // f64 MFMAs take four times those of f32 per element, and a long K in few columns is a chain of them: one row stays from
+    // 2^22 elements or K = 4096 on (1 x 512 x 4096 11.5 against 16.5, 1 x 4096 x 1024 10.2 against 10.6, 1 x 2048 x 1024 9.9
+    // against 7.2), two rows from 2^23 or K = 4096 on (2 x 4096 x 4096 28.3 against 35.1, 2 x 4096 x 1024 11.6 against 10.6), or in
+    // contracted rows with K = 4096 and at most 1024 of them (2 x 1024 x 8192 21.9 against 26.5, 2 x 2048 x 8192 38.8 against
+    // 33.3), and three and four rows with K = 4096 and at most 512 columns (4 x 512 x 8192 23.6 against 26.6; three in
+    // contracted rows only: 18.0 against 26.5, otherwise 35.2 against 26.8).
+    const int64_t big = std::max(lt.numel(), rt.numel()), rows = r.big_is_lhs ? nfree : mfree, cols = big / kprod;
     const bool wide = info(lt.dt).size >= 4;
-    const bool streams = wide && (rows == 1 || rows == 4) && (big >= (1 << 24) || (rows == 4 && big < (1 << 21)));
+    bool streams = wide && (rows == 1 || rows == 4) && (big >= (1 << 24) || (rows == 4 && big < (1 << 21)));
     if (opt.mfma && is_float(lt.dt) && lt.dt != DT::F8E5M2 && big >= (1 << 18) && !streams) {
       const DotForm f = dot_form(d);
-      if (f.ok && d.ty.rank() == 2 && choose_gemm(lt.dt, rt.dt, d.ty.dt, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig).skeleton == "rx_gemm_body_g") return r;
+      const bool kc = r.big_is_lhs ? f.a_k_contig : f.b_k_contig, lng = kprod >= 4096;
+      if (wide && rows == 1 && kc) streams = true;
+      if (lt.dt == DT::F64 && rows <= 4) {
+        if (rows == 1) streams = streams || lng || big >= (1 << 22);
+        else if (rows == 2) streams = kc ? lng && cols <= 1024 : lng || big >= (1 << 23);
+        else streams = lng && cols <= 512 && (rows == 4 || kc);
+      }
+      if (!streams && f.ok && d.ty.rank() == 2 && choose_gemm(lt.dt, rt.dt, d.ty.dt, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig).skeleton == "rx_gemm_body_g") return r;
     }
     r.ok = true;
     return r;

@@ -62,3 +62,13 @@ def test_many_rounds_of_tiles_are_not_those_of_lone_wavefronts(dt, m, n, k):
     text = rx.compile_offline(dot_module(m, n, k, dt, dt, True, False)[0], with_source=True)
     wm, wn = re.search(r"rx_gemm_body_g<rx_el_\w+, \d+, \d+, (\d+), (\d+), ", text).groups()
     assert int(wm) * int(wn) > 2
+
+
+# rows, columns, K and whether the matrix is stored [o][k]
+@pytest.mark.parametrize("dt,m,n,k,kc,gemm", [("f32", 1, 1024, 8192, True, False), ("f32", 1, 8192, 1024, True, False), ("f32", 1, 2048, 4096, False, True), ("f32", 2, 1024, 8192, True, True),
+                                              ("f64", 1, 512, 4096, False, False), ("f64", 1, 2048, 1024, False, True), ("f64", 1, 2048, 1024, True, False), ("f64", 2, 4096, 4096, False, False),
+                                              ("f64", 2, 2048, 4096, True, True), ("f64", 2, 1024, 4096, True, False), ("f64", 3, 4096, 4096, False, True), ("f64", 3, 512, 8192, True, False),
+                                              ("f64", 4, 512, 8192, False, False), ("f64", 4, 1024, 4096, False, True), ("bf16", 1, 1024, 8192, True, True), ("f8E4M3FN", 6, 4096, 4096, True, True)])
+def test_few_rows_go_where_they_are_fast(dt, m, n, k, kc, gemm):
+    out = "f32" if dt.startswith("f8") else dt
+    assert ("kind=gemm" in rx.compile_offline(dot_module(m, n, k, dt, out, True, kc)[0])) == gemm
