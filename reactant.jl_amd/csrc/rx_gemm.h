@@ -38,6 +38,10 @@ inline int64_t gemm_grid(int64_t gm, int64_t gn, int rb = 4, int cb = 8) {
 GemmChoice choose_gemm(DT a, DT b, DT out, int64_t batch, int64_t M, int64_t N, int64_t K, bool a_k_contig, bool b_k_contig,
                        bool staged_only = false, int split = 1, bool groups = true);
 
+// Few rows against a matrix with a long K, and into how many slices the ring skeleton cuts it (1: it is not the one to): the
+// rows of both operands are K, or those of the matrix are its columns.
+int ring_slices(DT dt, int64_t M, int64_t N, int64_t K, bool a_k_contig, bool b_k_contig);
+
 // Text of the `extern "C"` kernel <kbase>_gemm that runs the skeleton with epilogue type <kbase>_epi.
 // `epi_params` is the tail of the parameter list (epilogue operands and out0), `epi_ctor` builds `epi`.
 // An operand computed by a functor: `type` names the functor struct ("" = read from memory), `params` the

@@ -1015,16 +1015,15 @@ struct Planner {
       // the slices' sums cost a launch and a pass over them, and a result that elementwise ops consume loses its epilogue:
       // another launch (4 us each between dependent launches)
       const double extra = followed[d.id] ? 8.0 : 4.0;
-      int S = 1;
+      int S = ring_slices(a, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig);
       double best = whole.est_us > 0 ? whole.est_us : 1e30;   // the skeletons that slices compete with have an estimate
-      // Cut whatever the estimates say: products that nothing elementwise follows, of at most 128 whole tiles and K >= 2048 (f32 256 x 256 x
-      // 2048 11.6 against 7.9 us uncut, bf16 128 x 128 x 16384 15.7 against 23.7); and 17 to 32 rows of 16-bit elements against
-      // [k][n] weights with K >= 4096 (32 x 4096 x 25088 57 against 104 us, 32 x 4096 x 4096 15.5 against 11.2).
       const bool few = !followed[d.id] && tiles <= 128 && f.M % 64 == 0 && f.N % 64 == 0 && f.K >= 2048;
-      const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= 4096;
-      if (few || dense) {   // two workgroups per compute unit, slices of at least 512
+      // 17 to 32 rows of 16-bit elements against [k][n] weights, K >= 16384, that the ring skeleton does not take: the estimates
+      // leave them whole (32 x 1000 x 25088 22 us cut, 31 not; 32 x 8192 x 18432 118 and 141; 32 x 8192 x 8192 39 and 37)
+      const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= 16384;
+      if (S == 1 && (few || dense)) {   // two workgroups per compute unit, slices of at least 512
         while (S < 256 && tiles * S < 512 && f.K / (2 * S) >= 512) S *= 2;
-      } else {
+      } else if (S == 1) {
         for (int q = 2; q <= 256 && f.K / q >= 256; q *= 2) {
           GemmChoice c = choose_gemm(a, b, DT::F32, 1, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig, false, q);
           if (!c.ok || c.split != q) continue;

@@ -72,3 +72,18 @@ def test_many_rounds_of_tiles_are_not_those_of_lone_wavefronts(dt, m, n, k):
 def test_few_rows_go_where_they_are_fast(dt, m, n, k, kc, gemm):
     out = "f32" if dt.startswith("f8") else dt
     assert ("kind=gemm" in rx.compile_offline(dot_module(m, n, k, dt, out, True, kc)[0])) == gemm
+
+
+@pytest.mark.parametrize("dt,m,n,k,orders,slices", [("bf16", 32, 4096, 25088, (True, False), 8), ("bf16", 16, 2048, 8192, (True, False), 16), ("f16", 64, 4096, 18432, (True, True), 8),
+                                                    ("bf16", 4096, 20, 8192, (False, True), 8), ("f8E4M3FN", 16, 4096, 8192, (True, False), 8), ("bf16", 32, 4096, 4096, (True, False), 1),
+                                                    ("bf16", 32, 8192, 8192, (True, False), 1), ("bf16", 16, 1000, 25088, (True, False), 0), ("bf16", 32, 1000, 25088, (True, False), 0),
+                                                    ("bf16", 32, 8192, 18432, (True, False), 0), ("bf16", 32, 4096, 18432, (True, True), 1)])
+def test_long_matrices_against_few_rows_are_cut_on_the_ring_skeleton(dt, m, n, k, orders, slices):
+    """0: cut, but not on that skeleton."""
+    out = "f32" if dt.startswith("f8") else dt
+    text, _, _ = dot_module(m, n, k, dt, out, *orders)
+    text = text.replace("return %0", "%%1 = stablehlo.add %%0, %%0 : (T, T) -> T\n    return %%1".replace("%%", "%").replace("T", "tensor<%dx%dx%s>" % (m, n, out)))
+    src = rx.compile_offline(text, with_source=True)
+    cut = int(re.search(r"kind=gemm_\w+ grid=\d+x(\d+)x1", src).group(1))
+    assert ("rx_gemm_body_dl<" in src) == (slices > 1)
+    assert cut == slices if slices else cut > 1
