@@ -1017,7 +1017,12 @@ struct Planner {
       const double extra = followed[d.id] ? 8.0 : 4.0;
       int S = ring_slices(a, f.M, f.N, f.K, f.a_k_contig, f.b_k_contig);
       double best = whole.est_us > 0 ? whole.est_us : 1e30;   // the skeletons that slices compete with have an estimate
-      const bool few = !followed[d.id] && tiles <= 128 && f.M % 64 == 0 && f.N % 64 == 0 && f.K >= 2048;
+      // Products of whole 64 x 64 tiles, at most 16 with K >= 2048 or 128 with K >= 4096, that nothing elementwise follows are cut for
+      // their sums, whose error is half to two thirds of the uncut product's (f32 256 x 256 x 2048 2.1e-7 against 4.1e-7, 256 x 2048 x 4096
+      // 4.1e-7 against 5.8e-7, bf16 320 x 192 x 4096 1.1e-7 against 1.4e-7).  That costs a launch: cut and uncut 9.9 and 7.4 us, 41.4 and
+      // 37.4, 9.9 and 8.4, bf16 128 x 128 x 16384 13.4 and 24.8, 512 x 1024 x 4096 15.7 and 16.3, e4m3 256 x 128 x 8192 10.8 and 7.8.  The
+      // others follow the estimates (bf16 512 x 1024 x 2048 12.1 cut, 8.0 not).
+      const bool few = !followed[d.id] && f.M % 64 == 0 && f.N % 64 == 0 && (tiles <= 16 ? f.K >= 2048 : tiles <= 128 && f.K >= 4096);
       // 17 to 32 rows of 16-bit elements against [k][n] weights, K >= 16384, that the ring skeleton does not take: the estimates
       // leave them whole (32 x 1000 x 25088 22 us cut, 31 not; 32 x 8192 x 18432 118 and 141; 32 x 8192 x 8192 39 and 37)
       const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= 16384;

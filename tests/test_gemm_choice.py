@@ -87,3 +87,9 @@ def test_long_matrices_against_few_rows_are_cut_on_the_ring_skeleton(dt, m, n, k
     cut = int(re.search(r"kind=gemm_\w+ grid=\d+x(\d+)x1", src).group(1))
     assert ("rx_gemm_body_dl<" in src) == (slices > 1)
     assert cut == slices if slices else cut > 1
+
+
+@pytest.mark.parametrize("dt,m,n,k,cut", [("f32", 256, 256, 2048, True), ("bf16", 512, 1024, 4096, True), ("bf16", 512, 1024, 2048, False), ("f32", 512, 1024, 2048, False)])
+def test_which_products_without_a_consumer_are_cut(dt, m, n, k, cut):
+    rep = rx.compile_offline(dot_module(m, n, k, dt, dt, False, False)[0])
+    assert (int(re.search(r"kind=gemm_\w+ grid=\d+x(\d+)x1", rep).group(1)) > 1) == cut
