@@ -1895,11 +1895,12 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
 // f32 products on the bf16 matrix cores: every operand as a sum of three bf16 numbers.
 // x = h + m + l with h = bf16(x), m = bf16(x - h), l = bf16(x - h - m): 3 x 8 bits and two signs hold the 24 bits exactly,
 // and so do subnormal parts (neither the conversion nor the bf16 MFMA flushes them).  A product is then six terms,
-// l h + h l + m m + m h + h m + h h; what is left out, m l + l m + l l, is at most 2^-25 of |x||y| and of either sign, below
-// the rounding of the sum.  Per K tile of 32 the five small terms are summed from zero, the smallest first, added to the
-// running sum, and h h goes into that: it is rounded twice per 32 k.  Error against 64 bits (2-norm, N(0,1) operands), this
-// body and the f32 MFMA bodies: 4096^3 4.4e-7 and 1.14e-6, 8192 x 4096 x 1024 2.1e-7 and 5.7e-7, 2048^3 3.1e-7 (two groups
-// 2.2e-7) and 5.7e-7, 2000 x 3000 x 500 1.5e-7 and 4.0e-7.
+// l h + h l + m m + m h + h m + h h; what is left out, m l + l m + l l, is at most 2^-24 of |x||y| (1.98 2^-25 of it for
+// x = y = 1 + 2^-8 - 2^-17), of either sign: a rounding of the product.  Per K tile of 32 the five small terms are summed from
+// zero, the smallest first, added to the running sum, and h h goes into that: it is rounded twice per 32 k.  Error against 64
+// bits (2-norm, N(0,1) operands), this body and the f32 MFMA bodies: 4096^3 4.4e-7 and 1.14e-6, 8192 x 4096 x 1024 2.1e-7 and
+// 5.7e-7, 2048^3 3.1e-7 (two groups 2.1e-7) and 8.1e-7, 2000 x 3000 x 500 1.4e-7 and 4.0e-7; uniform in [0, 1): 4096^3 3.3e-7
+// and 8.5e-7, 2048^3 1.3e-7 and 6.0e-7; all operands the x above: 5.9e-8 and 5.9e-8.
 // Two kinds of input do not split: an infinity (and a finite number that rounds to one) leaves inf - inf, so its
 // products become NaN; a number below 2^-102 may have bits below 2^-133, the last that bf16 holds.  The first is seen in the
 // result, which is not finite; the second while splitting, x - h - m being subnormal and not zero.  A workgroup that sees

@@ -217,3 +217,32 @@ def test_tiny_numbers_where_they_matter_and_where_not(rx, client, monkeypatch, t
     a0[..., 299, 3] = np.inf
     got = run(a0, b0)
     assert not np.isfinite(got[..., 299, :]).any() and np.isfinite(got[..., :299, :]).all()
+
+
+# K is no whole number of K tiles, of 16-byte chunks or of slices, N odd (f32) or two more than a vector
+SLICED = [("f32", 21, 35, 20001), ("f32", 101, 203, 20001), ("bf16", 20, 34, 20002), ("bf16", 100, 202, 20002), ("f16", 20, 34, 20002), ("f16", 100, 202, 20002), ("f8E4M3FN", 20, 36, 20004)]
+
+
+@pytest.mark.parametrize("dt,M,N,K,order", [c + (o,) for c in SLICED for o in ORDERS])
+def test_slices_of_ragged_products(rx, client, dt, M, N, K, order):
+    """K cut into slices of a workgroup's groups where nothing divides anything: the last slices' tiles lie past K."""
+    out = {"f8E4M3FN": "f32"}.get(dt, dt)
+    text, sa, sb = dot_module(M, N, K, dt, out, *order)
+    a, b = (I.tensor(np.random.default_rng(s).normal(size=z), dt) for s, z in ((14, sa), (15, sb)))
+    got, exe = gpu_run(rx, client, text, [a, b])
+    slices = int(re.search(r"kind=gemm_\w+ grid=\d+x(\d+)x1", exe.report()).group(1))
+    assert slices > 1 and K % slices and exe.launches()[1]["kind"].startswith("reduce")
+    ref = oracle_run(text, [a, b], hifi=True)
+    assert contraction_err(got[0].a, ref[0].a, dot_bound(text, [a, b])) <= cw_tol(dt, out)
+
+
+def test_the_terms_that_the_split_leaves_out(rx, client):
+    """Constant operands whose left-out terms m l + l m + l l are largest, 1.98 2^-25 of every product and all of one sign."""
+    M, N, K = 2048, 2048, 256
+    text, sa, sb = dot_module(M, N, K, "f32", "f32", True, True)
+    assert "rx_gemm_body_x<" in rx.compile_offline(text, with_source=True)
+    x = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    got, _ = gpu_run(rx, client, text, [I.Tensor(np.full(sa, x), "f32"), I.Tensor(np.full(sb, x), "f32")])
+    exact = K * np.float64(x) ** 2
+    # 2^-24 left out, and two roundings per 32 k of sums that are half the result in the mean
+    assert np.abs(got[0].a / exact - 1).max() <= 2.0 ** -24 * (1 + K / 32)
