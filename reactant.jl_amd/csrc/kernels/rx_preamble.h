@@ -79,6 +79,14 @@ RX_DEV float rx_u2f(rx_u32 u) { return __builtin_bit_cast(float, u); }
 // ---------------------------------------------------------------------------
 // bf16: storage is the upper half of binary32; conversion rounds to nearest even
 // ---------------------------------------------------------------------------
+// The argument of sin, cos and tan, which reduce large arguments (beyond 2^17 in f32) on a path of 90 instructions.  Where a
+// thread takes one element at a time the compiler computes both paths and selects, unless the argument comes from something it
+// cannot look into: sum(sin(x) + y) over 10379445 f32 34 -> 20 us.
+template <typename T>
+RX_DEV T rx_apart(T x) {
+  asm("" : "+v"(x));
+  return x;
+}
 RX_DEV float rx_bf16_to_f32(rx_u16 b) { return rx_u2f(((rx_u32)b) << 16); }
 // gfx950 converts in hardware (v_cvt_pk_bf16_f32, round to nearest even, NaN stays NaN)
 RX_DEV rx_u16 rx_f32_to_bf16(float f) { return __builtin_bit_cast(rx_u16, (__bf16)f); }

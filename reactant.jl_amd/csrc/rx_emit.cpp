@@ -414,9 +414,9 @@ std::string Emitter::emit_op(const Node& n, const Index& ix) {
           if (op == m) return def(fn(m, dbl) + "(" + x + ")");
         if (op == "erf_inv") return def(fn("erfinv", dbl) + "(" + x + ")");
         if (op == "digamma") return def("rx_digamma(" + x + ")");
-        if (op == "sine") return def(fn("sin", dbl) + "(" + x + ")");
-        if (op == "cosine") return def(fn("cos", dbl) + "(" + x + ")");
-        if (op == "tan") return def(fn("tan", dbl) + "(" + x + ")");
+        if (op == "sine") return def(fn("sin", dbl) + "(rx_apart(" + x + "))");
+        if (op == "cosine") return def(fn("cos", dbl) + "(rx_apart(" + x + "))");
+        if (op == "tan") return def(fn("tan", dbl) + "(rx_apart(" + x + "))");
         if (op == "tanh") return def((is_narrow_float(dt) ? std::string("rx_tanh_fast") : fn("tanh", dbl)) + "(" + x + ")");
         if (op == "exponential") return def((is_narrow_float(dt) ? std::string("rx_exp_fast") : fn("exp", dbl)) + "(" + x + ")");
         if (op == "exponential_minus_one") return def(fn("expm1", dbl) + "(" + x + ")");
