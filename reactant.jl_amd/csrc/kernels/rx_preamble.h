@@ -87,6 +87,13 @@ RX_DEV T rx_apart(T x) {
   asm("" : "+v"(x));
   return x;
 }
+// A negation whose result is rounded to a narrow float: two of them side by side become one of a pair of floats, which the
+// compiler fails to select with packed f32 instructions off ("Cannot select ... v2f32 = bitcast"), so the sign is flipped as an integer.
+RX_DEV float rx_neg_narrow(float x) {
+  rx_u32 u = rx_f2u(x) ^ 0x80000000u;
+  asm("" : "+v"(u));
+  return rx_u2f(u);
+}
 RX_DEV float rx_bf16_to_f32(rx_u16 b) { return rx_u2f(((rx_u32)b) << 16); }
 // gfx950 converts in hardware (v_cvt_pk_bf16_f32, round to nearest even, NaN stays NaN)
 RX_DEV rx_u16 rx_f32_to_bf16(float f) { return __builtin_bit_cast(rx_u16, (__bf16)f); }

@@ -426,7 +426,7 @@ std::string Emitter::emit_op(const Node& n, const Index& ix) {
         if (op == "cbrt") return def(fn("cbrt", dbl) + "(" + x + ")");
         if (op == "rsqrt") return def("rx_rsqrt(" + x + ")");
         if (op == "abs") return def(fn("fabs", dbl) + "(" + x + ")");
-        if (op == "negate") return def("(-" + x + ")");
+        if (op == "negate") return def(is_narrow_float(dt) ? "rx_neg_narrow(" + x + ")" : "(-" + x + ")");
         if (op == "logistic") return def((is_narrow_float(dt) ? "rx_logistic_fast(" : "rx_logistic(") + x + ")");
         if (op == "floor") return def(fn("floor", dbl) + "(" + x + ")");
         if (op == "ceil") return def(fn("ceil", dbl) + "(" + x + ")");
@@ -477,6 +477,8 @@ std::string Emitter::emit_op(const Node& n, const Index& ix) {
       if (is_float(dt)) {
         if (op == "add") return def("(" + a + " + " + b + ")");
         if (op == "subtract") return def("(" + a + " - " + b + ")");
+        if (op == "multiply" && is_narrow_float(dt) && (a == float_lit(-1.0, false) || b == float_lit(-1.0, false)))   // the compiler's negation
+          return def("rx_neg_narrow(" + (a == float_lit(-1.0, false) ? b : a) + ")");
         if (op == "multiply") return def("(" + a + " * " + b + ")");
         if (op == "divide") {
           // a divisor that is one value for the whole tensor (a broadcast scalar, e.g. a
