@@ -1502,7 +1502,7 @@ RX_DEV void rx_gemm_body_f64(const double* __restrict__ A, const double* __restr
 // Measured (kernel time, against the skeletons above and the launches they needed): f32 777 x 1001 x 1531 32 us = 74 TFLOP/s
 // (the MFMAs of one 64 x 64 tile alone are 20 us; 9 + 89 + 4 us through padded copies and the register-staged body); bf16
 // 16 x 4096 x 4096 10 (7.4 + 4.1 + 4.1 cut along K), 926 x 1024 x 2048 9 (24.7 + 4.7 + 4.1), 1024 x 2048 x 784 8 (21); e4m3
-// 200 x 6144 x 4096 11.6 (17), 6 x 4096 x 4096 4.2 (130 as a reduction), 3000 x 4096 x 4096 51 (59); f64 4096^3 1.90 ms = 72 of
+// 200 x 6144 x 4096 11.6 (17), 6 x 4096 x 4096 8.2 (226 as a reduction), 3000 x 4096 x 4096 51 (59); f64 4096^3 1.90 ms = 72 of
 // 78.6 TFLOP/s (2.20), 1000^3 44 us (65).
 // ===========================================================================
 struct rx_el_f32 {

@@ -438,7 +438,7 @@ static GemmChoice choose_tiled(DT a, DT out, int64_t batch, int64_t M, int64_t N
 // for two workgroups per 64 columns and compute unit, reads long matrices at 5 to 7 TB/s where the tiles of the group body
 // (whose estimate does not show it) keep to 2 to 3.5; with two more launches it pays from some length on.  Slices and all
 // against the group body, bf16, us: matrices stored [k][o] 16 x 2048 x 8192 11.7 and 19.5, 64 x 2048 x 8192 15.0 and 20.3, 32 x 4096 x 8192
-// 16.9 and 21.1, 32 x 4096 x 4096 12.6 and 11.7, 32 x 4096 x 25088 35.9 and 60.5, 32 x 1024 x 8192 11.6 and 8.9, 32 x 1024 x 18432 14.9
+// 16.9 and 21.1, 32 x 4096 x 4096 12.6 and 11.7 (15.6 in slices of the group body, which 17 to 32 rows are cut into), 32 x 4096 x 25088 35.9 and 60.5, 32 x 1024 x 8192 11.6 and 8.9, 32 x 1024 x 18432 14.9
 // and 17.3; stored [o][k] 64 x 4096 x 18432 32.1 and 39.8, 32 x 4096 x 18432 29.5 and 23.9, 64 x 4096 x 8192 19.6 and 18.7; e4m3
 // stored [k][o] 32 x 4096 x 8192 12.4 and 18.1, 32 x 2048 x 8192 11.3 and 11.0.  More than 4096 columns: 32 x 8192 x 8192 63.8
 // and 37.0.  With fewer than 128 workgroups (K is no multiple of enough slices) only 33 and more rows: 16 x 1024 x 25088 29.2 and
@@ -448,7 +448,7 @@ int ring_slices(DT dt, int64_t M, int64_t N, int64_t K, bool a_kc, bool b_kc) {
   const int64_t rows = std::min(M, N), cols = std::max(M, N);
   const bool rows_kc = M < N ? a_kc : b_kc, kc = M < N ? b_kc : a_kc;
   if (es > 2 || !rows_kc || rows < 9 || rows > 64 || cols > 4096) return 1;
-  if (es == 1 ? kc || K < 8192 || cols < 3072 : kc ? rows <= 32 || K < 16384 || cols < 900 : K < 8192 || cols < (K < 16384 ? 1536 : 900)) return 1;
+  if (es == 1 ? kc || K < 8192 || cols < 3072 : kc ? rows <= 32 || K < 16384 || cols < 900 : K < (rows > 16 && rows <= 32 ? 4096 : 8192) || cols < (K < 16384 ? 1536 : 900)) return 1;
   const int64_t tiles = (cols + 63) / 64;
   int64_t S = 1;
   while (S < 256 && tiles * S < 512 && K / (2 * S) >= 512) S *= 2;

@@ -1023,9 +1023,11 @@ struct Planner {
       // 37.4, 9.9 and 8.4, bf16 128 x 128 x 16384 13.4 and 24.8, 512 x 1024 x 4096 15.7 and 16.3, e4m3 256 x 128 x 8192 10.8 and 7.8.  The
       // others follow the estimates (bf16 512 x 1024 x 2048 12.1 cut, 8.0 not).
       const bool few = !followed[d.id] && f.M % 64 == 0 && f.N % 64 == 0 && (tiles <= 16 ? f.K >= 2048 : tiles <= 128 && f.K >= 4096);
-      // 17 to 32 rows of 16-bit elements against [k][n] weights, K >= 16384, that the ring skeleton does not take: the estimates
-      // leave them whole (32 x 1000 x 25088 22 us cut, 31 not; 32 x 8192 x 18432 118 and 141; 32 x 8192 x 8192 39 and 37)
-      const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= 16384;
+      // 17 to 32 rows of 16-bit elements against [k][n] weights, the dense layers of the vision models on a batch of 32, that the ring
+      // skeleton does not take.  From K = 16384 on the estimates leave whole what is faster cut (32 x 1000 x 25088 22 us cut, 31 not; 32 x
+      // 8192 x 18432 118 and 141; 32 x 8192 x 8192 39 and 37); from 4096 on, up to 4096 columns, it is the three-launch plan of those
+      // models' last layers that is kept, not the time (32 x 1000 x 4096 12 us cut, 7 not).
+      const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= (f.N <= 4096 ? 4096 : 16384);
       if (S == 1 && (few || dense)) {   // two workgroups per compute unit, slices of at least 512
         while (S < 256 && tiles * S < 512 && f.K / (2 * S) >= 512) S *= 2;
       } else if (S == 1) {

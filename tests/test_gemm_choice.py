@@ -75,7 +75,7 @@ def test_few_rows_go_where_they_are_fast(dt, m, n, k, kc, gemm):
 
 
 @pytest.mark.parametrize("dt,m,n,k,orders,slices", [("bf16", 32, 4096, 25088, (True, False), 8), ("bf16", 16, 2048, 8192, (True, False), 16), ("f16", 64, 4096, 18432, (True, True), 8),
-                                                    ("bf16", 4096, 20, 8192, (False, True), 8), ("f8E4M3FN", 16, 4096, 8192, (True, False), 8), ("bf16", 32, 4096, 4096, (True, False), 1),
+                                                    ("bf16", 4096, 20, 8192, (False, True), 8), ("f8E4M3FN", 16, 4096, 8192, (True, False), 8), ("bf16", 32, 4096, 4096, (True, False), 8), ("bf16", 16, 4096, 4096, (True, False), 1), ("bf16", 40, 4096, 4096, (True, False), 1),
                                                     ("bf16", 32, 8192, 8192, (True, False), 1), ("bf16", 16, 1000, 25088, (True, False), 0), ("bf16", 32, 1000, 25088, (True, False), 0),
                                                     ("bf16", 32, 8192, 18432, (True, False), 0), ("bf16", 32, 4096, 18432, (True, True), 1)])
 def test_long_matrices_against_few_rows_are_cut_on_the_ring_skeleton(dt, m, n, k, orders, slices):
