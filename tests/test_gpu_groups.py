@@ -236,10 +236,11 @@ def test_slices_of_ragged_products(rx, client, dt, M, N, K, order):
     assert contraction_err(got[0].a, ref[0].a, dot_bound(text, [a, b])) <= cw_tol(dt, out)
 
 
-def test_the_terms_that_the_split_leaves_out(rx, client):
+def test_the_terms_that_the_split_leaves_out(rx, client, monkeypatch):
     """Constant operands whose left-out terms m l + l m + l l are largest, 1.98 2^-25 of every product and all of one sign."""
-    M, N, K = 2048, 2048, 256
+    M, N, K = 256, 256, 256
     text, sa, sb = dot_module(M, N, K, "f32", "f32", True, True)
+    monkeypatch.setenv("RX_GEMM_G", "128,128,2,2,1,1,1")
     assert "rx_gemm_body_x<" in rx.compile_offline(text, with_source=True)
     x = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
     got, _ = gpu_run(rx, client, text, [I.Tensor(np.full(sa, x), "f32"), I.Tensor(np.full(sb, x), "f32")])
