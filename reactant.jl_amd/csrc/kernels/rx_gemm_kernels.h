@@ -1912,13 +1912,13 @@ RX_DEV void rx_gemm_body_g(const typename EL::elem* __restrict__ A, const typena
 //
 // Time: six 16 x 16 x 32 bf16 MFMAs take 96 cycles of the matrix pipe where eight 16 x 16 x 4 f32 MFMAs take 256.  What bounds
 // it is the sum of the MFMAs and the vector instructions (per element 5.5 to split it and one to test it, and four per
-// MFMA block and K tile to add the small terms): 786 and 589 thousand cycles per SIMD for 4096^3 on 128 x 128 tiles, of
-// the 1540 that the kernel takes.  They did not overlap in any order that was tried (a wavefront splitting while its partner
+// MFMA block and K tile to add the small terms): 786 and 473 thousand cycles per SIMD for 4096^3 on 128 x 256 tiles, of
+// the 1450 that the kernel takes (on 128 x 128 tiles 786 and 589 of 1540).  They did not overlap in any order that was tried (a wavefront splitting while its partner
 // multiplies, with and without priorities, and instruction by instruction as here: 704, 722, 697 us), so
 // the splitting is done once per workgroup, between the global load into registers and the LDS tile, which holds three
 // bf16 planes of 32 k per operand: on the fragments, once per wavefront that reads them, 4096^3 took 842 us.  128 x 256 tiles
-// split less per product than 128 x 128 (4096^3 668 against 697 us).  4096^3 977 -> 668 us (206 TFLOP/s), 8192 x 4096 x 1024
-// 545 -> 370, 2048^3 128 -> 98, 2000 x 3000 x 500 66 -> 49.
+// split less per product than 128 x 128 (4096^3 668 against 697 us).  4096^3 955 -> 634 to 668 us (206 to 217 TFLOP/s), 8192 x
+// 4096 x 1024 545 -> 331, 2048^3 139 -> 91, 2000 x 3000 x 500 66 -> 43.
 // One LDS stage; the next K tile waits split in registers, and the one after it is on its way into the registers that the
 // splitting has left.  K in groups (KG), range checks and sizes are those of rx_gemm_body_g.
 // LDS rows are 64 bytes, four chunks of 16.  A [row][k] operand is loaded as 16-byte vectors along k (a row of 32 k is
