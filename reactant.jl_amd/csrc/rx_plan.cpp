@@ -999,9 +999,57 @@ struct Planner {
     if (!opt.mfma || !opt.split_k) return;
     std::map<int, int> splits;
     std::vector<char> followed(g.nodes.size(), 0);   // read by an elementwise op
+    std::vector<std::vector<int>> readers(g.nodes.size());
+    for (const Node& n : g.nodes)
+      for (int i : n.in) readers[i].push_back(n.id);
+    // Does a 16-bit product reach, through arithmetic that has no other reader, a value from which several results of elementwise
+    // ops are computed?  That value is the epilogue's result then, and rounded to 16 bits in between; as a sum of slices the product is
+    // held in f32 and every reader computes the value from it, rounded once in the end (a training step's y, with y + b - t read by the
+    // loss and by the gradient: the gradients' 2-norm error 3.1e-3 against 3.35e-3 for 185 rows in bf16).
+    auto elementwise = [](const Node& n) {
+      return n.k == OpK::Unary || n.k == OpK::Binary || n.k == OpK::Compare || n.k == OpK::Select || n.k == OpK::Clamp || n.k == OpK::Convert || n.k == OpK::Gelu;
+    };
+    const std::set<int> results(g.results.begin(), g.results.end());
+    // the elementwise values computed from v, short of `without`; how many of them something else reads
+    auto computed_from = [&](int v, int without, std::set<int>* seen) {
+      std::vector<int> todo = {v};
+      int read = 0;
+      while (!todo.empty() && seen->size() < 100) {
+        const int at = todo.back();
+        todo.pop_back();
+        bool outside = results.count(at) != 0;
+        for (int r : readers[at]) {
+          if (!elementwise(g.nodes[r])) outside = true;
+          else if (r != without && seen->insert(r).second) todo.push_back(r);
+        }
+        read += outside;
+      }
+      return read;
+    };
+    auto several_results = [&](int v) {   // and no one value that all of them are computed from, as from the end of a gelu
+      std::set<int> from, rest;
+      if (computed_from(v, -1, &from) < 2 || from.size() >= 100) return false;
+      return std::none_of(from.begin(), from.end(), [&](int x) { rest.clear(); return computed_from(v, x, &rest) == 0; });
+    };
+    auto held = [&](const Node& d) {
+      if (!is_narrow_float(d.ty.dt)) return false;
+      auto rounds = [&](const Node& n) {
+        return n.k == OpK::Gelu || n.k == OpK::Convert || (n.k == OpK::Unary && n.op != "negate" && n.op != "abs") ||
+               (n.k == OpK::Binary && n.op != "maximum" && n.op != "minimum");
+      };
+      bool computed = false;
+      for (int at = d.id;;) {
+        const std::vector<int>& r = readers[at];
+        if (r.size() != 1) return computed && several_results(at) && std::any_of(r.begin(), r.end(), [&](int i) { return rounds(g.nodes[i]); });
+        const Node& n = g.nodes[r[0]];
+        if (!elementwise(n)) return false;
+        computed = computed || rounds(n);
+        at = n.id;
+      }
+    };
     for (const Node& n : g.nodes)
       for (int i : n.in)
-        if (n.k == OpK::Unary || n.k == OpK::Binary || n.k == OpK::Compare || n.k == OpK::Select || n.k == OpK::Clamp || n.k == OpK::Convert || n.k == OpK::Gelu) followed[i] = 1;
+        if (elementwise(n)) followed[i] = 1;
     for (const Node& d : g.nodes) {
       if (d.k != OpK::DotGeneral || d.ty.rank() != 2 || !d.a0.empty()) continue;
       DotForm f = dot_form(d);
@@ -1028,7 +1076,7 @@ struct Planner {
       // 8192 x 18432 118 and 141; 32 x 8192 x 8192 39 and 37); from 4096 on, up to 4096 columns, it is the three-launch plan of those
       // models' last layers that is kept, not the time (32 x 1000 x 4096 12 us cut, 7 not).
       const bool dense = followed[d.id] && info(a).size == 2 && !f.b_k_contig && f.M > 16 && f.M <= 32 && f.K >= (f.N <= 4096 ? 4096 : 16384);
-      if (S == 1 && (few || dense)) {   // two workgroups per compute unit, slices of at least 512
+      if (S == 1 && (few || dense || held(d))) {   // two workgroups per compute unit, slices of at least 512
         while (S < 256 && tiles * S < 512 && f.K / (2 * S) >= 512) S *= 2;
       } else if (S == 1) {
         for (int q = 2; q <= 256 && f.K / q >= 256; q *= 2) {

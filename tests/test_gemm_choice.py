@@ -93,3 +93,29 @@ def test_long_matrices_against_few_rows_are_cut_on_the_ring_skeleton(dt, m, n, k
 def test_which_products_without_a_consumer_are_cut(dt, m, n, k, cut):
     rep = rx.compile_offline(dot_module(m, n, k, dt, dt, False, False)[0])
     assert (int(re.search(r"kind=gemm_\w+ grid=\d+x(\d+)x1", rep).group(1)) > 1) == cut
+
+
+HELD = """module {
+  func.func @main(%%arg0: tensor<%(m)dx2048x%(dt)s>, %%arg1: tensor<1024x2048x%(dt)s>, %%arg2: tensor<%(m)dx1024x%(dt)s>) -> (%(types)s) {
+    %%0 = stablehlo.dot_general %%arg0, %%arg1, contracting_dims = [1] x [1], precision = [DEFAULT, DEFAULT] : (tensor<%(m)dx2048x%(dt)s>, tensor<1024x2048x%(dt)s>) -> T
+%(body)s
+  }
+}
+"""
+D = "    %1 = stablehlo.subtract %0, %arg2 : T\n"
+TWO = D + "    %2 = stablehlo.multiply %1, %1 : T\n    %3 = stablehlo.tanh %1 : T\n    return %2, %3 : T, T"
+ONE = D + "    %2 = stablehlo.tanh %1 : T\n    return %2 : T"
+JOINED = D + "    %2 = stablehlo.tanh %1 : T\n    %3 = stablehlo.multiply %1, %2 : T\n    return %3 : T"
+LATE = D + "    %2 = stablehlo.tanh %1 : T\n    %3 = stablehlo.multiply %1, %2 : T\n    %4 = stablehlo.multiply %3, %3 : T\n    %5 = stablehlo.exponential %3 : T\n    return %4, %5 : T, T"
+EXACT = D + "    %2 = stablehlo.abs %1 : T\n    %3 = stablehlo.negate %1 : T\n    return %2, %3 : T, T"
+
+
+# what is computed from the product: several results of one value, one result, one result by two ways, one value by two ways that
+# several results are computed from, several results without a rounding of their own
+@pytest.mark.parametrize("dt,m,body,results,cut", [("bf16", 185, TWO, 2, True), ("f16", 64, TWO, 2, True), ("bf16", 185, ONE, 1, False), ("bf16", 185, JOINED, 1, False),
+                                                   ("bf16", 185, LATE, 2, False), ("bf16", 185, EXACT, 2, False), ("bf16", 4096, TWO, 2, False)])
+def test_products_that_several_results_are_computed_from_are_held_in_f32(dt, m, body, results, cut):
+    ty = "tensor<%dx1024x%s>" % (m, dt)
+    text = HELD % {"m": m, "dt": dt, "types": ", ".join([ty] * results), "body": body}
+    rep = rx.compile_offline(re.sub(r"\bT\b", ty, text))
+    assert (int(re.search(r"kind=gemm\w* grid=\d+x(\d+)x1", rep).group(1)) > 1) == cut
