@@ -95,3 +95,26 @@ RX_CHECK_G(rx_check_g_f8b_nn, rx_el_f8b, float, 16, 16, 1, 1, 8, 3, 1, true, tru
 RX_CHECK_X(rx_check_x_nt, 128, 256, 2, 4, 1, true, true, 301, 277, 131)
 RX_CHECK_X(rx_check_x_nn, 128, 128, 2, 2, 2, true, false, 512, 512, 784)
 RX_CHECK_X(rx_check_x_tn, 128, 128, 2, 2, 1, false, false, 300, 200, 100)
+
+// direct convolution on split operands: whole and partial slabs, features and tiles, strides and dilations, one group and several
+struct rx_check_conv_epi {
+  float* out;
+  int O, HO, WO;
+  template <int NV>
+  __device__ __forceinline__ void operator()(const float (&acc)[NV], int b, int o, int y, int x) const {
+#pragma unroll
+    for (int l = 0; l < NV; ++l) out[((b * O + o) * HO + y) * WO + x + l] = acc[l];
+  }
+};
+extern "C" __global__ __launch_bounds__(256, 2) void rx_check_conv_x(const float* x, const float* w, const rx_u8* ws, float* out) {
+  rx_check_conv_epi epi{out, 128, 112, 112};
+  rx_conv_body_x<4, 64, 112, 112, 128, 3, 3, 1, 1, 1, 1, 1, 1, 112, 112, 4, 28, 4, 1, rx_check_conv_epi>(x, w, ws, epi);
+}
+extern "C" __global__ __launch_bounds__(512, 2) void rx_check_conv_x_groups(const float* x, const float* w, const rx_u8* ws, float* out) {
+  rx_check_conv_epi epi{out, 70, 13, 11};
+  rx_conv_body_x<2, 40, 28, 30, 70, 3, 5, 2, 2, 1, 2, 1, 0, 13, 11, 3, 6, 2, 4, rx_check_conv_epi>(x, w, ws, epi);
+}
+extern "C" __global__ __launch_bounds__(256) void rx_check_split_filter(const float* w, rx_u8* ws) {
+  __shared__ float lds[16 * (32 * 15 + 1)];
+  rx_split_filter<70, 40, 15>(w, ws, blockIdx.x, lds);
+}

@@ -2457,3 +2457,341 @@ RX_DEV void rx_conv_body(const float* __restrict__ x, const float* __restrict__ 
     }
   }
 }
+
+// ===========================================================================
+// Direct convolution of f32 images on the bf16 matrix cores: every element as a sum of three bf16 numbers, six terms a product
+// and the two kinds of input that do not split as in rx_gemm_body_x; image, filter and result as in rx_conv_body.
+// What bounds it is the matrix cores at the clock that power leaves (1.7 to 1.8 GHz with all of them busy): six 16 x 16 x 32
+// MFMAs per 32 channels and tap, 224 workgroups of 8 wavefronts.  Of the 71 us that 256 -> 256 features on four 56 x 56
+// images take, staging is 7, the filter's loads 3 and the pixels' LDS reads 3 (timed with each switched off).
+// So the image is split once per tile, between the load and the LDS patch, [pixel][plane][32 channels], where every tap
+// reads it; the filter is split once per call by a launch of its own (rx_split_filter) into the order in which the
+// wavefronts take it from L2 straight into registers, one tap ahead (three where few pixels leave the registers).  A pixel
+// of the patch takes 208 bytes: sixteen consecutive pixels then read different banks.  The five small terms have
+// accumulators of their own, as there is no running sum for them to disturb otherwise.  A tile is up to 112 pixels: with 32
+// features per wavefront the sums take 112 registers, two wavefronts fit a SIMD; the channels are cut into
+// groups of wavefronts rather than the tile into smaller ones, which would read more of the filter (choose_conv_split).
+// Four images, 3 x 3, rx_conv_body or the product on the window matrix -> this kernel, us (TFLOP/s): 112 x 112, 64 -> 128: 72 ->
+// 39 (190); 56 x 56, 128 -> 256: 76 -> 40 (185), 256 -> 256: 142 -> 68 (218); 28 x 28, 256 -> 512: 85 -> 44 (168), 512 -> 512:
+// 166 -> 69 (215); 14 x 14, 512 -> 512: 51 -> 33 (112).  Splitting the filters of all of these: 25 (92 MB).
+// Error against 64 bits (2-norm, N(0,1)): 64 channels 9.8e-8 (f32 MFMAs 4.3e-7), 256 2.0e-7 (4.4e-7 and more), 512 1.9e-7 (3.8e-7).
+// ===========================================================================
+// The filter in fragment order: [slab of 32 channels][tap][block of 16 features][plane][lane][8 channels] (lane: feature lane % 16,
+// channels 8 (lane / 16) ..), zeros past O and C; after it, per slab and block, the largest magnitude and whether an element did not split.
+template <int O, int C, int TAPS>
+struct rx_filter_x {
+  static constexpr int NS = (C + 31) / 32, NOB = (O + 127) / 128 * 8;
+  static constexpr int FRAGS = NS * TAPS * NOB * 3 * 1024;   // bytes
+  static constexpr int BYTES = FRAGS + NS * NOB * 8;
+};
+// One workgroup of 256 threads: the fragments of block `bid` = slab * NOB + block of features.
+template <int O, int C, int TAPS>
+RX_DEV void rx_split_filter(const float* __restrict__ w, rx_u8* __restrict__ out, int bid, float* lds) {
+  typedef rx_filter_x<O, C, TAPS> F;
+  constexpr int ROW = 32 * TAPS, LDR = ROW + 1;   // floats of a feature in this slab
+  __shared__ int top, odd_any;
+  const int tid = threadIdx.x, s = bid / F::NOB, ob = bid % F::NOB;
+  if (tid == 0) { top = 0; odd_any = 0; }
+  const int left = (C - s * 32) * TAPS;
+  for (int e = tid; e < 16 * ROW; e += 256) {
+    const int o = ob * 16 + e / ROW, q = e % ROW;
+    lds[e / ROW * LDR + q] = o < O && q < left ? w[((long long)o * C + s * 32) * TAPS + q] : 0.f;
+  }
+  __syncthreads();
+  float mx = 0.f;
+  bool odd = false;
+  for (int it = tid; it < TAPS * 64; it += 256) {
+    const int tap = it >> 6, lane = it & 63;
+    rx_split4 sp[2];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const float* at = lds + (lane & 15) * LDR + (8 * (lane >> 4) + 2 * p) * TAPS + tap;
+      float x = at[0], y = at[TAPS];
+      mx = __builtin_fmaxf(mx, __builtin_fmaxf(__builtin_fabsf(x), __builtin_fabsf(y)));
+      rx_static_for<0, 6>([&](auto H) { rx_split_step<decltype(H)::value>(x, y, sp[p / 2], p % 2, odd); });
+    }
+    rx_u8* at = out + ((long long)(s * TAPS + tap) * F::NOB + ob) * 3072 + lane * 16;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *(rx_i32x4*)(at + p * 1024) = rx_i32x4{(int)sp[0].p[p][0], (int)sp[0].p[p][1], (int)sp[1].p[p][0], (int)sp[1].p[p][1]};
+  }
+  // (magnitudes are ordered as their bits are)
+  __hip_atomic_fetch_max(&top, __builtin_bit_cast(int, mx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (odd) odd_any = 1;
+  __syncthreads();
+  if (tid == 0) *(long long*)(out + F::FRAGS + (long long)bid * 8) = (long long)(rx_u32)top | (long long)odd_any << 32;
+}
+
+// WF wavefronts, each with 32 features and all pixels of the tile, per group; group g contracts slabs g, g + KG, ..
+template <int B, int C, int H, int W, int O, int KH, int KW, int SH, int SW, int DH, int DW, int PT, int PL, int HO, int WO, int TR, int TC, int WF, int KG, class Epi>
+RX_DEV void rx_conv_body_x(const float* __restrict__ x, const float* __restrict__ w, const rx_u8* __restrict__ ws, const Epi& epi) {
+  constexpr int TAPS = KH * KW, NT = WF * 64;
+  typedef rx_filter_x<O, C, TAPS> F;
+  constexpr int PR = (TR - 1) * SH + (KH - 1) * DH + 1, PW = (TC - 1) * SW + (KW - 1) * DW + 1, NPP = PR * PW;   // patch of the image
+  constexpr int PX = 208, PXF = 144;                                 // bytes of a pixel of the patch: three planes of 32 channels; 32 f32 numbers
+  constexpr int NPX = TR * TC, NPB = (NPX + 15) / 16;
+  constexpr int NS = F::NS, NSG = (NS + KG - 1) / KG;
+  constexpr int TX = (WO + TC - 1) / TC, TILES = (HO + TR - 1) / TR * TX, FG = (O + 32 * WF - 1) / (32 * WF);
+  constexpr int NI = (NPP * 4 + NT - 1) / NT;                        // (pixel, 8 channels) per thread
+  constexpr int HW = H * W;
+  static_assert((long long)C * HW * 4 < (1ll << 31), "32-bit offsets in an image");
+  extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];
+  __shared__ int again[16], largest[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave / WF, wf = wave % WF, t = tid - grp * NT;
+  RX_LDS rx_u8* const patch = (RX_LDS rx_u8*)rx_smem + grp * (NPP * PX);
+  // workgroups of one group of features share an XCD where the groups divide the XCDs (or the other way round)
+  const int fg = blockIdx.x % FG, tile = blockIdx.x / FG;
+  const int b = tile / TILES, y0 = tile % TILES / TX * TR, x0 = tile % TX * TC;
+  const int o0 = fg * 32 * WF + wf * 32, kk = lane >> 4, li = lane & 15;
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (long long)b * C * HW), 0, (unsigned)C * (unsigned)HW * 4u, 0x00020000);
+
+  // loader: item i of this thread is 8 channels of one pixel; outside of the image, and past the channels, reads give zero
+  float raw[NI][8];
+  auto load = [&](int s) __attribute__((always_inline)) {
+    int tt = t;
+    asm volatile("" : "+v"(tt));                                      // positions are computed for each slab: they would take registers all the time
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int e = i * NT + tt, oct = e / NPP, px = e % NPP;
+      const int y = y0 * SH - PT + px / PW, xc = x0 * SW - PL + px % PW;
+      const unsigned at = e < NPP * 4 && y >= 0 && y < H && xc >= 0 && xc < W ? (unsigned)(oct * 8 * HW + y * W + xc) * 4u : 0xf0000000u;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        raw[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rx, at + (unsigned)(j * HW * 4), s * (32 * HW * 4), 0));
+    }
+  };
+  float la = 0.f;
+  bool odd = false;
+  auto put = [&]() __attribute__((always_inline)) {
+    int tt = t;
+    asm volatile("" : "+v"(tt));
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int e = i * NT + tt;
+      if (i + 1 < NI || e < NPP * 4) {
+        RX_LDS rx_u8* const at = patch + e % NPP * PX + e / NPP * 16;
+        rx_split4 sp[2];
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          float u = raw[i][2 * p], v = raw[i][2 * p + 1];
+          la = __builtin_fmaxf(la, __builtin_fmaxf(__builtin_fabsf(u), __builtin_fabsf(v)));
+          rx_static_for<0, 6>([&](auto Q) { rx_split_step<decltype(Q)::value>(u, v, sp[p / 2], p % 2, odd); });
+        }
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *(RX_LDS rx_i32x4*)(at + p * 64) = rx_i32x4{(int)sp[0].p[p][0], (int)sp[0].p[p][1], (int)sp[1].p[p][0], (int)sp[1].p[p][1]};
+      }
+    }
+  };
+  int pofs[NPB];   // a lane's pixel of each block, in pixels of the patch
+#pragma unroll
+  for (int i = 0; i < NPB; ++i) {
+    int p = i * 16 + li;
+    if (p >= NPX) p = NPX - 1;                                        // ragged last block: those results are not stored
+    pofs[i] = p / TC * SH * PW + p % TC * SW;
+  }
+  rx_f32x4v hi[NPB][2], lo[NPB][2];                                   // the h h terms; the five small ones
+  auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NPB; ++i)
+#pragma unroll
+      for (int f = 0; f < 2; ++f) hi[i][f] = lo[i][f] = rx_f32x4v{0.f, 0.f, 0.f, 0.f};
+  };
+  auto barrier = [&]() __attribute__((always_inline)) {               // LDS operations are complete, loads into registers stay under way
+    asm volatile("" ::: "memory");
+    rx_wait_vmcnt_lgkm0<63>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  constexpr int FD = NPB <= 4 ? 4 : 2;                                // taps whose filters are in registers or on their way
+  rx_bf16x8 fw[FD][2][3], fp[2][3];
+  auto filter = [&](auto BUF, int s, int tap) __attribute__((always_inline)) {
+    const rx_u8* const at = ws + ((long long)(s * TAPS + tap) * F::NOB + o0 / 16) * 3072;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int p = 0; p < 3; ++p) fw[decltype(BUF)::value][f][p] = *(const rx_bf16x8*)(at + (f * 3 + p) * 1024 + lane * 16);
+  };
+  RX_LDS rx_u8* pa[NPB];
+#pragma unroll
+  for (int i = 0; i < NPB; ++i) pa[i] = patch + pofs[i] * PX + kk * 16;
+  auto pixels = [&](auto BUF, auto I, auto TAP) __attribute__((always_inline)) {
+    constexpr int tap = decltype(TAP)::value, at = (tap / KW * DH * PW + tap % KW * DW) * PX;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) fp[decltype(BUF)::value][p] = *(const RX_LDS rx_bf16x8*)(pa[decltype(I)::value] + at + p * 64);
+  };
+  auto filters_first = [&](int s) __attribute__((always_inline)) {
+    rx_static_for<0, (FD - 1 < TAPS ? FD - 1 : TAPS)>([&](auto T) { filter(T, s, decltype(T)::value); });
+  };
+  // one slab: steps (tap, block); the next step's pixels are read, and the next tap's filter requested, under this step's MFMAs
+  auto compute = [&](int s) __attribute__((always_inline)) {
+    pixels(rx_int<0>{}, rx_int<0>{}, rx_int<0>{});
+    rx_static_for<0, TAPS * NPB>([&](auto ST) {
+      constexpr int st = decltype(ST)::value, tap = st / NPB, i = st % NPB;
+      if constexpr (i == 0 && tap + FD - 1 < TAPS) filter(rx_int<(tap + FD - 1) % FD>{}, s, tap + FD - 1);
+      if constexpr (st + 1 < TAPS * NPB) pixels(rx_int<(st + 1) % 2>{}, rx_int<(st + 1) % NPB>{}, rx_int<(st + 1) / NPB>{});
+      const rx_bf16x8 (&u)[3] = fp[st % 2];
+      const rx_bf16x8 (&v)[2][3] = fw[tap % FD];
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          rx_f32x4v& c = q < 5 ? lo[i][f] : hi[i][f];
+          c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u[q == 0 ? 2 : (q == 2 || q == 3 ? 1 : 0)], v[f][q == 1 ? 2 : (q == 2 || q == 4 ? 1 : 0)], c, 0, 0, 0);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  // sums of the groups, in group order: group g ends with blocks q = 2 i + f, q % KG = g
+  auto combine = [&]() __attribute__((always_inline)) {
+    if constexpr (KG > 1) {
+      RX_LDS rx_f32x4v* const part = (RX_LDS rx_f32x4v*)rx_smem;
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NPB; ++i)
+#pragma unroll
+        for (int f = 0; f < 2; ++f) part[((wf * NPB * 2 + 2 * i + f) * KG + grp) * 64 + lane] = hi[i][f];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NPB; ++i)
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+          if ((2 * i + f) % KG == grp) {
+            rx_f32x4v c = part[(wf * NPB * 2 + 2 * i + f) * KG * 64 + lane];
+#pragma unroll
+            for (int g = 1; g < KG; ++g) c += part[((wf * NPB * 2 + 2 * i + f) * KG + g) * 64 + lane];
+            hi[i][f] = c;
+          }
+    }
+  };
+  auto vote = [&](int mine) __attribute__((always_inline)) {
+    const int any = __builtin_amdgcn_ballot_w64((mine & 1) != 0) != 0 ? 1 : 0, both = any | (__builtin_amdgcn_ballot_w64((mine & 2) != 0) != 0 ? 2 : 0);
+    __syncthreads();
+    if (lane == 0) again[wave] = both;
+    __syncthreads();
+    int r = 0;
+#pragma unroll
+    for (int u = 0; u < WF * KG; ++u) r |= again[u];
+    return __builtin_amdgcn_readfirstlane(r);
+  };
+
+  clear();
+  load(grp < NS ? grp : 0);
+  filters_first(grp < NS ? grp : 0);
+  put();
+  barrier();
+  for (int i = 0; i < NSG; ++i) {
+    const int s = grp + i * KG;
+    const bool more = s + KG < NS;
+    if (more) load(s + KG);
+    if (s < NS) compute(s);
+    if (i + 1 < NSG) {
+      if (more) filters_first(s + KG);
+      barrier();
+      if (more) put();
+      barrier();
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NPB; ++i)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) hi[i][f] += lo[i][f];
+  combine();
+
+  // Elements that did not split, of the patch or of the filter; sums that are not finite
+  float fin = 0.f;
+#pragma unroll
+  for (int i = 0; i < NPB; ++i)
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+      if ((2 * i + f) % KG == grp)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) fin = __builtin_fmaf(hi[i][f][r], 0.f, fin);
+  float lb = 0.f;
+  for (int e = tid; e < NS * 2 * WF; e += NT * KG) {
+    const long long m = *(const long long*)(ws + F::FRAGS + ((long long)(e / (2 * WF)) * F::NOB + fg * 2 * WF + e % (2 * WF)) * 8);
+    lb = __builtin_fmaxf(lb, __builtin_bit_cast(float, (int)m));
+    odd = odd || (m >> 32) != 0;
+  }
+  if (tid < 2) largest[tid] = 0;
+  int any = vote((fin != fin ? 2 : 0) | (odd ? 1 : 0));
+  if (any == 1) {
+    // lost bits matter only to a sum below K 2^-109 (max |x| + max |w|) (see rx_gemm_body_x)
+    __hip_atomic_fetch_max(&largest[0], __builtin_bit_cast(int, la), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_max(&largest[1], __builtin_bit_cast(int, lb), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    const float least = (__builtin_bit_cast(float, largest[0]) + __builtin_bit_cast(float, largest[1])) * ((float)(C * TAPS) * 0x1p-109f);
+    bool low = false;
+#pragma unroll
+    for (int i = 0; i < NPB; ++i)
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+        if ((2 * i + f) % KG == grp)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) low = low || (o0 + 16 * f + li < O && !(__builtin_fabsf(hi[i][f][r]) >= least));
+    any = vote(low ? 2 : 0);
+  }
+  if (any & 2) {
+    // contracted again with f32 MFMAs, the patch in f32 in its place, the filter as it is stored
+    clear();
+#pragma unroll 1
+    for (int i = 0; i < NSG; ++i) {
+      const int s = grp + i * KG;
+      __syncthreads();
+      if (s < NS) {
+        load(s);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          const int e = j * NT + t;
+          if (j + 1 < NI || e < NPP * 4) {
+            RX_LDS rx_u8* const at = patch + e % NPP * PXF + e / NPP * 32;
+            *(RX_LDS rx_f32x4v*)at = rx_f32x4v{raw[j][0], raw[j][1], raw[j][2], raw[j][3]};
+            *(RX_LDS rx_f32x4v*)(at + 16) = rx_f32x4v{raw[j][4], raw[j][5], raw[j][6], raw[j][7]};
+          }
+        }
+      }
+      __syncthreads();
+      if (s < NS)
+#pragma unroll 1
+        for (int tap = 0; tap < TAPS; ++tap) {
+          struct F8 { float f[8]; } v[2];
+#pragma unroll
+          for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const int o = o0 + 16 * f + li, c = s * 32 + 8 * kk + j;
+              v[f].f[j] = o < O && c < C ? w[((long long)(o < O ? o : 0) * C + (c < C ? c : 0)) * TAPS + tap] : 0.f;
+            }
+          const int at = (tap / KW * DH * PW + tap % KW * DW) * PXF;
+#pragma unroll
+          for (int j = 0; j < NPB; ++j) {
+            const RX_LDS rx_u8* const p = patch + pofs[j] * PXF + kk * 32 + at;
+            struct { rx_i32x4 a, b; } both = {*(const RX_LDS rx_i32x4*)p, *(const RX_LDS rx_i32x4*)(p + 16)};
+#pragma unroll
+            for (int f = 0; f < 2; ++f) rx_el_f32::mma(hi[j][f], __builtin_bit_cast(rx_i32x8, both), __builtin_bit_cast(rx_i32x8, v[f]));
+          }
+        }
+    }
+    combine();
+  }
+  // a lane holds pixels 4 (lane / 16) .. + 3 of a block for feature lane % 16 (see rx_conv_body)
+  int ol = o0 + li;
+  asm volatile("" : "+v"(ol));                                        // (what the epilogue computes from the feature stays behind the contraction)
+#pragma unroll
+  for (int i = 0; i < NPB; ++i)
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      const int o = ol + 16 * f, p = i * 16 + 4 * kk;
+      if ((2 * i + f) % KG != grp || o >= O) continue;
+      constexpr int NV = WO % 4 == 0 && TC % 4 == 0 ? 4 : 1;         // whole vectors: rows of the result and of the tile are multiples of 4 words
+#pragma unroll
+      for (int r = 0; r < 4; r += NV) {
+        const int yo = y0 + (p + r) / TC, xo = x0 + (p + r) % TC;
+        const bool inside = p + r < NPX && yo < HO && (WO % TC == 0 || xo < WO);
+        float v[NV];
+#pragma unroll
+        for (int l = 0; l < NV; ++l) v[l] = hi[i][f][r + l];
+        if constexpr (rx_epi_masks_rows<Epi>::value) epi(v, b, o, yo, xo, inside);
+        else if (inside) epi(v, b, o, yo, xo);
+      }
+    }
+}

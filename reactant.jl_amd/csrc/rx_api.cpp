@@ -262,6 +262,7 @@ rx::PlanOptions plan_options() {
   if (const char* e = getenv("RX_EPILOGUES")) o.product_epilogues = atoi(e) != 0;
   if (const char* e = getenv("RX_EPILOGUE_INIT")) o.epilogue_init = atoi(e) != 0;
   if (const char* e = getenv("RX_CHAIN_CONVS")) o.chain_convs = atoi(e) != 0;
+  if (const char* e = getenv("RX_CONV_SPLIT")) o.split_convs = atoi(e) != 0;
   if (const char* e = getenv("RX_IN_PLACE")) o.in_place_updates = atoi(e) != 0;
   if (const char* e = getenv("RX_CHAIN_STEPS")) o.chain_steps = atoi(e);
   if (const char* e = getenv("RX_CHAIN_TILE")) { int v[3] = {0, 0, 0}; if (sscanf(e, "%d,%d,%d", &v[0], &v[1], &v[2]) >= 1) { o.chain_tile[0] = v[0]; o.chain_tile[1] = v[1]; o.chain_tile[2] = v[2]; } }
@@ -845,10 +846,23 @@ RX_EXPORT void PjRtBufferFree(RxBuffer* b) {
   delete b;
 }
 
+namespace {
+// Split filters are temporaries: a module that RxExecuteNoAlloc holds without them is planned without them.
+rx::Plan plan_module(const char* text, size_t len, rx::PlanOptions opt) {
+  rx::Plan p = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
+  const char* force = getenv("RX_CONV_SPLIT");
+  if (p.split_filters > 0 && !(force && atoi(force) == 2) && p.temporary_bytes() > (int64_t)RX_NOALLOC_SCRATCH_BYTES) {
+    opt.split_convs = false;
+    rx::Plan plain = rx::make_plan(rx::parse_module(text, len, false), opt);
+    if (plain.temporary_bytes() <= (int64_t)RX_NOALLOC_SCRATCH_BYTES) return plain;
+  }
+  return p;
+}
+}  // namespace
+
 RX_EXPORT int RxCompileOffline(const char* text, size_t len, int with_source, char** report) {
   try {
-    rx::Graph g = rx::parse_module(text, len);
-    rx::Plan p = rx::make_plan(g, plan_options());
+    rx::Plan p = plan_module(text, len, plan_options());
     std::string code = rx::rtc_compile(p.source, "gfx950");
     if (report) {
       std::string r = p.report() + "code object: " + std::to_string(code.size()) + " bytes\n";
@@ -869,8 +883,7 @@ void load_plan(RxExecutable* ex, rx::PlanOptions opt) {
   RxDevice* d = ex->device;
   if (d->waits_failed) opt.single_pass_scan = false;   // a wait between workgroups has expired on this device before
   try {
-    rx::Graph g = rx::parse_module(ex->text.data(), ex->text.size());
-    ex->plan = rx::make_plan(g, opt);
+    ex->plan = plan_module(ex->text.data(), ex->text.size(), opt);
   } catch (const std::exception& e) {
     // same shape of message as the reference: module text followed by the status (API.cpp:1499-1505)
     throw Error(ex->text.substr(0, 4000) + "\n" + e.what());

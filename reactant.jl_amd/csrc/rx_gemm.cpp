@@ -513,6 +513,15 @@ std::string gemm_instance(const GemmChoice& c, const std::string& kbase, const s
   return o.str();
 }
 
+// The matrix product on the window matrix: 70 TFLOP/s, a layout map of the result, three launches, and the window matrix
+// written and read when there are more than 128 features.  Up to 128 it is evaluated while the tiles are loaded, 0.04 us per
+// k whatever the number of pixels (28 x 28 images, 128 -> 128: 50 us for one and 48 for four; 14 x 14, 96 -> 96: 37)
+static double conv_product_us(int64_t B, int64_t C, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO) {
+  const double flops = 2.0 * (double)B * (double)O * (double)HO * (double)WO * (double)C * (double)(KH * KW);
+  const double window_bytes = O > 128 ? 2.0 * 4.0 * (double)B * (double)C * (double)(KH * KW) * (double)HO * (double)WO : 0.0;
+  return std::max(flops / 70e6, O > 128 ? 0.0 : 0.04 * (double)(C * KH * KW)) + (window_bytes + 2.0 * 4.0 * (double)B * (double)O * (double)HO * (double)WO) / 5e6 + 5.0 + 8.0;
+}
+
 ConvChoice choose_conv(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl,
                        int64_t sh, int64_t sw, int64_t dh, int64_t dw) {
   ConvChoice c;
@@ -553,18 +562,15 @@ ConvChoice choose_conv(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, in
   // workgroup of this kernel passes all channels of its 64 features through LDS for one tile of one image, about 1.5 us
   // per slab however few pixels the tile has.  Estimates in microseconds, fitted to 3 x 3 layers of 64 to 512 features
   // on 7 x 7 to 56 x 56 images in batches of 4 and 32 (512 -> 512 on 14 x 14, 4 images: 0.097 ms direct against 0.055;
-  // 32 images of 256 -> 256: 0.086 against 0.103): slabs of max(1.5 us, 1.35 x their MFMA time) here; 70 TFLOP/s, a
-  // window matrix written and read when there are more than 128 features, a layout map of the result and two more
-  // launches there.
+  // 32 images of 256 -> 256: 0.086 against 0.103): slabs of max(1.5 us, 1.35 x their MFMA time) here, conv_product_us there.
   {
     const int64_t tiles = (HO + c.rows - 1) / c.rows, npb = (c.rows * WO + 15) / 16;
     const double rounds = (double)((B * tiles * groups + 255) / 256);
     const double nslab = (double)((C + slab - 1) / slab), nstep = (double)(KH * KW * (slab / 4));
     const double direct_us = rounds * nslab * std::max(1.5, 1.35 * (double)npb * nstep * 32.0 / 2200.0) + 5.0;
-    const double flops = 2.0 * (double)B * (double)O * (double)HO * (double)WO * (double)C * (double)(KH * KW);
-    const double window_bytes = O > 128 ? 2.0 * 4.0 * (double)B * (double)C * (double)(KH * KW) * (double)HO * (double)WO : 0.0;
-    const double product_us = flops / 70e6 + (window_bytes + 2.0 * 4.0 * (double)B * (double)O * (double)HO * (double)WO) / 5e6 + 5.0 + 8.0;   // three launches
+    const double product_us = conv_product_us(B, C, O, KH, KW, HO, WO);
     const char* force = getenv("RX_CONV_DIRECT");   // 2: this kernel wherever it covers the case
+    c.us = direct_us;
     if (direct_us > product_us && !(force && atoi(force) == 2)) { c.rows = 0; return c; }
   }
   c.slab = slab;
@@ -573,6 +579,86 @@ ConvChoice choose_conv(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, in
   c.lds_bytes = (unsigned)lds_of(c.rows);
   c.ok = true;
   return c;
+}
+
+ConvSplitChoice choose_conv_split(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO,
+                                  int64_t sh, int64_t sw, int64_t dh, int64_t dw) {
+  ConvSplitChoice best;
+  if (getenv("RX_MFMA") && atoi(getenv("RX_MFMA")) == 0) return best;
+  const int64_t taps = KH * KW, ns = (C + 31) / 32, nob = (O + 127) / 128 * 8;
+  // Fewer channels than a slab, or features than two wavefronts' of two groups, would be padding; more taps do not fit the
+  // splitting kernel's LDS.
+  if (B < 1 || HO < 1 || WO < 1 || C < 32 || O <= 64 || taps > 25 || sh < 1 || sw < 1 || dh < 1 || dw < 1 || sh > 4 || sw > 4) return best;
+  if (C * H * W * 4 >= ((int64_t)1 << 31) || H * W >= ((int64_t)1 << 22) || B * O * HO * WO >= ((int64_t)1 << 31) || B * C * H * W >= ((int64_t)1 << 31) || ns * taps * nob * 3072 >= ((int64_t)1 << 31)) return best;
+  for (int wf : {4, 2, 1})
+    for (int kg : {1, 2, 4, 8}) {
+      if (wf * kg != 4 && wf * kg != 8) continue;
+      const int64_t fg = (O + 32 * wf - 1) / (32 * wf), nsg = (ns + kg - 1) / kg, nt = 64 * wf;
+      for (int64_t parts = 1; parts <= (WO + 7) / 8; ++parts) {
+        int64_t tc = (WO + parts - 1) / parts;
+        if (WO % 4 == 0) tc = (tc + 3) / 4 * 4;
+        for (int64_t tr = 1; tr <= HO && tr * tc <= 112; ++tr) {
+          const int64_t npb = (tr * tc + 15) / 16;
+          const int64_t pw = (tc - 1) * sw + (KW - 1) * dw + 1, npp = ((tr - 1) * sh + (KH - 1) * dh + 1) * pw;
+          const int64_t ni = (npp * 4 + nt - 1) / nt;
+          if (npb * 16 + ni * 8 > 160) break;   // registers: sums and the next slab's elements
+          const int64_t lds = std::max(kg * npp * 208, kg > 1 ? wf * npb * 2 * kg * 1024 : (int64_t)0);
+          if (lds > 160 * 1024 - 256) break;
+          const int64_t wgs = B * ((HO + tr - 1) / tr) * ((WO + tc - 1) / tc) * fg;
+          // Wavefronts that share a SIMD, rounds of workgroups, cycles of a slab: 12 MFMAs per tap and pixel block, and 300 to
+          // stage 8 channels of 64 pixels, at the 1.75 GHz that are left while all matrix cores multiply; or the filter, which
+          // every workgroup reads from L2, at 9 TB/s
+          const bool pair = wf * kg == 4 && lds <= 80 * 1024 && wgs > 256;
+          const double share = wf * kg == 8 || pair ? 2.0 : 1.1, rounds = (double)((wgs + (pair ? 511 : 255)) / (pair ? 512 : 256));
+          const double body = rounds * (double)nsg * ((double)(taps * npb) * 192.0 + (double)ni * 300.0) * share / 1750.0;
+          const double us = (std::max(body, (double)(wgs * 32 * wf * C * taps) * 6.0 / 9e6) + 8.0 * rounds) * (parts > 1 ? 1.03 : 1.0);
+          if (!best.ok || us < best.us - 0.01) {
+            best.ok = true;
+            best.us = us;
+            best.rows = (int)tr;
+            best.cols = (int)tc;
+            best.wf = wf;
+            best.groups = kg;
+            best.grid = (unsigned)wgs;
+            best.block = (unsigned)(64 * wf * kg);
+            best.lds_bytes = (unsigned)lds;
+          }
+        }
+      }
+    }
+  // The filter: read once, written as 6 bytes an element, at 4 TB/s; the launch is shared by the filters of a module
+  best.us += 4.0 + 10.0 * (double)(O * C * taps) / 4e6;
+  best.filter_bytes = ns * taps * nob * 3072 + ns * nob * 8;
+  best.filter_grid = (unsigned)(ns * nob);
+  if (const char* e = getenv("RX_CONV_SPLIT_TILE")) {   // rows, columns, wavefronts of features, groups of channels
+    int v[4];
+    if (sscanf(e, "%d,%d,%d,%d", &v[0], &v[1], &v[2], &v[3]) == 4 && best.ok) {
+      const int64_t pw = (v[1] - 1) * sw + (KW - 1) * dw + 1, npp = ((v[0] - 1) * sh + (KH - 1) * dh + 1) * pw, npb = (v[0] * v[1] + 15) / 16;
+      const int64_t lds = std::max(v[3] * npp * 208, v[3] > 1 ? v[2] * npb * 2 * v[3] * 1024 : (int64_t)0);
+      if (v[0] < 1 || v[1] < 1 || v[2] < 1 || v[3] < 1 || v[0] * v[1] > 112 || (v[2] * v[3] != 4 && v[2] * v[3] != 8) || lds > 160 * 1024 - 256) throw Error("RX_CONV_SPLIT_TILE cannot be honoured");
+      best.rows = v[0]; best.cols = v[1]; best.wf = v[2]; best.groups = v[3];
+      best.block = 64 * v[2] * v[3];
+      best.lds_bytes = (unsigned)lds;
+      best.grid = (unsigned)(B * ((HO + v[0] - 1) / v[0]) * ((WO + v[1] - 1) / v[1]) * ((O + 32 * v[2] - 1) / (32 * v[2])));
+    }
+  }
+  return best;
+}
+
+bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl, int64_t sh, int64_t sw, int64_t dh, int64_t dw) {
+  if (getenv("RX_CONV_DIRECT") && atoi(getenv("RX_CONV_DIRECT")) == 0) return false;
+  const char* force = getenv("RX_CONV_SPLIT");   // 0: never; 2: wherever the kernel covers the case
+  if (force && atoi(force) == 0) return false;
+  const ConvSplitChoice c = choose_conv_split(B, C, H, W, O, KH, KW, HO, WO, sh, sw, dh, dw);
+  if (!c.ok) return false;
+  if (force && atoi(force) == 2) return true;
+  const ConvChoice d = choose_conv(B, C, H, W, O, KH, KW, HO, WO, pl, sh, sw, dh, dw);
+  const double product = conv_product_us(B, C, O, KH, KW, HO, WO);
+  // In us, kernels alone, f32 kernel or product -> this one with the splitting (7 to 15 by itself, 25 for all filters of
+  // VGG-11): 8 images of 14 x 14, 512 -> 512: 112 -> 54 + 14; 4 of 28 x 28, 256 -> 256: 53 -> 29 + 11; 8 of 56 x 56, 64 -> 128:
+  // 43 -> 23 + 9; 2 of 32 x 32, 64 -> 128: 11.3 -> 6.3 + 6.7; against the product: 4 of 14 x 14, 512 -> 512: 60 -> 34 + 15; one:
+  // 21 -> 18 + 14; 8 x 8: 15 -> 14 + 13; 2 of 10 x 10, 160 -> 160: 15 -> 7 + 8.  The product's estimate is a quarter too high.
+  return c.us < (d.ok ? d.us : 0.8 * product);
 }
 
 }  // namespace rx

@@ -61,8 +61,24 @@ struct ConvChoice {
   int slab = 0;             // channels per LDS stage
   unsigned grid[2] = {1, 1};
   unsigned lds_bytes = 0;
+  double us = 0;            // estimated time
 };
 ConvChoice choose_conv(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl,
                        int64_t sh = 1, int64_t sw = 1, int64_t dh = 1, int64_t dw = 1);
+
+// The same on the bf16 matrix cores (rx_conv_body_x).  `us`: estimated time, with that of splitting the filter.
+struct ConvSplitChoice {
+  bool ok = false;
+  int rows = 0, cols = 0;   // of the result per workgroup
+  int wf = 0, groups = 0;   // wavefronts of 32 features, groups of slabs of channels
+  unsigned grid = 1, block = 0, lds_bytes = 0;
+  int64_t filter_bytes = 0; // of the split filter (rx_filter_x)
+  unsigned filter_grid = 0;
+  double us = 0;
+};
+ConvSplitChoice choose_conv_split(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO,
+                                  int64_t sh, int64_t sw, int64_t dh, int64_t dw);
+// Is that kernel the faster one?  `pl`: zero columns before the image.
+bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl, int64_t sh, int64_t sw, int64_t dh, int64_t dw);
 
 }  // namespace rx

@@ -14,10 +14,6 @@
 #include "rx_ir.h"
 #include "rx_plan.h"
 
-namespace rx {
-Graph parse_module(const char* text, size_t len);
-}
-
 int main(int argc, char** argv) {
   int failures = 0;
   for (int i = 1; i < argc; ++i) {

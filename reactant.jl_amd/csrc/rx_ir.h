@@ -109,8 +109,8 @@ struct Graph {
   }
 };
 
-// Parse a module; functions called from @main are inlined.  Throws rx::Error.
-Graph parse_module(const char* text, size_t len);
+// Parse a module; functions called from @main are inlined.  Throws rx::Error.  `split_convs`: PlanOptions::split_convs.
+Graph parse_module(const char* text, size_t len, bool split_convs = true);
 
 // Constant payload helpers
 double splat_as_double(const Node& n);

@@ -3584,6 +3584,77 @@ struct Planner {
     plan.launches.push_back(L);
   }
 
+  // The filter of a convolution on split operands, in the order its kernel reads it: a buffer and the launch that writes it.
+  // The launches of filters that are arguments of the module run first, as one (merge_filter_splits).
+  struct FilterSplit {
+    int64_t O, C, taps;
+    unsigned grid;
+  };
+  std::map<int, int> split_of;                   // filter -> buffer
+  std::map<int, FilterSplit> filter_splits;      // that buffer -> sizes
+  int split_filter(int w, const ConvSplitChoice& cx) {
+    auto it = split_of.find(w);
+    if (it != split_of.end()) return it->second;
+    const TType& wt = g.nodes[w].ty;
+    const int buf = scratch(cx.filter_bytes);
+    const FilterSplit f{wt.dims[0], wt.dims[1], wt.dims[2] * wt.dims[3], cx.filter_grid};
+    Launch L;                                    // (its kernel follows in merge_filter_splits)
+    L.kind = "filter_split";
+    L.args = {buffer_for(w), buf};
+    plan.launches.push_back(L);
+    filter_splits[buf] = f;
+    return split_of[w] = buf;
+  }
+  Launch split_launch(const std::vector<std::pair<int, int>>& bufs, const std::vector<FilterSplit>& f) {
+    Launch L;
+    std::ostringstream o;
+    int64_t taps = 0;
+    for (auto& x : f) taps = std::max(taps, x.taps);
+    o << "// filters as sums of three bf16 numbers\nextern \"C\" __global__ __launch_bounds__(256) void @K@_split(";
+    for (size_t k = 0; k < f.size(); ++k) o << (k ? ", " : "") << "const float* __restrict__ w" << k << ", rx_u8* __restrict__ s" << k;
+    o << ") {\n  __shared__ float lds[" << 16 * (32 * taps + 1) << "];\n";
+    unsigned first = 0;
+    for (size_t k = 0; k < f.size(); ++k) {
+      o << "  if (blockIdx.x < " << first + f[k].grid << "u) { rx_split_filter<" << f[k].O << ", " << f[k].C << ", " << f[k].taps << ">(w" << k << ", s" << k << ", blockIdx.x - " << first
+        << "u, lds); return; }\n";
+      first += f[k].grid;
+      L.args.push_back(bufs[k].first);
+      L.args.push_back(bufs[k].second);
+      L.algo_bytes += 4.0 * (double)(f[k].O * f[k].C * f[k].taps) + (double)plan.buffers[bufs[k].second].bytes;
+    }
+    o << "}\n\n";
+    L.kernel = named("@K@_split", finalize(o.str()));
+    L.kind = "filter_split";
+    L.grid[0] = first;
+    L.block[0] = 256;
+    L.desc = "split filter";
+    return L;
+  }
+  void merge_filter_splits() {
+    plan.split_filters = (int)filter_splits.size();
+    if (filter_splits.empty()) return;
+    std::vector<char> written(plan.buffers.size(), 0);
+    for (auto& L : plan.launches)
+      for (int k = 0; k < L.n_outputs; ++k) written[L.args[L.args.size() - 1 - k]] = 1;
+    std::vector<std::pair<int, int>> bufs;
+    std::vector<FilterSplit> f;
+    std::vector<Launch> rest;
+    for (auto& L : plan.launches) {
+      const BufferDesc& B = plan.buffers[L.args.empty() ? 0 : L.args[0]];
+      if (L.kind == "filter_split" && (B.kind == BufferDesc::Param || B.kind == BufferDesc::Const) && !written[L.args[0]] && f.size() < 64) {
+        bufs.push_back({L.args[0], L.args[1]});
+        f.push_back(filter_splits.at(L.args[1]));
+      } else if (L.kind == "filter_split") {
+        rest.push_back(split_launch({{L.args[0], L.args[1]}}, {filter_splits.at(L.args[1])}));
+      } else {
+        rest.push_back(L);
+      }
+    }
+    plan.launches.clear();
+    if (!f.empty()) plan.launches.push_back(split_launch(bufs, f));
+    plan.launches.insert(plan.launches.end(), rest.begin(), rest.end());
+  }
+
   // ------------------------------------------------------------------ direct convolution
   // `root` is the convolution itself or the elementwise root that consumes it at the identity index (a bias, an
   // activation): that cone becomes the kernel's epilogue functor, as for a dot_general.
@@ -3594,7 +3665,12 @@ struct Planner {
     const TType& wt = g.nodes[cn.in[1]].ty;
     const bool shifted = !cn.a3.empty();   // the product with row shifts (16-bit images)
     ConvChoice cc;
-    if (!shifted) {
+    ConvSplitChoice cx;
+    if (!shifted && opt.split_convs && conv_split_pays(xt.dims[0], xt.dims[1], xt.dims[2], xt.dims[3], wt.dims[0], wt.dims[2], wt.dims[3], cn.ty.dims[2], cn.ty.dims[3],
+                                                       cn.a0[2], cn.a1[0], cn.a1[1], cn.a2[0], cn.a2[1]))
+      cx = choose_conv_split(xt.dims[0], xt.dims[1], xt.dims[2], xt.dims[3], wt.dims[0], wt.dims[2], wt.dims[3], cn.ty.dims[2], cn.ty.dims[3], cn.a1[0], cn.a1[1],
+                             cn.a2[0], cn.a2[1]);
+    if (!shifted && !cx.ok) {
       cc = choose_conv(xt.dims[0], xt.dims[1], xt.dims[2], xt.dims[3], wt.dims[0], wt.dims[2], wt.dims[3], cn.ty.dims[2], cn.ty.dims[3], cn.a0[2],
                        cn.a1[0], cn.a1[1], cn.a2[0], cn.a2[1]);
       if (!cc.ok) throw Error("internal: convolution node without a tiling");
@@ -3755,6 +3831,39 @@ struct Planner {
       L.algo_bytes = algo_bytes(all_in, {root});
       // of the results that are kept
       L.flops = 2.0 * (double)(cn.a3.size() == 8 ? cn.ty.dims[0] * cn.a3[5] * cn.a3[6] * cn.ty.dims[3] : cn.ty.numel()) * (double)wt.dims[1];
+      L.desc = describe(root);
+      plan.launches.push_back(L);
+      return;
+    }
+    if (cx.ok) {
+      const bool few = !choose_conv(xt.dims[0], xt.dims[1], xt.dims[2], xt.dims[3], wt.dims[0], wt.dims[2], wt.dims[3], cn.ty.dims[2], cn.ty.dims[3], cn.a0[2], cn.a1[0],
+                                    cn.a1[1], cn.a2[0], cn.a2[1]).ok;
+      const int64_t taps = wt.dims[2] * wt.dims[3];
+      const int split = split_filter(cn.in[1], cx);
+      o << "// direct convolution on split operands: " << xt.str() << " * " << wt.str() << " -> " << cn.ty.str() << ", tiles of " << cx.rows << " x " << cx.cols << " results, "
+        << cx.wf * 32 << " features, channels in " << cx.groups << " groups\n";
+      o << "extern \"C\" __global__ __launch_bounds__(" << cx.block << ", 2) void @K@_conv(const float* __restrict__ X, const float* __restrict__ Wt, const rx_u8* __restrict__ ws";
+      for (size_t k = 0; k < em.inputs.size(); ++k) o << ", const " << info(g.nodes[em.inputs[k]].ty.dt).stype << "* __restrict__ e" << k;
+      o << ", " << ost << "* __restrict__ out0) {\n";
+      o << "  @K@_epi epi{";
+      for (size_t k = 0; k < em.inputs.size(); ++k) o << "e" << k << ", ";
+      o << "out0};\n";
+      o << "  rx_conv_body_x<" << xt.dims[0] << ", " << xt.dims[1] << ", " << xt.dims[2] << ", " << xt.dims[3] << ", " << wt.dims[0] << ", " << wt.dims[2] << ", " << wt.dims[3] << ", "
+        << cn.a1[0] << ", " << cn.a1[1] << ", " << cn.a2[0] << ", " << cn.a2[1] << ", " << cn.a0[0] << ", " << cn.a0[2] << ", " << cn.ty.dims[2] << ", " << cn.ty.dims[3] << ", " << cx.rows
+        << ", " << cx.cols << ", " << cx.wf << ", " << cx.groups << ", @K@_epi>(X, Wt, ws, epi);\n}\n\n";
+      Launch L;
+      L.kernel = named("@K@_conv", finalize(o.str()));
+      L.kind = few ? "conv_few" : "conv";
+      L.grid[0] = cx.grid;
+      L.block[0] = cx.block;
+      L.lds_bytes = cx.lds_bytes;
+      L.args = {buffer_for(cn.in[0]), buffer_for(cn.in[1]), split};
+      for (int i : em.inputs) L.args.push_back(buffer_for(i));
+      L.args.push_back(buffer_for(root));
+      std::vector<int> all_in{cn.in[0], cn.in[1]};
+      for (int i : em.inputs) if (std::find(all_in.begin(), all_in.end(), i) == all_in.end()) all_in.push_back(i);
+      L.algo_bytes = algo_bytes(all_in, {root});
+      L.flops = 2.0 * (double)cn.ty.numel() * (double)(wt.dims[1] * taps);
       L.desc = describe(root);
       plan.launches.push_back(L);
       return;
@@ -5410,6 +5519,7 @@ struct Planner {
       plan.result_buffers.push_back(b);
     }
     merge_parameter_maps();
+    merge_filter_splits();
     // liveness over the launch list
     for (size_t li = 0; li < plan.launches.size(); ++li) {
       auto& L = plan.launches[li];
@@ -5424,6 +5534,13 @@ struct Planner {
 };
 
 }  // namespace
+
+int64_t Plan::temporary_bytes() const {
+  int64_t n = 0;
+  for (auto& b : buffers)
+    if ((b.kind == BufferDesc::Temp || b.kind == BufferDesc::Scratch) && !b.is_result && (b.first_def >= 0 || b.last_use >= 0)) n += (b.bytes + 255) & ~(int64_t)255;
+  return n;
+}
 
 std::string Plan::report() const {
   std::ostringstream o;

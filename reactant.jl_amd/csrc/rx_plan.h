@@ -44,6 +44,8 @@ struct Plan {
   double hlo_flops = 0, hlo_transcendentals = 0, hlo_bytes_accessed = 0, hlo_output_bytes = 0;
   double hlo_operand_bytes[2] = {0, 0};
   std::string report() const;          // text summary for debugging
+  int split_filters = 0;               // temporaries that hold a filter split in three
+  int64_t temporary_bytes() const;     // what its temporaries take when each has memory of its own (RxExecuteNoAlloc)
 };
 
 struct PlanOptions {
@@ -61,6 +63,7 @@ struct PlanOptions {
   bool merge_parameter_maps = true;  // plain maps that read only the module's arguments run first, several of them as one launch
   bool nhwc_regions = true;     // the same for regions with several readers per value (residual additions): transposed once on the way in and out where needed
   double nhwc_region_ratio = 1.5;   // a region is rebuilt when the transposes that disappear move this many times the bytes of those that are added (two residual blocks: 3 against 2 tensors, 0.129 -> 0.115 ms)
+  bool split_convs = true;      // f32 convolutions of many channels on the bf16 matrix cores, operands split in three
   bool pad_into_pools = true;   // zero padding of a pooled value (windows that do not overlap) moves onto the pooling's operand: no padding map
   bool epilogue_init = true;    // a bias added to a product on the streaming skeletons becomes the accumulators' first values
   bool row_fusion = true;       // fuse row reductions with their elementwise consumers
