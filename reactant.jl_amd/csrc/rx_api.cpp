@@ -241,6 +241,7 @@ rx::PlanOptions plan_options() {
   if (const char* e = getenv("RX_LDS_TILE2")) { int v[3]; if (sscanf(e, "%d,%d,%d", &v[0], &v[1], &v[2]) == 3) { o.lds_tile2[0] = v[0]; o.lds_tile2[1] = v[1]; o.lds_tile2[2] = v[2]; } }
   if (const char* e = getenv("RX_SLAB_YTILES")) o.slab_ytiles = atoi(e);
   if (const char* e = getenv("RX_LDS2_THREADS")) o.lds2_threads = atoi(e);
+  if (const char* e = getenv("RX_ONE_WORKGROUP_REDUCE")) o.one_workgroup_reduce = atoll(e);
   if (const char* e = getenv("RX_SINGLE_PASS_REDUCE")) o.single_pass_reduce = atoi(e) != 0;
   if (const char* e = getenv("RX_SINGLE_PASS_SCAN")) o.single_pass_scan = atoi(e) != 0;
   if (const char* e = getenv("RX_LDS_TRANSPOSE")) o.lds_transpose = atoi(e) != 0;

@@ -3915,7 +3915,11 @@ struct Planner {
     return s;
   }
 
-  // full reduction (all dims): two kernels
+  // full reduction (all dims): two kernels, or one workgroup of 16 wavefronts for up to 8192 elements, where the second launch
+  // and the gap before it cost more than other compute units would save.  Kernels of sum(sin.(x) .+ y), us, two launches and
+  // one: f32 4099 elements 8.2 and 3.9, 8192 8.2 and 4.0, 32768 8.1 and 6.9, 65536 8.1 and 12; f64 4096 8.3 and 3.9, 8192 8.4
+  // and 5.4, 16384 7.9 and 9.1.  A thread adds at most eight elements, as it does in the two-launch form.  Several
+  // transcendental functions per element: fewer elements.
   void emit_reduce_full(int root) {
     const Node& rn = g.nodes[root];
     const Node& inn = g.nodes[rn.in[0]];
@@ -3926,8 +3930,12 @@ struct Planner {
     const int vec = pick_vec(inn.ty);
     const int64_t nv = inn.ty.numel() / vec;
     const int U = 4;
+    int64_t slow_ops = 0;
+    for (int x : cone_nodes(rn.in[0])) slow_ops += g.nodes[x].k == OpK::Unary || g.nodes[x].k == OpK::Gelu || g.nodes[x].op == "power" || g.nodes[x].op == "atan2";
+    const bool one = n > 0 && inn.ty.numel() * std::max<int64_t>(1, slow_ops) <= opt.one_workgroup_reduce;
+    const int BLK = one ? 1024 : kBlock;
     int64_t tiles = (nv + (int64_t)kBlock * U - 1) / ((int64_t)kBlock * U);
-    const int G = (int)std::max<int64_t>(1, std::min<int64_t>(tiles, 2048));
+    const int G = one ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(tiles, 2048));
     const std::string k1 = "@K@_reduce", k2 = "@K@_reduce_final";
 
     Emitter em(g, [&](int x) { return mat[x]; });
@@ -3941,17 +3949,23 @@ struct Planner {
     em.direct_expr = vec_name;
     em.indent = 10;
     std::string val = em.emit(rn.in[0], root_index(dims));
-    std::string body = em.take_code();
+    std::string body = em.take_code(), one_init, one_code;
+    if (one) {   // the init value's operands come after the reduction's
+      em.indent = 4;
+      one_init = em.emit(rn.in[1], Index{});
+      one_code = em.take_code();
+    }
 
     std::ostringstream o;
-    o << "// reduce (pass 1): " << describe(rn.in[0]) << " -> partials\n";
-    o << signature(k1, em.inputs, {{ACC, "partial"}}) << " {\n";
+    o << "// reduce" << (one ? ": " : " (pass 1): ") << describe(rn.in[0]) << (one ? ", one workgroup\n" : " -> partials\n");
+    if (one) o << signature(k1, em.inputs, {{info(dt).stype, "out0"}}, BLK) << " {\n";
+    else o << signature(k1, em.inputs, {{ACC, "partial"}}) << " {\n";
     o << "  " << ACC << " acc[" << U << "];\n";
     o << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) acc[u] = " << red_identity(rn.red, dt) << ";\n";
-    o << "  for (" << it << " base = (" << it << ")blockIdx.x * " << kBlock * U << "; base < " << nv << "; base += (" << it << ")gridDim.x * " << kBlock * U
+    o << "  for (" << it << " base = (" << it << ")blockIdx.x * " << BLK * U << "; base < " << nv << "; base += (" << it << ")gridDim.x * " << BLK * U
       << ") {\n";
     o << "#pragma unroll\n    for (int u = 0; u < " << U << "; ++u) {\n";
-    o << "      const " << it << " vid = base + u * " << kBlock << " + threadIdx.x;\n";
+    o << "      const " << it << " vid = base + u * " << BLK << " + threadIdx.x;\n";
     o << "      if (vid < " << nv << ") {\n";
     decode_index(o, it, "vid", dims, vec, "        ");
     o << "        const " << it << " lin0 = vid * " << vec << ";\n";
@@ -3968,8 +3982,24 @@ struct Planner {
     o << "        }\n      }\n    }\n  }\n";
     o << "  " << ACC << " a = acc[0];\n";
     o << "#pragma unroll\n  for (int u = 1; u < " << U << "; ++u) a = " << red_apply(rn.red, dt, "a", "acc[u]") << ";\n";
-    o << "  __shared__ " << ACC << " lds[" << kBlock / 64 << "];\n";
-    o << "  a = rx_block_reduce<" << ACC << ", decltype(" << red_functor(rn.red) << "), " << kBlock / 64 << ">(a, " << red_functor(rn.red) << ", lds);\n";
+    o << "  __shared__ " << ACC << " lds[" << BLK / 64 << "];\n";
+    o << "  a = rx_block_reduce<" << ACC << ", decltype(" << red_functor(rn.red) << "), " << BLK / 64 << ">(a, " << red_functor(rn.red) << ", lds);\n";
+    if (one) {
+      o << "  if (threadIdx.x == 0) {\n" << one_code;
+      o << "    const " << ACC << " r = " << red_apply(rn.red, dt, "a", "(" + ACC + ")" + one_init) << ";\n";
+      o << "    out0[0] = " << Emitter::store_conv(dt, is_narrow_float(dt) ? Emitter::round_narrow(dt, "r") : std::string("(") + info(dt).ctype + ")r") << ";\n  }\n}\n\n";
+      Launch L;
+      L.kernel = named(k1, finalize(o.str()));
+      L.kind = "reduce";
+      L.grid[0] = 1;
+      L.block[0] = BLK;
+      for (int i : em.inputs) L.args.push_back(buffer_for(i));
+      L.args.push_back(buffer_for(root));
+      L.algo_bytes = algo_bytes(em.inputs, {}) + info(dt).size;
+      L.desc = describe(rn.in[0]) + " reduce";
+      plan.launches.push_back(L);
+      return;
+    }
     // the init value and the final store, evaluated by one thread
     Emitter e2(g, [&](int x) { return mat[x]; });
     e2.excess_precision = opt.excess_precision;

@@ -70,6 +70,7 @@ struct PlanOptions {
   bool lds_stencil = true;      // 3-D maps that read an input at several offsets stage it through LDS halo tiles
   int slab_ytiles = 0;          // stencil kernels: y-tiles per XCD slab (0: one slab per XCD)
   int lds_tile[3] = {3, 4, 128};  // outputs per workgroup tile (slowest .. fastest dimension)
+  int64_t one_workgroup_reduce = 8192;   // full reductions of up to this many elements are one workgroup's, and one launch
   // full reductions in one launch: every workgroup publishes its partial as flagged words and the
   // workgroup with the last index waits for all of them and combines.  Off: it saves the 1-workgroup
   // combine launch (1.4 us of an 85 us step over 2^26 elements, 1.2 us of a 485 us FP8 step), and it
