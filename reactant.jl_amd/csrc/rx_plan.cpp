@@ -2823,12 +2823,15 @@ struct Planner {
   // steps per kernel: a 1-d tile's halo grows by a cell or two per step, so long chains stay cheap
   int chain_cap(int rank) const { return opt.chain_steps > 0 ? opt.chain_steps : rank == 1 ? 64 : rank == 2 ? 16 : 4; }
 
+  // ... and per run that is divided into kernels
+  int chain_run(int rank) const { return rank == 3 && opt.chain_steps <= 0 ? 64 : chain_cap(rank); }
+
   bool probe_chain_step(int x, ChainProbe* cp) {
     const Node& n = g.nodes[x];
     const int r = n.ty.rank();
     // rank 3: only small arrays, whose steps are bound by the launch gap (32^3 and 64^3 heat steps: 1.6x and 1.4x
     // faster in chains of four); at 128^3 the redundant halo cells cost more than the launches saved
-    if (r < 1 || r > 3 || (r > opt.chain_max_rank && !(r == 3 && n.ty.numel() <= opt.chain_rank3_numel))) return false;
+    if (r < 1 || r > 3 || (r > opt.chain_max_rank && r != 3)) return false;
     if (n.k == OpK::Param || n.k == OpK::Constant || n.k == OpK::Reduce || n.k == OpK::Scan || n.k == OpK::Scatter || n.k == OpK::Conv || n.k == OpK::DotGeneral) return false;
     const int es = info(n.ty.dt).size;
     if (es != 4 && es != 8) return false;
@@ -2895,8 +2898,70 @@ struct Planner {
     return true;
   }
 
+  // Rank-3 steps that read further arrays at their own position (velocities, coefficients; a chain keeps them in registers):
+  // the tile and the number of steps per launch, by the time of the launches that `n` steps take.  Only tiles that give a compute
+  // unit one workgroup; larger arrays stay maps, which move them from L2 with less arithmetic (116 x 116 x 70 f64: the best
+  // chain 87 us for 10 steps, maps 100; 171 x 100 x 29: 48 and 45; 206 x 106 x 106: 196 and 230).  Fitted to 51 (f64) and 26 (f32)
+  // timings of 8 to 10 advection-diffusion steps on 36 x 36 x 26 to 165 x 100 x 29 points, tiles of 6 x 6 x 12 to 10 x 10 x 32 and
+  // 2 to 4 steps (9 and 8 % rms): rounds are of a workgroup over its cells, MB what all of them stage.  A map per step takes
+  // 4.4 us.  10 steps, us, tiles of 8 x 8 x 16 and two steps (f32: four) before -> as chosen: 67 x 53 x 39 f64 32.2 -> 26.2,
+  // f32 20 -> 17.5; 36 x 36 x 26 f64 28.7 -> 17.7.
+  // (Runs of up to three steps are left as they are.)
+  // how many further arrays (0: the choice above is not for these steps)
+  int chain3_others(const std::vector<int>& steps, const std::vector<ChainProbe>& probes) const {
+    if (g.nodes[steps[0]].ty.rank() != 3 || steps.size() < 4 || opt.chain_steps > 0 || opt.chain_tile[0] > 0 || !opt.chain_fixed_cells) return 0;
+    std::set<int> moved, others;
+    for (auto& p : probes)
+      for (auto& kv : p.reads) {
+        bool own = true;
+        for (int d = 0; d < 3; ++d) {
+          own = own && kv.second.lo[d] == 0 && kv.second.hi[d] == 0;
+          if (kv.second.lo[d] > 1 || kv.second.hi[d] > 1) return 0;
+        }
+        (own ? others : moved).insert(kv.first);
+      }
+    for (int x : moved) others.erase(x);
+    for (int x : steps) others.erase(x);
+    return (int)others.size();
+  }
+  int choose_chain3(size_t n, const int64_t* D, int es, int others, int64_t* T) const {
+    const size_t cap = 5;
+    double cost[6];
+    int64_t tile[6][3] = {};
+    cost[1] = 4.4;
+    for (size_t k = 2; k <= cap; ++k) {
+      cost[k] = 1e30;
+      for (int64_t a : {4, 5, 6, 8, 10})
+        for (int64_t b : {6, 7, 8, 10, 16})
+          for (int64_t c : {8, 12, 16, 32}) {
+            const int64_t t[3] = {std::min(a, D[0]), std::min(b, D[1]), std::min(c, D[2])};
+            const int64_t kk = (int64_t)k, plane = (t[1] + 2 * kk) * (t[2] + 2 * kk), box = (t[0] + 2 * kk) * plane;
+            const int64_t nb = std::min<int64_t>(1024, (box + 63) / 64 * 64), per = (box + nb - 1) / nb;
+            const int64_t wgs = ((D[0] + t[0] - 1) / t[0]) * ((D[1] + t[1] - 1) / t[1]) * ((D[2] + t[2] - 1) / t[2]);
+            if (box * 2 * es > 96 * 1024 || per > 8 || others * per * (es / 4) > 48 || wgs > 256) continue;
+            int64_t rounds = 0;
+            for (int64_t i = 1; i <= kk; ++i) rounds += std::min(per, ((t[0] + 2 * kk - i) * plane + nb - 1) / nb) - i * plane / nb;
+            const double fill = (double)nb / 1024.0, mb = 1e-6 * (double)(wgs * box * es * (others + 1));
+            const double us = es == 8 ? 2.1 + fill * (0.59 * (double)per + 0.13 * (double)rounds) + 0.09 * mb : 2.5 + fill * (0.28 * (double)per + 0.16 * (double)rounds) + 0.04 * mb;
+            if (us < cost[k]) { cost[k] = us; for (int d = 0; d < 3; ++d) tile[k][d] = t[d]; }
+          }
+    }
+    std::vector<double> best(n + 1, 0);
+    std::vector<size_t> first(n + 1, 1);
+    for (size_t m = 1; m <= n; ++m) {
+      best[m] = 1e30;
+      for (size_t k = 1; k <= std::min(cap, m); ++k)
+        if (cost[k] + best[m - k] < best[m] - 1e-9) { best[m] = cost[k] + best[m - k]; first[m] = k; }
+    }
+    // the longest launch of the best division first
+    size_t k = 1;
+    for (size_t m = n; m > 0; m -= first[m]) k = std::max(k, first[m]);
+    for (int d = 0; d < 3; ++d) T[d] = tile[k][d];
+    return (int)k;
+  }
+
   // Kernel for a prefix of `steps`; returns how many steps it covers (0: none, nothing emitted).
-  size_t emit_chain(const std::vector<int>& steps, const std::vector<ChainProbe>& probes) {
+  size_t emit_chain(const std::vector<int>& steps, const std::vector<ChainProbe>& probes, int others) {
     const Node& n0 = g.nodes[steps[0]];
     const int r = n0.ty.rank();
     const auto& D = n0.ty.dims;
@@ -2913,7 +2978,13 @@ struct Planner {
         T[d] = std::min<int64_t>(T[d], D[d]);
       }
     }
-    for (size_t k = std::min<size_t>(steps.size(), (size_t)chain_cap(r)); k >= 2; --k) {
+    size_t longest = std::min<size_t>(steps.size(), (size_t)chain_cap(r));
+    const bool chosen = others > 0;
+    if (chosen) {
+      longest = (size_t)choose_chain3(steps.size(), D.data(), es, others, T);
+      if (longest < 2) return 0;
+    }
+    for (size_t k = longest; k >= 2; --k) {
       // fields of the first k steps: version at kernel entry, and which field each node is a version of
       std::vector<int> entry;
       std::map<int, int> field_of;
@@ -2951,7 +3022,7 @@ struct Planner {
       for (int d = 0; d < r; ++d) { E[d] = T[d] + HL[d] + HH[d]; box *= E[d]; tile *= T[d]; }
       const int64_t lds_bytes = box * ntiles_lds * es;
       if (getenv("RX_CHAIN_DEBUG")) fprintf(stderr, "[chain] k=%zu box=%lld tile=%lld tiles_in_lds=%d bytes=%lld\n", k, (long long)box, (long long)tile, ntiles_lds, (long long)lds_bytes);
-      if (lds_bytes > opt.chain_lds_bytes || (double)box > (r == 3 ? 2.0 : 1.0) * opt.chain_redundancy * (double)tile) continue;
+      if (!chosen && (lds_bytes > opt.chain_lds_bytes || (double)box > (r == 3 ? 2.0 : 1.0) * opt.chain_redundancy * (double)tile)) continue;
       const int NB = opt.chain_threads > 0 ? opt.chain_threads : (int)std::min<int64_t>(1024, (box + 63) / 64 * 64);
       if (NB < 64 || NB > 1024 || NB % 64) continue;
 
@@ -2969,6 +3040,13 @@ struct Planner {
       auto tile_name = [&](int f) { return "lds" + std::to_string(f) + (side[f] ? "b" : ""); };
       int64_t margin = 0;   // farthest neighbour read, in cells: the tiles sit that far inside the LDS allocation
       std::set<int> group(steps.begin(), steps.begin() + k);
+      const int64_t R = (box + NB - 1) / NB;   // box cells per thread
+      const bool fixed = R <= 8 && opt.chain_fixed_cells;
+      // Such an array's values at a thread's own cells are read once for all steps, with the boxes of the others: a read in
+      // every step was a trip to memory between two barriers.  Registers: as many as a wavefront gets when NB / 256 share a SIMD.
+      int in_memory = 0;
+      for (int f = 0; f < nf; ++f) in_memory += !has_tile[f];
+      const bool keep = fixed && in_memory > 0 && in_memory * R * (es / 4) <= 48;
       bool ok = true;
       for (size_t i = 0; i < k && ok; ++i) {
         const int x = steps[i];
@@ -2983,7 +3061,11 @@ struct Planner {
           auto f = field_of.find(node);
           if (f == field_of.end() || !(g.nodes[node].ty == n0.ty)) return false;
           if (cur[f->second] != node) { ok = false; return false; }
-          if (!has_tile[f->second]) return false;
+          if (!has_tile[f->second]) {
+            if (!keep) return false;
+            *expr = "m" + std::to_string(f->second) + "[q]";
+            return true;
+          }
           int64_t delta = 0, stride = 1;
           for (int d = r - 1; d >= 0; --d) { delta += off[d] * stride; stride *= E[d]; }
           margin = std::max<int64_t>(margin, delta < 0 ? -delta : delta);
@@ -3047,8 +3129,6 @@ struct Planner {
         o << "  const int t" << d << " = (tb % " << nt[d] << ") * " << T[d] << ";\n";
         if (d) o << "  tb /= " << nt[d] << ";\n";
       }
-      const int64_t R = (box + NB - 1) / NB;   // box cells per thread
-      const bool fixed = R <= 8 && opt.chain_fixed_cells;
       if (!fixed) {
       // Loops over the cells of a region run a fixed number of rounds per thread without branches
       // (cells past the end repeat the last one, array positions are clamped into the array, and
@@ -3128,7 +3208,13 @@ struct Planner {
           return e;
         };
         for (int d = 0; d < r; ++d) o << "  int C" << d << "[" << R << "], G" << d << "[" << R << "];\n";
-        o << "  bool IN[" << R << "];\n";
+        // Every step reaches one cell to each side: a cell takes part in as many steps as it lies cells inside the box, which
+        // is one comparison per step instead of three.
+        bool unit = true;
+        for (size_t i = 0; i < k; ++i)
+          for (int d = 0; d < r; ++d) unit = unit && lo[i][d] == 1 && hi[i][d] == 1;
+        o << (unit ? "  int IN[" : "  bool IN[") << R << "];\n";
+        for (int f = 0; f < nf; ++f) if (keep && !has_tile[f]) o << "  " << st << " m" << f << "[" << R << "];\n";
         o << "#pragma unroll\n  for (int q = 0; q < " << R << "; ++q) {\n";
         o << "    const int p = threadIdx.x + q * " << NB << ";\n    int rr = rx_min(p, " << box - 1 << ");\n";
         for (int d = r - 1; d >= 0; --d) {
@@ -3142,9 +3228,16 @@ struct Planner {
           o << "    C" << d << "[q] = c" << d << "; G" << d << "[q] = g" << d << ";\n";
           in_arr += " && a" + std::to_string(d) + " == g" + std::to_string(d);
         }
-        o << "    IN[q] = " << in_arr << ";\n";
+        if (unit) {
+          std::string nest = "rx_min(c0, " + std::to_string(E[0] - 1) + " - c0)";
+          for (int d = 1; d < r; ++d) nest = "rx_min(" + nest + ", rx_min(c" + std::to_string(d) + ", " + std::to_string(E[d] - 1) + " - c" + std::to_string(d) + "))";
+          o << "    IN[q] = " << in_arr << " ? " << nest << " : -1;\n";
+        } else {
+          o << "    IN[q] = " << in_arr << ";\n";
+        }
         o << "    const int lin = " << array_index() << ";\n";
         for (int f = 0; f < nf; ++f) if (has_tile[f]) o << "    const " << st << " s" << f << " = in" << slot_in(entry[f]) << "[lin];\n";
+        for (int f = 0; f < nf; ++f) if (keep && !has_tile[f]) o << "    m" << f << "[q] = in" << slot_in(entry[f]) << "[lin];\n";
         o << "    if (p < " << box << ") {\n";
         for (int f = 0; f < nf; ++f) if (has_tile[f]) o << "      lds" << f << "[p] = s" << f << ";\n";
         o << "    }\n  }\n  __syncthreads();\n";
@@ -3158,10 +3251,10 @@ struct Planner {
           rounds_of(first[0], first[0] + ext[0], &qlo, &qhi);
           o << "#pragma unroll\n  for (int q = " << qlo << "; q < " << qhi << "; ++q) {\n";
           o << "    const int li = rx_min((int)threadIdx.x + q * " << NB << ", " << box - 1 << ");\n";
-          std::string live = "IN[q]";
+          std::string live = unit ? "IN[q] >= " + std::to_string(first[0]) : std::string("IN[q]");
           for (int d = 0; d < r; ++d) {
             o << "    const int g" << d << " = G" << d << "[q];\n";
-            live += " && (unsigned)(C" + std::to_string(d) + "[q] - " + std::to_string(first[d]) + ") < " + std::to_string(ext[d]) + "u";
+            if (!unit) live += " && (unsigned)(C" + std::to_string(d) + "[q] - " + std::to_string(first[d]) + ") < " + std::to_string(ext[d]) + "u";
           }
           o << "    const bool live = " << live << ";\n";
         };
@@ -5488,7 +5581,7 @@ struct Planner {
         std::set<int> group;
         std::map<int, int> field_of;
         std::vector<int> cur;
-        for (size_t j = i; j < jobs.size() && (steps.empty() || steps.size() < (size_t)chain_cap(g.nodes[steps[0]].ty.rank())); ++j) {
+        for (size_t j = i; j < jobs.size() && (steps.empty() || steps.size() < (size_t)chain_run(g.nodes[steps[0]].ty.rank())); ++j) {
           const int x = jobs[j].first;
           if (absorbed_roots.count(x) || reshape_alias.count(x) || !row_phases(x).empty()) break;
           ChainProbe q;
@@ -5511,13 +5604,15 @@ struct Planner {
           probes.push_back(q);
         }
         if (getenv("RX_CHAIN_DEBUG")) fprintf(stderr, "[chain] job %zu (node %d, %s): run of %zu steps\n", i, jobs[i].first, g.nodes[jobs[i].first].ty.str().c_str(), steps.size());
+        const int others = steps.empty() ? 0 : chain3_others(steps, probes);
+        if (!steps.empty() && others == 0 && g.nodes[steps[0]].ty.rank() > opt.chain_max_rank && g.nodes[steps[0]].ty.numel() > opt.chain_rank3_numel) { ++i; continue; }
         if (steps.size() < 2) { ++i; continue; }
         chain_at[steps[0]] = steps;
         auto plain0 = jobs[i].second;
-        jobs[i].second = [this, steps, probes, plain0] {
+        jobs[i].second = [this, steps, probes, plain0, others] {
           size_t at = 0;
           while (steps.size() - at >= 2) {
-            const size_t used = emit_chain(std::vector<int>(steps.begin() + at, steps.end()), std::vector<ChainProbe>(probes.begin() + at, probes.end()));
+            const size_t used = emit_chain(std::vector<int>(steps.begin() + at, steps.end()), std::vector<ChainProbe>(probes.begin() + at, probes.end()), others);
             if (!used) break;
             for (size_t q = 0; q < used; ++q) chain_member.insert(steps[at + q]);
             at += used;
