@@ -385,6 +385,7 @@ class LoadedExecutable:
         self.handle = handle
         self.client = client
         self.num_results = _call("RxExecutableNumResults", handle)
+        self.result_types = None   # (shape in Julia order, element type) of every result: the module's, read off the first execution's
 
     def report(self):
         return _call("RxExecutableReport", self.handle).decode()
@@ -416,17 +417,15 @@ class LoadedExecutable:
         """XLA.execute_sharded: returns AsyncBuffers (src/xla/PJRT/LoadedExecutable.jl:175-246)."""
         n = len(buffers)
         args = (_vp * n)(*[b.handle for b in buffers])
-        don = (_u8 * n)(*([1 if d else 0 for d in donated] if donated else [0] * n))
+        don = (_u8 * n)(*[1 if d else 0 for d in donated]) if donated else None
         nres = self.num_results
         res = (_vp * nres)()
         futs = (_vp * nres)()
         has = _u8(0)
-        dev = (device or self.client.default_device()).handle
+        dev = device.handle if device is not None else None   # none: the executable's
         _call("XLAExecuteSharded", self.handle, n, args, dev, don, nres, res, ctypes.byref(has), futs)
-        out = []
-        for k in range(nres):
-            out.append(AsyncBuffer(Buffer(res[k], self.client), Future(futs[k]) if has.value else None))
-        return out
+        client, future = self.client, has.value
+        return [AsyncBuffer(Buffer(r, client), Future(f) if future else None) for r, f in zip(res, futs)]
 
     def execute_timed(self, buffers, donated=None, device=None):
         """Like execute_sharded, with a HIP event pair around every kernel launch: (buffers, ms list)."""
@@ -676,13 +675,14 @@ class Thunk:
             for a, d in zip(args, donated):
                 if d:
                     a.donated = True
-        outs = []
-        for ab in res:
-            if sync:
+        if sync:
+            for ab in res:
                 ab.synced_buffer()
-            b = ab.buffer
-            outs.append(ConcreteRArray(ab, b.shape()[::-1], b.dtype()))
-        return outs[0] if len(outs) == 1 else tuple(outs)
+        types = self.exec.result_types
+        if types is None:
+            types = self.exec.result_types = [(ab.buffer.shape()[::-1], ab.buffer.dtype()) for ab in res]
+        outs = tuple([ConcreteRArray(ab, shape, dtype) for ab, (shape, dtype) in zip(res, types)])
+        return outs[0] if len(outs) == 1 else outs
 
 
 def compile(mlir_text, client=None):
