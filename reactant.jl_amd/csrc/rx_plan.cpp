@@ -177,6 +177,7 @@ struct Planner {
         }
       }
     }
+    masks_of_maxima();
     dots_to_reductions();
     normalize_dots();
     align_dots();
@@ -185,6 +186,40 @@ struct Planner {
     chain_convs();
     channel_minor_regions();
     pad_into_pools();
+  }
+
+  // x > 0 is max(x, 0) > 0 (of a NaN too: both are false).  Where x is read by such maxima and comparisons only -- a layer's
+  // relu and, in the reverse pass, its mask -- the comparisons read the maximum: x then belongs to one kernel, the product's,
+  // which writes max(x, 0) itself, and the map between the products goes (training step of 784 -> 2048 -> 1000, 1024 rows
+  // in bf16: 4.8 us and 8 MB).
+  void masks_of_maxima() {
+    const int N = (int)g.nodes.size();
+    std::vector<std::vector<int>> use(N);
+    for (auto& n : g.nodes) for (int i : n.in) use[i].push_back(n.id);
+    std::vector<char> is_res(N, 0);
+    for (int r : g.results) is_res[r] = 1;
+    auto zero = [&](int x) {
+      if (g.nodes[x].k == OpK::BroadcastInDim) x = g.nodes[x].in[0];
+      const Node& c = g.nodes[x];
+      return c.k == OpK::Constant && c.splat && is_float(c.ty.dt) && splat_as_double(c) == 0.0;
+    };
+    for (int m = 0; m < N; ++m) {
+      const Node& mn = g.nodes[m];
+      if (mn.k != OpK::Binary || mn.op != "maximum" || !is_float(mn.ty.dt) || zero(mn.in[0]) == zero(mn.in[1])) continue;
+      const int x = zero(mn.in[0]) ? mn.in[1] : mn.in[0];
+      std::vector<int> masks;
+      bool only = !is_res[x];
+      for (int u : use[x]) {
+        const Node& un = g.nodes[u];
+        const bool gt = un.k == OpK::Compare && un.op == "GT" && un.in[0] == x && zero(un.in[1]), lt = un.k == OpK::Compare && un.op == "LT" && un.in[1] == x && zero(un.in[0]);
+        if (u == m) continue;
+        only = only && u > m && (gt || lt);
+        masks.push_back(u);
+      }
+      if (!only) continue;
+      for (int u : masks)
+        for (int& i : g.nodes[u].in) if (i == x) i = m;
+    }
   }
 
   // Zero padding of a pooled value, where the windows do not overlap (size = stride, no dilation, the extent a whole
