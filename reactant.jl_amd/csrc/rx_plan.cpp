@@ -4048,8 +4048,10 @@ struct Planner {
   // one: f32 4099 elements 8.2 and 3.9, 8192 8.2 and 4.0, 32768 8.1 and 6.9, 65536 8.1 and 12; f64 4096 8.3 and 3.9, 8192 8.4
   // and 5.4, 16384 7.9 and 9.1.  A thread adds at most eight elements, as it does in the two-launch form.  Several
   // transcendental functions per element: fewer elements.
-  void emit_reduce_full(int root) {
+  // `tail`: the reduction itself, or the elementwise root that is its only reader: evaluated by the thread that stores.
+  void emit_reduce_full(int root, int tail) {
     const Node& rn = g.nodes[root];
+    const DT tdt = g.nodes[tail].ty.dt;
     const Node& inn = g.nodes[rn.in[0]];
     const auto& dims = inn.ty.dims;
     const int n = inn.ty.rank();
@@ -4066,7 +4068,8 @@ struct Planner {
     const int G = one ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(tiles, 2048));
     const std::string k1 = "@K@_reduce", k2 = "@K@_reduce_final";
 
-    Emitter em(g, [&](int x) { return mat[x]; });
+    auto in_memory = [&, tail, root](int x) { return mat[x] && (tail == root || x != tail); };
+    Emitter em(g, in_memory);
     em.excess_precision = opt.excess_precision;
     em.idx64 = needs64(cone_nodes(rn.in[0]));
     const std::string it = em.idx_t();
@@ -4077,16 +4080,26 @@ struct Planner {
     em.direct_expr = vec_name;
     em.indent = 10;
     std::string val = em.emit(rn.in[0], root_index(dims));
-    std::string body = em.take_code(), one_init, one_code;
-    if (one) {   // the init value's operands come after the reduction's
-      em.indent = 4;
-      one_init = em.emit(rn.in[1], Index{});
-      one_code = em.take_code();
-    }
+    std::string body = em.take_code(), one_code;
+    // the stored value, from the sum `a` (an expression) and the init value
+    auto stored = [&](Emitter& e, const std::string& a) {
+      e.indent = 4;
+      std::string code;
+      const std::string init = e.emit(rn.in[1], Index{});
+      code = e.take_code() + "    const " + ACC + " r = " + red_apply(rn.red, dt, a, "(" + ACC + ")" + init) + ";\n";
+      const std::string rv = is_narrow_float(dt) ? Emitter::round_narrow(dt, "r") : std::string("(") + info(dt).ctype + ")r";
+      if (tail == root) return code + "    out0[0] = " + Emitter::store_conv(dt, rv) + ";\n";
+      code += "    const " + std::string(info(dt).ctype) + " red_ = " + rv + ";\n";
+      e.bound[root] = "red_";
+      const std::string v = e.emit(tail, Index{});
+      code += e.take_code();
+      return code + "    out0[0] = " + e.store_value(tdt, v) + ";\n";
+    };
+    if (one) one_code = stored(em, "a");   // (its operands come after the reduction's)
 
     std::ostringstream o;
     o << "// reduce" << (one ? ": " : " (pass 1): ") << describe(rn.in[0]) << (one ? ", one workgroup\n" : " -> partials\n");
-    if (one) o << signature(k1, em.inputs, {{info(dt).stype, "out0"}}, BLK) << " {\n";
+    if (one) o << signature(k1, em.inputs, {{info(tdt).stype, "out0"}}, BLK) << " {\n";
     else o << signature(k1, em.inputs, {{ACC, "partial"}}) << " {\n";
     o << "  " << ACC << " acc[" << U << "];\n";
     o << "#pragma unroll\n  for (int u = 0; u < " << U << "; ++u) acc[u] = " << red_identity(rn.red, dt) << ";\n";
@@ -4113,29 +4126,24 @@ struct Planner {
     o << "  __shared__ " << ACC << " lds[" << BLK / 64 << "];\n";
     o << "  a = rx_block_reduce<" << ACC << ", decltype(" << red_functor(rn.red) << "), " << BLK / 64 << ">(a, " << red_functor(rn.red) << ", lds);\n";
     if (one) {
-      o << "  if (threadIdx.x == 0) {\n" << one_code;
-      o << "    const " << ACC << " r = " << red_apply(rn.red, dt, "a", "(" + ACC + ")" + one_init) << ";\n";
-      o << "    out0[0] = " << Emitter::store_conv(dt, is_narrow_float(dt) ? Emitter::round_narrow(dt, "r") : std::string("(") + info(dt).ctype + ")r") << ";\n  }\n}\n\n";
+      o << "  if (threadIdx.x == 0) {\n" << one_code << "  }\n}\n\n";
       Launch L;
       L.kernel = named(k1, finalize(o.str()));
       L.kind = "reduce";
       L.grid[0] = 1;
       L.block[0] = BLK;
       for (int i : em.inputs) L.args.push_back(buffer_for(i));
-      L.args.push_back(buffer_for(root));
-      L.algo_bytes = algo_bytes(em.inputs, {}) + info(dt).size;
+      L.args.push_back(buffer_for(tail));
+      L.algo_bytes = algo_bytes(em.inputs, {}) + info(tdt).size;
       L.desc = describe(rn.in[0]) + " reduce";
       plan.launches.push_back(L);
       return;
     }
     // the init value and the final store, evaluated by one thread
-    Emitter e2(g, [&](int x) { return mat[x]; });
+    Emitter e2(g, in_memory);
     e2.excess_precision = opt.excess_precision;
-    e2.indent = 4;
-    std::string initv = e2.emit(rn.in[1], Index{});
-    std::string ibody = e2.take_code();
+    const std::string ibody = stored(e2, "c");
     std::vector<int> in2 = e2.inputs;
-    std::string rv = is_narrow_float(dt) ? Emitter::round_narrow(dt, "r") : std::string("(") + info(dt).ctype + ")r";
     auto combine = [&](std::ostringstream& oo, const std::string& src) {
       // partials are combined in index order by a fixed tree: the result does not depend on
       // which workgroup finished last
@@ -4143,8 +4151,6 @@ struct Planner {
       oo << "  for (int i = threadIdx.x; i < " << G << "; i += " << kBlock << ") c = " << red_apply(rn.red, dt, "c", src + "[i]") << ";\n";
       oo << "  c = rx_block_reduce<" << ACC << ", decltype(" << red_functor(rn.red) << "), " << kBlock / 64 << ">(c, " << red_functor(rn.red) << ", lds);\n";
       oo << "  if (threadIdx.x == 0) {\n" << ibody;
-      oo << "    const " << ACC << " r = " << red_apply(rn.red, dt, "c", "(" + ACC + ")" + initv) << ";\n";
-      oo << "    out0[0] = " << Emitter::store_conv(dt, rv) << ";\n";
     };
     const bool single = opt.single_pass_reduce && G > 1;
     const int NW = (dt == DT::F64 || info(dt).size == 8) ? 2 : 1;   // 32-bit words of one partial
@@ -4160,7 +4166,7 @@ struct Planner {
       sig.pop_back();
       sig += ", unsigned long long* __restrict__ slots";
       for (size_t k = 0; k < in2.size(); ++k) sig += ", " + ptr_decl(info(g.nodes[in2[k]].ty.dt).stype, true, "fin" + std::to_string(k));
-      sig += ", " + ptr_decl(info(dt).stype, false, "out0") + ")";
+      sig += ", " + ptr_decl(info(tdt).stype, false, "out0") + ")";
       // the pass-1 text was written against `signature(k1, ...)`; swap the header
       std::string text = o.str();
       const std::string old_sig = signature(k1, em.inputs, {{ACC, "partial"}});
@@ -4193,7 +4199,7 @@ struct Planner {
       {
         std::string s2 = "extern \"C\" __global__ __launch_bounds__(" + std::to_string(kBlock) + ") void " + k2 + "(const " + ACC + "* __restrict__ partial";
         for (size_t k = 0; k < in2.size(); ++k) s2 += ", " + ptr_decl(info(g.nodes[in2[k]].ty.dt).stype, true, "in" + std::to_string(k));
-        s2 += ", " + ptr_decl(info(dt).stype, false, "out0") + ")";
+        s2 += ", " + ptr_decl(info(tdt).stype, false, "out0") + ")";
         o << s2 << " {\n";
       }
       o << "  __shared__ " << ACC << " lds[" << kBlock / 64 << "];\n";
@@ -4222,7 +4228,7 @@ struct Planner {
       plan.buffers.push_back(cb);
       L1.args.push_back((int)plan.buffers.size() - 1);
       for (int i : in2) L1.args.push_back(buffer_for(i));
-      L1.args.push_back(buffer_for(root));
+      L1.args.push_back(buffer_for(tail));
       plan.launches.push_back(L1);
       return;
     }
@@ -4234,7 +4240,7 @@ struct Planner {
     L2.block[0] = kBlock;
     L2.args.push_back(sc);
     for (int i : in2) L2.args.push_back(buffer_for(i));
-    L2.args.push_back(buffer_for(root));
+    L2.args.push_back(buffer_for(tail));
     L2.desc = "combine partials";
     plan.launches.push_back(L2);
   }
@@ -5524,6 +5530,20 @@ struct Planner {
       }
     }
 
+    // A full reduction whose only reader is elementwise on its scalar (a mean's division, a root) runs that as well: no launch
+    // for one number (4 us).
+    std::map<int, int> reduce_of;   // that root -> the reduction
+    for (int x = 0; x < N && opt.product_epilogues; ++x) {
+      if (!live[x] || g.nodes[x].k != OpK::Reduce || ctx[x].size() != 1) continue;
+      if (std::find(g.results.begin(), g.results.end(), x) != g.results.end() || red_shape(g.nodes[x]).nkeep != 0 || g.nodes[g.nodes[x].in[0]].ty.numel() == 0) continue;
+      const int r = ctx[x].begin()->first;
+      const Node& n = g.nodes[r];
+      if (n.ty.rank() != 0 || !mat[r] || absorbed_roots.count(r) || reduce_of.count(r) || reshape_alias.count(r)) continue;
+      if (n.k == OpK::Param || n.k == OpK::Constant || n.k == OpK::Reduce || n.k == OpK::Scan || n.k == OpK::Scatter || n.k == OpK::Conv || n.k == OpK::DotGeneral || n.k == OpK::Reshape) continue;
+      reduce_of[r] = x;
+      absorbed_roots.insert(r);
+    }
+
     lap("epilogues and aliases");
     // kernels in topological order of their roots
     std::vector<std::pair<int, std::function<void()>>> jobs;
@@ -5535,6 +5555,11 @@ struct Planner {
         auto e = epilogue_of.find(x);
         if (e != epilogue_of.end()) continue;  // emitted with its root
         jobs.push_back({x, [this, x] { emit_dot(x, x); }});
+        continue;
+      }
+      if (reduce_of.count(x)) {
+        const int red = reduce_of[x];
+        jobs.push_back({x, [this, x, red] { emit_reduce_full(red, x); }});
         continue;
       }
       if (absorbed_roots.count(x)) {
@@ -5559,12 +5584,13 @@ struct Planner {
       }
       if (reshape_alias.count(x)) continue;
       if (n.k == OpK::Reduce) {
+        if (std::any_of(reduce_of.begin(), reduce_of.end(), [x](const std::pair<const int, int>& kv) { return kv.second == x; })) continue;   // emitted with its reader
         jobs.push_back({x, [this, x, &fused_reduces] {
           if (fused_reduces.count(x)) return;
           const Node& r = g.nodes[x];
           RedShape rs = red_shape(r);
           if (g.nodes[r.in[0]].ty.numel() == 0 || r.ty.numel() == 0) { emit_reduce_generic(x); return; }
-          if (rs.nkeep == 0) { emit_reduce_full(x); return; }
+          if (rs.nkeep == 0) { emit_reduce_full(x, x); return; }
           if (rs.trailing && rs.cols >= 64) { emit_row(x, {x}); return; }
           emit_reduce_generic(x);
         }});
