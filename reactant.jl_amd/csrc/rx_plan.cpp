@@ -4445,6 +4445,49 @@ struct Planner {
   }
 
   // generic reduction: one thread per output element, sequential loops over reduced dims
+  void emit_reduce_columns(int root, Emitter& em, const std::vector<int>& kept, int red, int64_t nout, int VEC, int NC, int NG, int PER, int CX, int CY, const std::string& body,
+                 const std::string& val, const std::string& ibody, const std::string& initv) {
+    const Node& rn = g.nodes[root];
+    const Node& inn = g.nodes[rn.in[0]];
+    const DT dt = rn.ty.dt;
+    const std::string ACC = acc_ctype(dt), it = em.idx_t();
+    const int64_t len = inn.ty.dims[red], nvec = nout / VEC;
+    std::ostringstream o;
+    o << "// reduce (columns): " << describe(rn.in[0]) << " -> " << rn.ty.str() << "\n";
+    o << signature("@K@_reduce_generic", em.inputs, {{info(dt).stype, "out0"}}) << " {\n";
+    o << "  __shared__ " << ACC << " part[" << CY << "][" << NC << "], sums[" << NG << "][" << NC << "];\n";
+    o << "  const int cx = threadIdx.x % " << CX << ", cy = threadIdx.x / " << CX << ";\n";
+    o << "  {\n    const " << it << " vid = rx_min<" << it << ">((" << it << ")blockIdx.x * " << CX << " + cx, " << nvec - 1 << ");\n";
+    o << "    " << it << " rr = vid * " << VEC << ";\n";
+    for (int k = (int)kept.size() - 1; k >= 0; --k) {
+      o << "    const " << it << " o" << k << (k == (int)kept.size() - 1 ? "b" : "") << " = rr % " << inn.ty.dims[kept[k]] << ";\n";
+      o << "    rr /= " << inn.ty.dims[kept[k]] << ";\n";
+    }
+    o << "    " << ACC << " accv[" << VEC << "];\n#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) accv[l] = " << red_identity(rn.red, dt) << ";\n";
+    o << "#pragma unroll 8\n    for (" << it << " r0 = cy; r0 < " << len << "; r0 += " << CY << ") {\n#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) {\n";
+    o << "      const " << it << " o" << kept.size() - 1 << " = o" << kept.size() - 1 << "b + l;\n" << body;
+    o << "      accv[l] = " << red_apply(rn.red, dt, "accv[l]", "(" + ACC + ")" + val) << ";\n    }\n    }\n";
+    o << "#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) part[cy][cx * " << VEC << " + l] = accv[l];\n  }\n  __syncthreads();\n";
+    o << "  const int c = threadIdx.x % " << NC << ", q = threadIdx.x / " << NC << ";\n";
+    o << "  {\n    " << ACC << " a = part[q * " << PER << "][c];\n#pragma unroll\n    for (int y = 1; y < " << PER << "; ++y) a = "
+      << red_apply(rn.red, dt, "a", "part[q * " + std::to_string(PER) + " + y][c]") << ";\n    sums[q][c] = a;\n  }\n  __syncthreads();\n";
+    o << "  const " << it << " oid = (" << it << ")blockIdx.x * " << NC << " + c;\n";
+    o << "  if (threadIdx.x >= " << NC << " || oid >= " << nout << ") return;\n";
+    o << "  " << ACC << " acc = sums[0][c];\n#pragma unroll\n  for (int i = 1; i < " << NG << "; ++i) acc = " << red_apply(rn.red, dt, "acc", "sums[i][c]") << ";\n";
+    o << ibody;
+    o << "  const " << ACC << " r = " << red_apply(rn.red, dt, "acc", "(" + ACC + ")" + initv) << ";\n";
+    o << "  out0[oid] = " << Emitter::store_conv(dt, is_narrow_float(dt) ? Emitter::round_narrow(dt, "r") : std::string("(") + info(dt).ctype + ")r") << ";\n}\n\n";
+    Launch L;
+    L.kernel = named("@K@_reduce_generic", finalize(o.str()));
+    L.kind = "reduce_generic";
+    L.grid[0] = (unsigned)((nvec + CX - 1) / CX);
+    L.block[0] = kBlock;
+    for (int i : em.inputs) L.args.push_back(buffer_for(i));
+    L.args.push_back(buffer_for(root));
+    L.algo_bytes = algo_bytes(em.inputs, {root});
+    L.desc = describe(rn.in[0]) + " reduce";
+    plan.launches.push_back(L);
+  }
   void emit_reduce_generic(int root) {
     const Node& rn = g.nodes[root];
     const Node& inn = g.nodes[rn.in[0]];
@@ -4545,6 +4588,17 @@ struct Planner {
     const bool two_pass = split >= 2;
     const int64_t chunk = two_pass ? (inn.ty.dims[red[ks]] + split - 1) / split : 0;
     if (two_pass) split = (inn.ty.dims[red[ks]] + chunk - 1) / chunk;
+    // One launch where the second one would cost more than it spares: a workgroup takes CX vectors of outputs, its threads
+    // every CY-th row of them (64 bytes of a row and 64 rows at a time), and adds the threads' sums through LDS in a fixed
+    // order.  A chain of additions is no longer than that of the chunks (a chunk, the partials of a wavefront, four of those).
+    // Kernels, us, two launches -> one: 1024 x 2048 bf16 4.3 + 4.0 -> 4.0, 1024 x 1000 4.8 + 4.4 -> 4.8, 4096 x 2048 7.4 + 4.2 -> 7.4; f32 1024^2 4.6 + 4.6 -> 5.0, 4096 x 960 4.6 + 5.8 -> 7.2; f64 1024^2 4.4 + 4.1 -> 4.1.
+    constexpr int CX = 4, CY = kBlock / CX;
+    const bool columns = two_pass && RB == 1 && VEC > 1 && red.size() == 1 && opt.column_reduce && red_len <= 4096 && inn.ty.numel() * esz <= (int64_t)16 << 20;
+    if (columns) {
+      const int NC = CX * VEC, NG = kBlock / NC, PER = CY / NG;   // outputs of a workgroup, groups of threads that add them, rows of sums per group
+      emit_reduce_columns(root, eu, kept, red[0], nout, VEC, NC, NG, PER, CX, CY, body, val, ibody, initv);
+      return;
+    }
     std::ostringstream o;
     o << "// reduce (generic" << (two_pass ? ", reduced dimension cut into " + std::to_string(split) + " chunks" : std::string()) << "): " << describe(rn.in[0])
       << " over dims -> " << rn.ty.str() << "\n";
