@@ -264,6 +264,7 @@ rx::PlanOptions plan_options() {
   if (const char* e = getenv("RX_EPILOGUE_INIT")) o.epilogue_init = atoi(e) != 0;
   if (const char* e = getenv("RX_CHAIN_CONVS")) o.chain_convs = atoi(e) != 0;
   if (const char* e = getenv("RX_COLUMN_REDUCE")) o.column_reduce = atoi(e) != 0;
+  if (const char* e = getenv("RX_FOLD_FINALS")) o.fold_finals = atoi(e) != 0;
   if (const char* e = getenv("RX_JOIN_LAUNCHES")) o.join_launches = atoi(e) != 0;
   if (const char* e = getenv("RX_CONV_SPLIT")) o.split_convs = atoi(e) != 0;
   if (const char* e = getenv("RX_IN_PLACE")) o.in_place_updates = atoi(e) != 0;
