@@ -3209,7 +3209,7 @@ struct Planner {
   // 2 to 4 steps (9 and 8 % rms): rounds are of a workgroup over its cells, MB what all of them stage.  A map per step takes
   // 4.4 us.  10 steps, us, tiles of 8 x 8 x 16 and two steps (f32: four) before -> as chosen: 67 x 53 x 39 f64 32.2 -> 26.2,
   // f32 20 -> 17.5; 36 x 36 x 26 f64 28.7 -> 17.7.
-  // (Runs of up to three steps are left as they are.)
+  // (Runs of up to three steps are left as they are, and so are steps that update several arrays in turns.)
   // how many further arrays (0: the choice above is not for these steps)
   int chain3_others(const std::vector<int>& steps, const std::vector<ChainProbe>& probes) const {
     if (g.nodes[steps[0]].ty.rank() != 3 || steps.size() < 4 || opt.chain_steps > 0 || opt.chain_tile[0] > 0 || !opt.chain_fixed_cells) return 0;
@@ -3224,7 +3224,10 @@ struct Planner {
         (own ? others : moved).insert(kv.first);
       }
     for (int x : moved) others.erase(x);
-    for (int x : steps) others.erase(x);
+    for (int x : steps) { others.erase(x); moved.erase(x); }
+    // one array that every step supersedes: its tile and the twin are what the choice counts, and two such arrays may not fit
+    if (moved.size() != 1 || *moved.begin() != probes[0].base) return 0;
+    for (size_t i = 1; i < probes.size(); ++i) if (probes[i].base != steps[i - 1]) return 0;
     return (int)others.size();
   }
   int choose_chain3(size_t n, const int64_t* D, int es, int others, int64_t* T) const {

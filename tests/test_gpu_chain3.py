@@ -27,3 +27,45 @@ def test_chosen_chains_equal_maps(rx, client, monkeypatch, nx, ny, nz, steps, dt
     ref, plain = gpu_run(rx, client, text, args)
     assert all(l["kind"] != "map_chain" for l in plain.launches())
     assert np.array_equal(got[0].a, ref[0].a)
+
+
+def _two_fields(D, steps, dt):
+    """Two arrays that step in turns, each around its own points and those of the other, scaled by a third."""
+    tf, n = "tensor<%s%s>" % ("".join("%dx" % d for d in D), dt), [d - 2 for d in D]
+    ti = "tensor<%s%s>" % ("".join("%dx" % d for d in n), dt)
+    lines, cnt = [], [0]
+
+    def new(s):
+        cnt[0] += 1
+        lines.append("    %%%d = %s" % (cnt[0], s))
+        return "%%%d" % cnt[0]
+
+    def sh(x, *off):
+        return new("stablehlo.slice %s [%s] : (%s) -> %s" % (x, ", ".join("%d:%d" % (1 + o, 1 + o + m) for o, m in zip(off, n)), tf, ti))
+    zero, eighth = new("stablehlo.constant dense<0.0> : tensor<%s>" % dt), new("stablehlo.constant dense<0.125> : %s" % ti)
+    scale = sh("%arg2", 0, 0, 0)
+    f = ["%arg0", "%arg1"]
+    for i in range(2 * steps):
+        a, b = f[i % 2], f[1 - i % 2]
+        s = sh(a, -1, 0, 0)
+        for x, off in ((a, (1, 0, 0)), (a, (0, -1, 0)), (a, (0, 1, 0)), (a, (0, 0, -1)), (b, (0, 0, 1))):
+            s = new("stablehlo.add %s, %s : %s" % (s, sh(x, *off), ti))
+        s = new("stablehlo.multiply %s, %s : %s" % (new("stablehlo.multiply %s, %s : %s" % (s, eighth, ti)), scale, ti))
+        s = new("stablehlo.add %s, %s : %s" % (s, sh(a, 0, 0, 0), ti))
+        f[i % 2] = new("stablehlo.pad %s, %s, low = [1, 1, 1], high = [1, 1, 1], interior = [0, 0, 0] : (%s, tensor<%s>) -> %s" % (s, zero, ti, dt, tf))
+    return ("module {\n  func.func @main(%%arg0: %s, %%arg1: %s, %%arg2: %s) -> (%s, %s) {\n%s\n    return %s, %s : %s, %s\n  }\n}\n"
+            % (tf, tf, tf, tf, tf, "\n".join(lines), f[0], f[1], tf, tf))
+
+
+@pytest.mark.parametrize("dt", ["f64", "f32"])
+@pytest.mark.parametrize("D,steps", [((20, 18, 22), 3), ((39, 53, 67), 5), ((64, 64, 64), 4)])
+def test_steps_of_two_arrays_fit_the_local_memory(rx, client, monkeypatch, D, steps, dt):
+    """The choice counts the tiles of one array; a chain over two, with twice as many, was refused by the device."""
+    text = _two_fields(D, steps, dt)
+    rng = np.random.default_rng(3)
+    args = [I.tensor(rng.uniform(size=D), dt) for _ in range(3)]
+    got, _ = gpu_run(rx, client, text, args)
+    monkeypatch.setenv("RX_CHAIN_STEPS", "1")
+    ref, plain = gpu_run(rx, client, text, args)
+    assert all(l["kind"] != "map_chain" for l in plain.launches())
+    assert np.array_equal(got[0].a, ref[0].a) and np.array_equal(got[1].a, ref[1].a)
