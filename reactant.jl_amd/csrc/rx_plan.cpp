@@ -3204,7 +3204,7 @@ struct Planner {
   // Rank-3 steps that read further arrays at their own position (velocities, coefficients; a chain keeps them in registers):
   // the tile and the number of steps per launch, by the time of the launches that `n` steps take.  Only tiles that give a compute
   // unit one workgroup; larger arrays stay maps, which move them from L2 with less arithmetic (116 x 116 x 70 f64: the best
-  // chain 87 us for 10 steps, maps 100; 171 x 100 x 29: 48 and 45; 206 x 106 x 106: 196 and 230).  Fitted to 51 (f64) and 26 (f32)
+  // chain of those tiles 87 us for 10 steps, maps 100; 171 x 100 x 29: 48 and 45; 206 x 106 x 106: 196 and 230).  Fitted to 51 (f64) and 26 (f32)
   // timings of 8 to 10 advection-diffusion steps on 36 x 36 x 26 to 165 x 100 x 29 points, tiles of 6 x 6 x 12 to 10 x 10 x 32 and
   // 2 to 4 steps (9 and 8 % rms): rounds are of a workgroup over its cells, MB what all of them stage.  A map per step takes
   // 4.4 us.  10 steps, us, tiles of 8 x 8 x 16 and two steps (f32: four) before -> as chosen: 67 x 53 x 39 f64 32.2 -> 26.2,
@@ -3251,6 +3251,32 @@ struct Planner {
             const double us = es == 8 ? 2.1 + fill * (0.59 * (double)per + 0.13 * (double)rounds) + 0.09 * mb : 2.5 + fill * (0.28 * (double)per + 0.16 * (double)rounds) + 0.04 * mb;
             if (us < cost[k]) { cost[k] = us; for (int d = 0; d < 3; ++d) tile[k][d] = t[d]; }
           }
+    }
+    // f64 arrays that need more tiles and that, with the others, are far larger than L2 (a map per step then moves them at
+    // 4.7 TB/s): tiles that fill most of a compute unit's LDS, several rounds of them.  Rows of 32 or 40 results, the only ones
+    // that were never far behind; cells of a thread are not kept in registers (R > 8), which such boxes spill.  Per launch, over
+    // 61 timings of 2 and 3 steps on 0.6 to 3.8 M cells (6.6 % rms): 3.9 + 0.19 us for each round over a step's region, times the
+    // rounds of workgroups, + 4.2 us for 256 000 lines of 128 bytes staged and read.  On 50 further sizes of 1.5 to 4.2 M cells
+    // and 4 to 10 steps the chains took 0.65 to 0.99 of the maps, one 1.04 (mean 0.83: 267 x 136 x 72, 6 steps, 170 -> 116 us;
+    // 367 x 137 x 71, 4 steps, 131 -> 97; 111 x 453 x 31, 8 steps, 106 -> 95).  Below 60 MB, where maps hit L2, it was 0.72 to
+    // 1.26, and f32 0.83 to 1.15: those stay maps, as do sizes whose estimate is not 17 % below that of the maps.
+    const int64_t cells = D[0] * D[1] * D[2], moved = cells * es * (others + 2);
+    if (es == 8 && moved > 60000000) {
+      cost[1] = 2.5 + 0.21e-6 * (double)moved;
+      for (int64_t k = 2; k <= 3; ++k)
+        for (int64_t a = 6; a <= 16; ++a)
+          for (int64_t b = 6; b <= 20; ++b)
+            for (int64_t c : {32, 40}) {
+              const int64_t t[3] = {a, b, c}, box = (a + 2 * k) * (b + 2 * k) * (c + 2 * k);
+              const int64_t wgs = ((D[0] + a - 1) / a) * ((D[1] + b - 1) / b) * ((D[2] + c - 1) / c);
+              if (box <= 8 * 1024 || box > 9 * 1024 || wgs <= 256) continue;
+              int64_t rounds = 0;
+              for (int64_t i = 0; i < k; ++i) rounds += ((a + 2 * i) * (b + 2 * i) * (c + 2 * i) + 1023) / 1024;
+              const int64_t h = 2 * (k - 1), row = c + 2 * k, row1 = c + h;
+              const double lines = (double)((a + 2 * k) * (b + 2 * k)) * ((double)(row * es) / 128 + 1) + (double)(others * (a + h) * (b + h)) * ((double)(row1 * es) / 128 + 1);
+              const double us = 3.87 + 0.191 * (double)((wgs + 255) / 256 * rounds) + 4.16e-3 / 256 * (double)wgs * lines;
+              if (us < 0.83 * (double)k * cost[1] && us < cost[k]) { cost[k] = us; for (int d = 0; d < 3; ++d) tile[k][d] = t[d]; }
+            }
     }
     std::vector<double> best(n + 1, 0);
     std::vector<size_t> first(n + 1, 1);

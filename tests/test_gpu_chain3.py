@@ -29,6 +29,12 @@ def test_chosen_chains_equal_maps(rx, client, monkeypatch, nx, ny, nz, steps, dt
     assert np.array_equal(got[0].a, ref[0].a)
 
 
+@pytest.mark.parametrize("nx,ny,nz,steps", [(255, 72, 99, 5), (90, 250, 100, 6), (24, 455, 205, 4)])
+def test_chosen_chains_of_several_rounds_equal_maps(rx, client, monkeypatch, nx, ny, nz, steps):
+    """More tiles than compute units, boxes of more than eight cells a thread."""
+    test_chosen_chains_equal_maps(rx, client, monkeypatch, nx, ny, nz, steps, "f64")
+
+
 def _two_fields(D, steps, dt):
     """Two arrays that step in turns, each around its own points and those of the other, scaled by a third."""
     tf, n = "tensor<%s%s>" % ("".join("%dx" % d for d in D), dt), [d - 2 for d in D]
