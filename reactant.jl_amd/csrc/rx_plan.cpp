@@ -3203,7 +3203,7 @@ struct Planner {
 
   // Rank-3 steps that read further arrays at their own position (velocities, coefficients; a chain keeps them in registers):
   // the tile and the number of steps per launch, by the time of the launches that `n` steps take.  Only tiles that give a compute
-  // unit one workgroup; larger arrays stay maps, which move them from L2 with less arithmetic (116 x 116 x 70 f64: the best
+  // unit one workgroup; larger arrays (but for those further down) stay maps, which move them from L2 with less arithmetic (116 x 116 x 70 f64: the best
   // chain of those tiles 87 us for 10 steps, maps 100; 171 x 100 x 29: 48 and 45; 206 x 106 x 106: 196 and 230).  Fitted to 51 (f64) and 26 (f32)
   // timings of 8 to 10 advection-diffusion steps on 36 x 36 x 26 to 165 x 100 x 29 points, tiles of 6 x 6 x 12 to 10 x 10 x 32 and
   // 2 to 4 steps (9 and 8 % rms): rounds are of a workgroup over its cells, MB what all of them stage.  A map per step takes
