@@ -1646,6 +1646,21 @@ struct Planner {
     }
     return false;
   }
+  static void replace_all(std::string* t, const std::string& from, const std::string& to) {
+    for (size_t p = 0; (p = t->find(from, p)) != std::string::npos; p += to.size()) t->replace(p, from.size(), to);
+  }
+  // Functions of the text that look at the workgroup's number or at the grid by themselves: a kernel that calls one cannot
+  // be given another number.
+  static std::set<std::string> functions_of_the_grid(const std::string& text) {
+    std::set<std::string> names;
+    const std::string head = "static __device__ __forceinline__ void ";
+    for (size_t at = text.find(head); at != std::string::npos; at = text.find(head, at + 1)) {
+      const size_t name = at + head.size(), end = std::min(text.find(head, name), text.find("extern \"C\" __global__", name));
+      const std::string def = text.substr(name, end == std::string::npos ? end : end - name);
+      if (def.find("blockIdx") != std::string::npos || def.find("gridDim") != std::string::npos) names.insert(def.substr(0, def.find('(')));
+    }
+    return names;
+  }
   // the kernels of `gone` that no launch names any more
   void drop_kernels(const std::set<std::string>& gone) {
     std::string text = src.str();
@@ -1684,6 +1699,8 @@ struct Planner {
       KernelText f, m;
       if (!clear || !find_kernel(text, F.kernel, &f) || !find_kernel(text, M.kernel, &m) || f.params.size() != F.args.size() || m.params.size() != M.args.size()) continue;
       if (f.body.find("return") != std::string::npos || m.body.find("gridDim") != std::string::npos || f.body.find("blockIdx") != std::string::npos) continue;
+      replace_all(&m.body, "blockIdx.x", "bx_");   // a parameter: join_launches numbers the workgroups of its parts itself
+      if (m.body.find("blockIdx") != std::string::npos) continue;
       std::string type = f.params.back().first;   // "T* __restrict__"
       type = type.substr(0, type.find('*'));
       std::ostringstream o, sig, fa, ma;
@@ -1707,9 +1724,9 @@ struct Planner {
       };
       o << "// the end of a reduction and the map that reads its result\n";
       o << "static __device__ __forceinline__ void @K@_final(" << params_of(f) << ") " << f.body << "\n";
-      o << "static __device__ __forceinline__ void @K@_body(" << params_of(m) << ") " << m.body << "\n";
+      o << "static __device__ __forceinline__ void @K@_body(const unsigned bx_, " << params_of(m) << ") " << m.body << "\n";
       o << "extern \"C\" __global__ __launch_bounds__(" << m.bounds << ") void @K@_map(" << sig.str() << ") {\n  __shared__ " << type << " value;\n  @K@_final(" << fa.str()
-        << ");\n  __syncthreads();\n  if (blockIdx.x == 0 && threadIdx.x == 0) f" << F.args.size() - 1 << "[0] = value;\n  @K@_body(" << ma.str() << ");\n}\n\n";
+        << ");\n  __syncthreads();\n  if (blockIdx.x == 0 && threadIdx.x == 0) f" << F.args.size() - 1 << "[0] = value;\n  @K@_body(blockIdx.x, " << ma.str() << ");\n}\n\n";
       J.kernel = named("@K@_map", finalize(o.str()));
       // results: the scalar (in the middle of the arguments; no earlier launch names it) and the map's
       J.desc = F.desc + " ; " + M.desc;
@@ -1732,6 +1749,11 @@ struct Planner {
   void join_launches() {
     if (!opt.join_launches || plan.launches.size() < 3) return;
     std::string text = src.str();
+    const std::set<std::string> own_grid = functions_of_the_grid(text);
+    auto calls_own_grid = [&](const std::string& body) {
+      for (auto& f : own_grid) if (body.find(f + "(") != std::string::npos) return true;
+      return false;
+    };
     struct Group {
       std::vector<size_t> members;
       bool open = false, product = false, maps = false;
@@ -1776,7 +1798,7 @@ struct Planner {
       KernelText k;
       if (product || part) {
         const bool ok = find_kernel(text, L.kernel, &k) && k.params.size() == L.args.size() &&
-                        (product || (k.body.find("blockIdx.z") == std::string::npos && k.body.find("gridDim.y") == std::string::npos && k.body.find("rx_smem") == std::string::npos));
+                        (product || (k.body.find("blockIdx.z") == std::string::npos && k.body.find("gridDim.y") == std::string::npos && k.body.find("rx_smem") == std::string::npos && !calls_own_grid(k.body)));
         if (!ok) part = false;
         if (ok && (product || part)) {
           bool placed = false;
@@ -1839,13 +1861,10 @@ struct Planner {
         if (product) bounds = k.bounds;
         if (defined.insert(L.kernel).second) {
           std::string body = k.body;
-          auto replace = [&](const std::string& from, const std::string& to) {
-            for (size_t p = 0; (p = body.find(from, p)) != std::string::npos; p += to.size()) body.replace(p, from.size(), to);
-          };
           if (!product) {
-            replace("blockIdx.x", "bx_");
-            replace("blockIdx.y", "by_");
-            replace("gridDim.x", std::to_string(L.grid[0]) + "u");
+            replace_all(&body, "blockIdx.x", "bx_");
+            replace_all(&body, "blockIdx.y", "by_");
+            replace_all(&body, "gridDim.x", std::to_string(L.grid[0]) + "u");
           }
           parts << "static __device__ __forceinline__ void @K@_" << m << "(const unsigned bx_, const unsigned by_";
           for (auto& p : k.params) parts << ", " << p.first << " " << p.second;
