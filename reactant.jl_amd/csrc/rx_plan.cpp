@@ -4411,7 +4411,14 @@ struct Planner {
       code += e.take_code();
       return code + "    out0[0] = " + e.store_value(tdt, v) + ";\n";
     };
-    if (one) one_code = stored(em, "a");   // (its operands come after the reduction's)
+    if (one) {
+      // by an emitter of its own: the values that `em` remembers are declared inside the loop.  Its operands come after the reduction's.
+      Emitter last(g, in_memory);
+      last.excess_precision = opt.excess_precision;
+      last.inputs = em.inputs;
+      one_code = stored(last, "a");
+      em.inputs = last.inputs;
+    }
 
     std::ostringstream o;
     o << "// reduce" << (one ? ": " : " (pass 1): ") << describe(rn.in[0]) << (one ? ", one workgroup\n" : " -> partials\n");

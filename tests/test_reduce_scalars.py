@@ -1,0 +1,41 @@
+"""Reductions whose elements, initial value and scalar end read the same scalar: the end is code outside of the loop that read
+it for the elements."""
+import numpy as np
+import pytest
+
+from _harness import gpu_run, oracle_run
+from _loader import load_pkg
+from oracle import stablehlo_interp as I
+
+rx = load_pkg()
+BODIES = {
+    "init": ["%m = stablehlo.multiply %a, %b : T", "%r = stablehlo.reduce(%m init: %s) applies stablehlo.add across dimensions = [0] : (T, S) -> S"],
+    "tail": ["%m = stablehlo.subtract %a, %b : T", "%0 = stablehlo.reduce(%m init: %z) applies stablehlo.add across dimensions = [0] : (T, S) -> S", "%r = stablehlo.multiply %0, %s : S"],
+    "both": ["%d = stablehlo.subtract %a, %b : T", "%m = stablehlo.multiply %d, %d : T",
+             "%0 = stablehlo.reduce(%m init: %s) applies stablehlo.add across dimensions = [0] : (T, S) -> S", "%r = stablehlo.subtract %0, %s : S"],
+}
+
+
+def full(n, dt, form):
+    lines = ["%z = stablehlo.constant dense<0.0> : S", "%b = stablehlo.broadcast_in_dim %s, dims = [] : (S) -> T"] + BODIES[form]
+    text = "module {\n  func.func @main(%a: T, %s: S) -> S {\n    " + "\n    ".join(lines) + "\n    return %r : S\n  }\n}\n"
+    return text.replace("T", "tensor<%dx%s>" % (n, dt)).replace("S", "tensor<%s>" % dt)
+
+
+@pytest.mark.parametrize("form", sorted(BODIES))
+@pytest.mark.parametrize("n", [1, 2, 4099, 8192, 8193])
+def test_full_reductions_compile(n, form):
+    report = rx.compile_offline(full(n, "f32", form))
+    assert report.count("kind=") == (1 if n <= 8192 else 2), report
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["f32", "f64", "bf16"])
+@pytest.mark.parametrize("form", sorted(BODIES))
+@pytest.mark.parametrize("n", [1, 4099, 8192, 8193])
+def test_full_reductions(rx, client, n, form, dt):
+    text = full(n, dt, form)
+    rng = np.random.default_rng(n)
+    args = [I.tensor(rng.integers(-1, 2, size=n), dt), I.tensor(np.asarray(2), dt)]   # whole numbers: sums are exact in every accumulator
+    got, _ = gpu_run(rx, client, text, args)
+    assert np.array_equal(np.asarray(got[0].a), np.asarray(oracle_run(text, args, hifi=True)[0].a))
