@@ -4636,9 +4636,18 @@ struct Planner {
     em.clamp_guards = opt.clamp_pad_reads && opt.window_reduce_vectors && info(inn.ty.dt).size == 2 && !kept.empty() && kept.back() == inn.ty.rank() - 1;
     std::string val = em.emit(rn.in[0], ix);
     std::string body = em.take_code();
-    em.indent = 2;
-    std::string initv = em.emit(rn.in[1], Index{});
-    std::string ibody = em.take_code();
+    // the init value, outside of the loops: by an emitter of its own, since what `e` remembers is declared inside them
+    std::string initv, ibody;
+    auto emit_init = [&](Emitter& e) {
+      Emitter last(g, [&](int x) { return mat[x]; });
+      last.excess_precision = opt.excess_precision;
+      last.inputs = e.inputs;
+      last.indent = 2;
+      initv = last.emit(rn.in[1], Index{});
+      ibody = last.take_code();
+      e.inputs = last.inputs;
+    };
+    emit_init(em);
     // Few outputs and a long reduction: one thread per output would leave most of the chip idle
     // (a column sum of an 8192 x 8192 matrix has 8192 outputs).  The largest reduced dimension is
     // then cut into `split` chunks (blockIdx.y); each chunk writes a partial per output and a
@@ -4696,9 +4705,7 @@ struct Planner {
         emr.indent = 10;
         val = emr.emit(rn.in[0], ix);
         body = emr.take_code();
-        emr.indent = 2;
-        initv = emr.emit(rn.in[1], Index{});
-        ibody = emr.take_code();
+        emit_init(emr);
       }
     }
     Emitter& eu = RB > 1 ? emr : em;     // the emitter whose inputs the kernel takes

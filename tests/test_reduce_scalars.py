@@ -39,3 +39,32 @@ def test_full_reductions(rx, client, n, form, dt):
     args = [I.tensor(rng.integers(-1, 2, size=n), dt), I.tensor(np.asarray(2), dt)]   # whole numbers: sums are exact in every accumulator
     got, _ = gpu_run(rx, client, text, args)
     assert np.array_equal(np.asarray(got[0].a), np.asarray(oracle_run(text, args, hifi=True)[0].a))
+
+
+def some_dims(shape, dim, dt):
+    """sum(a .* s; dims, init = s)"""
+    text = ("module {\n  func.func @main(%a: T, %s: S) -> O {\n    %b = stablehlo.broadcast_in_dim %s, dims = [] : (S) -> T\n    %m = stablehlo.multiply %a, %b : T\n"
+            "    %r = stablehlo.reduce(%m init: %s) applies stablehlo.add across dimensions = [DIM] : (T, S) -> O\n    return %r : O\n  }\n}\n")
+    dims = ["".join("%dx" % d for k, d in enumerate(shape) if not drop or k != dim) for drop in (False, True)]
+    return text.replace("DIM", str(dim)).replace("T", "tensor<%s%s>" % (dims[0], dt)).replace("S", "tensor<%s>" % dt).replace("O", "tensor<%s%s>" % (dims[1], dt))
+
+
+# one launch by columns, two launches, one thread per output (eight and one at a time), two kept dimensions, a row kernel
+FORMS = [((1024, 1024), 0), ((65, 1000), 0), ((4097, 512), 0), ((300, 7), 0), ((20, 4096), 0), ((3, 3), 1), ((3, 130, 1024), 1), ((16, 40, 300), 1), ((8, 640, 128), 0), ((70, 400), 1)]
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f64"])
+@pytest.mark.parametrize("shape,dim", FORMS)
+def test_reductions_of_some_dimensions_compile(shape, dim, dt):
+    assert "code object" in rx.compile_offline(some_dims(shape, dim, dt))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f64"])
+@pytest.mark.parametrize("shape,dim", FORMS)
+def test_reductions_of_some_dimensions(rx, client, shape, dim, dt):
+    text = some_dims(shape, dim, dt)
+    rng = np.random.default_rng(shape[0])
+    args = [I.tensor(rng.integers(-1, 2, size=shape), dt), I.tensor(np.asarray(2), dt)]   # sums are exact in every accumulator
+    got, _ = gpu_run(rx, client, text, args)
+    assert np.array_equal(np.asarray(got[0].a), np.asarray(oracle_run(text, args, hifi=True)[0].a))
