@@ -58,6 +58,8 @@ const char* acc_ctype(DT dt) {
   return info(dt).ctype;
 }
 
+int acc_size(DT dt) { return dt == DT::F64 || info(dt).size == 8 ? 8 : 4; }   // bytes of an accumulator, at most
+
 std::string red_identity(Red r, DT dt) {
   const bool f = is_float(dt), d = dt == DT::F64;
   switch (r) {
@@ -1612,6 +1614,38 @@ struct Planner {
     plan.launches.insert(plan.launches.end(), rest.begin(), rest.end());
   }
 
+  // The LDS arrays of a kernel that may become a part of a joined one: one struct, whose bytes the launch states.  A
+  // kernel with arrays declared otherwise stays by itself.
+  struct SharedArray {
+    std::string type;
+    int size;                      // of an element, or more
+    std::string name;
+    std::vector<int64_t> dims;
+  };
+  static std::string declare_shared(const std::vector<SharedArray>& arrays, unsigned* bytes) {
+    std::string members, names;
+    *bytes = 0;
+    for (auto& a : arrays) {
+      std::string dims;
+      int64_t n = a.size;
+      for (int64_t d : a.dims) { dims += "[" + std::to_string(d) + "]"; n *= d; }
+      members += " __attribute__((aligned(16))) " + a.type + " " + a.name + dims + ";";
+      names += "  auto& " + a.name + " = lds_." + a.name + ";\n";
+      *bytes += (unsigned)((n + 15) / 16 * 16);
+    }
+    return "  __shared__ struct {" + members + " } lds_;\n" + names;
+  }
+  // The same kernel's body with that struct at an address given to it, `smem_` (16-byte aligned); false: it has other arrays.
+  static bool shared_at_address(std::string* body, unsigned bytes) {
+    const std::string head = "__shared__ struct {", tail = "} lds_;";
+    const size_t at = body->find(head), end = at == std::string::npos ? at : body->find(tail, at);
+    if (end != std::string::npos) {
+      const std::string members = body->substr(at + head.size(), end - at - head.size());
+      body->replace(at, end + tail.size() - at, "struct lds_t_ {" + members + "}; static_assert(sizeof(lds_t_) <= " + std::to_string(bytes) + "); lds_t_& lds_ = *reinterpret_cast<lds_t_*>(smem_);");
+    }
+    return body->find("__shared__") == std::string::npos;
+  }
+
   // A kernel of the text written so far, taken apart.
   struct KernelText {
     size_t begin = 0, end = 0;
@@ -1701,6 +1735,7 @@ struct Planner {
       if (f.body.find("return") != std::string::npos || m.body.find("gridDim") != std::string::npos || f.body.find("blockIdx") != std::string::npos) continue;
       replace_all(&m.body, "blockIdx.x", "bx_");   // a parameter: join_launches numbers the workgroups of its parts itself
       if (m.body.find("blockIdx") != std::string::npos) continue;
+      if (!shared_at_address(&f.body, F.shared_bytes) || m.body.find("__shared__") != std::string::npos) continue;
       std::string type = f.params.back().first;   // "T* __restrict__"
       type = type.substr(0, type.find('*'));
       std::ostringstream o, sig, fa, ma;
@@ -1708,11 +1743,11 @@ struct Planner {
       J.args.clear();
       for (size_t a = 0; a < F.args.size(); ++a) {   // the reduction's operands, its result last
         sig << (a ? ", " : "") << f.params[a].first << " f" << a;
-        fa << (a ? ", " : "") << (a + 1 < F.args.size() ? "f" + std::to_string(a) : std::string("&value"));
+        fa << ", " << (a + 1 < F.args.size() ? "f" + std::to_string(a) : std::string("&value"));
         J.args.push_back(F.args[a]);
       }
       for (size_t a = 0; a < M.args.size(); ++a) {
-        ma << (a ? ", " : "") << (M.args[a] == out ? std::string("&value") : "m" + std::to_string(a));
+        ma << ", " << (M.args[a] == out ? std::string("&value") : "m" + std::to_string(a));
         if (M.args[a] == out) continue;
         sig << ", " << m.params[a].first << " m" << a;
         J.args.push_back(M.args[a]);
@@ -1723,10 +1758,11 @@ struct Planner {
         return t;
       };
       o << "// the end of a reduction and the map that reads its result\n";
-      o << "static __device__ __forceinline__ void @K@_final(" << params_of(f) << ") " << f.body << "\n";
+      o << "static __device__ __forceinline__ void @K@_final(unsigned char* smem_, " << params_of(f) << ") " << f.body << "\n";
       o << "static __device__ __forceinline__ void @K@_body(const unsigned bx_, " << params_of(m) << ") " << m.body << "\n";
-      o << "extern \"C\" __global__ __launch_bounds__(" << m.bounds << ") void @K@_map(" << sig.str() << ") {\n  __shared__ " << type << " value;\n  @K@_final(" << fa.str()
-        << ");\n  __syncthreads();\n  if (blockIdx.x == 0 && threadIdx.x == 0) f" << F.args.size() - 1 << "[0] = value;\n  @K@_body(blockIdx.x, " << ma.str() << ");\n}\n\n";
+      o << "extern \"C\" __global__ __launch_bounds__(" << m.bounds << ") void @K@_map(" << sig.str() << ") {\n"
+        << declare_shared({{type, 8, "value", {}}, {"unsigned char", 1, "final_", {F.shared_bytes}}}, &J.shared_bytes)
+        << "  @K@_final(final_" << fa.str() << ");\n  __syncthreads();\n  if (blockIdx.x == 0 && threadIdx.x == 0) f" << F.args.size() - 1 << "[0] = value;\n  @K@_body(blockIdx.x" << ma.str() << ");\n}\n\n";
       J.kernel = named("@K@_map", finalize(o.str()));
       // results: the scalar (in the middle of the arguments; no earlier launch names it) and the map's
       J.desc = F.desc + " ; " + M.desc;
@@ -1745,7 +1781,11 @@ struct Planner {
   // nor written by them).  At most one product per group, first, so that its tiles' numbers are the grid's; beside it 128
   // workgroups of reductions, since all of them are given its LDS (maps, which take as long as their bytes do, stay by themselves);
   // without a product 2048 workgroups, of launches that move up to 32 MB each.
-  // Training step of 784 -> 2048 -> 1000 over 1024 rows in bf16: 12 launches -> 7, 77.4 -> 60.4 us.
+  // The parts' LDS lies over one another, and over the product's: a workgroup runs one of them, and a part beside a product
+  // leaves as many of its workgroups on a compute unit as there are without the part.
+  // Training steps, separate -> joined, us: 784 -> 2048 -> 1000 over 1024 rows in bf16 74.5 -> 56.7, 784 -> 1024 -> 1000 over 1992
+  // 93.5 -> 61.3 (its largest tile takes all of the LDS), 512 -> 4096 -> 10 .. 1024 -> 1024 -> 1024 over 84 to 3852 rows in bf16
+  // and f32, 26 of them: 0.78 to 1.00 of the separate launches.
   void join_launches() {
     if (!opt.join_launches || plan.launches.size() < 3) return;
     std::string text = src.str();
@@ -1798,7 +1838,7 @@ struct Planner {
       KernelText k;
       if (product || part) {
         const bool ok = find_kernel(text, L.kernel, &k) && k.params.size() == L.args.size() &&
-                        (product || (k.body.find("blockIdx.z") == std::string::npos && k.body.find("gridDim.y") == std::string::npos && k.body.find("rx_smem") == std::string::npos && !calls_own_grid(k.body)));
+                        (product || (k.body.find("blockIdx.z") == std::string::npos && k.body.find("gridDim.y") == std::string::npos && k.body.find("rx_smem") == std::string::npos && !calls_own_grid(k.body) && shared_at_address(&k.body, L.shared_bytes)));
         if (!ok) part = false;
         if (ok && (product || part)) {
           bool placed = false;
@@ -1851,6 +1891,7 @@ struct Planner {
       F.grid[0] = 0;
       F.grid[1] = 1;
       F.block[0] = G.block;
+      unsigned shared = 0;   // a workgroup runs one part: its LDS is the product's, or the largest of the parts'
       std::set<std::string> defined;
       std::string bounds = std::to_string(G.block);
       for (size_t m = 0; m < G.members.size(); ++m) {
@@ -1865,8 +1906,9 @@ struct Planner {
             replace_all(&body, "blockIdx.x", "bx_");
             replace_all(&body, "blockIdx.y", "by_");
             replace_all(&body, "gridDim.x", std::to_string(L.grid[0]) + "u");
+            shared_at_address(&body, L.shared_bytes);
           }
-          parts << "static __device__ __forceinline__ void @K@_" << m << "(const unsigned bx_, const unsigned by_";
+          parts << "static __device__ __forceinline__ void @K@_" << m << "(const unsigned bx_, const unsigned by_, unsigned char* smem_";
           for (auto& p : k.params) parts << ", " << p.first << " " << p.second;
           parts << ") " << body << "\n";
         }
@@ -1875,7 +1917,7 @@ struct Planner {
         const unsigned first = F.grid[0], wgs = L.grid[0] * L.grid[1];
         calls << "  if (blockIdx.x < " << first + wgs << "u) {";
         if (L.block[0] < G.block) calls << " if (threadIdx.x >= " << L.block[0] << "u) return;";
-        calls << " const unsigned b = blockIdx.x - " << first << "u; @K@_" << as << "(b % " << L.grid[0] << "u, b / " << L.grid[0] << "u";
+        calls << " const unsigned b = blockIdx.x - " << first << "u; @K@_" << as << "(b % " << L.grid[0] << "u, b / " << L.grid[0] << "u, smem_";
         for (size_t a = 0; a < L.args.size(); ++a) {
           sig << (F.args.empty() ? "" : ", ") << k.params[a].first << " p" << F.args.size();
           calls << ", p" << F.args.size();
@@ -1883,15 +1925,21 @@ struct Planner {
         }
         calls << "); return; }\n";
         F.grid[0] += wgs;
-        F.lds_bytes = std::max(F.lds_bytes, L.lds_bytes);
+        shared = std::max(shared, L.shared_bytes);
         F.algo_bytes += L.algo_bytes;
         F.flops += L.flops;
         F.desc += (m ? " | " : "") + L.desc;
         if (!uses.count(L.kernel)) gone.insert(L.kernel);
       }
       std::ostringstream o;
-      o << "// " << G.members.size() << " launches that do not depend on one another, as one\n" << parts.str() << "extern \"C\" __global__ __launch_bounds__(" << bounds << ") void @K@_joined(" << sig.str() << ") {\n"
-        << calls.str() << "}\n\n";
+      o << "// " << G.members.size() << " launches that do not depend on one another, as one\n" << parts.str() << "extern \"C\" __global__ __launch_bounds__(" << bounds << ") void @K@_joined(" << sig.str() << ") {\n";
+      if (G.product) {
+        F.lds_bytes = std::max(F.lds_bytes, shared);
+        o << "  extern __shared__ __attribute__((aligned(16))) unsigned char rx_smem[];\n  unsigned char* const smem_ = rx_smem;\n";
+      } else {
+        o << "  __shared__ __attribute__((aligned(16))) unsigned char smem_[" << std::max(16u, shared) << "];\n";
+      }
+      o << calls.str() << "}\n\n";
       F.kernel = named("@K@_joined", finalize(o.str()));
       out.push_back(F);
     }
@@ -4446,7 +4494,8 @@ struct Planner {
     o << "        }\n      }\n    }\n  }\n";
     o << "  " << ACC << " a = acc[0];\n";
     o << "#pragma unroll\n  for (int u = 1; u < " << U << "; ++u) a = " << red_apply(rn.red, dt, "a", "acc[u]") << ";\n";
-    o << "  __shared__ " << ACC << " lds[" << BLK / 64 << "];\n";
+    unsigned shared = 0, shared2 = 0;
+    o << declare_shared({{ACC, acc_size(dt), "lds", {BLK / 64}}}, &shared);
     o << "  a = rx_block_reduce<" << ACC << ", decltype(" << red_functor(rn.red) << "), " << BLK / 64 << ">(a, " << red_functor(rn.red) << ", lds);\n";
     if (one) {
       o << "  if (threadIdx.x == 0) {\n" << one_code << "  }\n}\n\n";
@@ -4455,6 +4504,7 @@ struct Planner {
       L.kind = "reduce";
       L.grid[0] = 1;
       L.block[0] = BLK;
+      L.shared_bytes = shared;
       for (int i : em.inputs) L.args.push_back(buffer_for(i));
       L.args.push_back(buffer_for(tail));
       L.algo_bytes = algo_bytes(em.inputs, {}) + info(tdt).size;
@@ -4525,7 +4575,7 @@ struct Planner {
         s2 += ", " + ptr_decl(info(tdt).stype, false, "out0") + ")";
         o << s2 << " {\n";
       }
-      o << "  __shared__ " << ACC << " lds[" << kBlock / 64 << "];\n";
+      o << declare_shared({{ACC, acc_size(dt), "lds", {kBlock / 64}}}, &shared2);
       combine(o, "partial");
       o << "  }\n}\n\n";
     }
@@ -4537,6 +4587,7 @@ struct Planner {
     L1.kind = "reduce";
     L1.grid[0] = G;
     L1.block[0] = kBlock;
+    L1.shared_bytes = shared;
     for (int i : em.inputs) L1.args.push_back(buffer_for(i));
     L1.args.push_back(sc);
     L1.algo_bytes = algo_bytes(em.inputs, {}) + info(dt).size;
@@ -4561,6 +4612,7 @@ struct Planner {
     L2.kind = "reduce_final";
     L2.grid[0] = 1;
     L2.block[0] = kBlock;
+    L2.shared_bytes = shared2;
     L2.args.push_back(sc);
     for (int i : in2) L2.args.push_back(buffer_for(i));
     L2.args.push_back(buffer_for(tail));
@@ -4579,7 +4631,8 @@ struct Planner {
     std::ostringstream o;
     o << "// reduce (columns): " << describe(rn.in[0]) << " -> " << rn.ty.str() << "\n";
     o << signature("@K@_reduce_generic", em.inputs, {{info(dt).stype, "out0"}}) << " {\n";
-    o << "  __shared__ " << ACC << " part[" << CY << "][" << NC << "], sums[" << NG << "][" << NC << "];\n";
+    unsigned shared = 0;
+    o << declare_shared({{ACC, acc_size(dt), "part", {CY, NC}}, {ACC, acc_size(dt), "sums", {NG, NC}}}, &shared);
     o << "  const int cx = threadIdx.x % " << CX << ", cy = threadIdx.x / " << CX << ";\n";
     o << "  {\n    const " << it << " vid = rx_min<" << it << ">((" << it << ")blockIdx.x * " << CX << " + cx, " << nvec - 1 << ");\n";
     o << "    " << it << " rr = vid * " << VEC << ";\n";
@@ -4606,6 +4659,7 @@ struct Planner {
     L.kind = "reduce_generic";
     L.grid[0] = (unsigned)((nvec + CX - 1) / CX);
     L.block[0] = kBlock;
+    L.shared_bytes = shared;
     for (int i : em.inputs) L.args.push_back(buffer_for(i));
     L.args.push_back(buffer_for(root));
     L.algo_bytes = algo_bytes(em.inputs, {root});
@@ -4800,6 +4854,7 @@ struct Planner {
     for (int k = (int)red.size() - 1; k >= 0 && RB == 1; --k) o << std::string(2 + 2 * k, ' ') << "}\n";
     std::string rv = is_narrow_float(dt) ? Emitter::round_narrow(dt, "r") : std::string("(") + info(dt).ctype + ")r";
     std::vector<int> fin_inputs;
+    unsigned shared = 0;     // of the combine kernel
     int comb_lanes = 1;      // wavefronts of the combine kernel that share an output
     if (!two_pass) {
       o << ibody;
@@ -4832,7 +4887,7 @@ struct Planner {
       // 8192 outputs (column sums of 8192^2: combine 7.8 -> 3 us).
       comb_lanes = split >= 16 ? kBlock / 64 : 1;
       if (comb_lanes > 1) {
-        o << "  __shared__ " << ACC << " part[" << kBlock << "];\n";
+        o << declare_shared({{ACC, acc_size(dt), "part", {kBlock}}}, &shared);
         o << "  const int oid = (int)blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;\n";
         o << "  " << ACC << " acc = " << red_identity(rn.red, dt) << ";\n";
         o << "  if (oid < " << nout << ")\n#pragma unroll 8\n    for (int s = w; s < " << split << "; s += " << comb_lanes << ") acc = "
@@ -4873,6 +4928,7 @@ struct Planner {
     L2.kind = "reduce_final";
     L2.grid[0] = (unsigned)(comb_lanes > 1 ? (nout + 63) / 64 : (nout + kBlock - 1) / kBlock);
     L2.block[0] = kBlock;
+    L2.shared_bytes = shared;
     L2.args.push_back(sc);
     for (int i : fin_inputs) L2.args.push_back(buffer_for(i));
     L2.args.push_back(buffer_for(root));

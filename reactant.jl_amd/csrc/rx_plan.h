@@ -23,7 +23,8 @@ struct Launch {
   std::string kind;            // "map" | "reduce" | "reduce_final" | "row" | "dot" | "gemm_*"
   unsigned grid[3] = {1, 1, 1};
   unsigned block[3] = {1, 1, 1};
-  unsigned lds_bytes = 0;
+  unsigned lds_bytes = 0;      // dynamic
+  unsigned shared_bytes = 0;   // static, of the arrays that Planner::declare_shared declares
   std::vector<int> args;       // buffer ids, in kernel parameter order
   int n_outputs = 1;           // trailing args written by the kernel
   double algo_bytes = 0;       // compulsory HBM traffic: distinct inputs once + outputs once

@@ -1,5 +1,7 @@
-"""Launches that run as one (folded reduction ends, joined launches): the plans' texts and resources, without a GPU."""
+"""Launches that run as one (folded reduction ends, joined launches): the texts and the local memory of such plans, and their results."""
+import os
 import re
+import subprocess
 
 import numpy as np
 
@@ -10,6 +12,7 @@ from _loader import load_pkg
 from oracle import stablehlo_interp as I
 
 rx = load_pkg()
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 
 
 def two_quantizations(shape0, shape1, dt):
@@ -59,3 +62,57 @@ def test_two_quantizations(rx, client, a, b, dt):
     for g, r in zip(got, oracle_run(text, args)):
         g, r = np.asarray(g.a, dtype=np.float64), np.asarray(r.a, dtype=np.float64)
         assert np.all(np.abs(g - r) <= {"bf16": 2.0 ** -8, "f32": 2.0 ** -23}[dt] * np.abs(r))      # a division, rounded: at most one unit in the last place
+
+
+def sums_beside(shapes, dt, product=None):
+    """Column sums and a full sum of independent tensors, and a matrix product of others, in one module."""
+    T = lambda *d: "tensor<%s%s>" % ("".join("%dx" % v for v in d), dt)   # noqa: E731
+    lines, types, outs = ["    %%z = stablehlo.constant dense<0.0> : %s" % T()], [], []
+    if product:
+        m, n, k = product
+        types += [T(m, k), T(k, n)]
+        lines.append("    %%p = stablehlo.dot_general %%arg0, %%arg1, contracting_dims = [1] x [0] : (%s, %s) -> %s" % (T(m, k), T(k, n), T(m, n)))
+        outs.append(("%p", T(m, n)))
+    for r, c in shapes:
+        i = len(types)
+        types.append(T(r, c))
+        for dims, out in (("0", T(c)), ("0, 1", T())):
+            lines.append("    %%r%d_%d = stablehlo.reduce(%%arg%d init: %%z) applies stablehlo.add across dimensions = [%s] : (%s, %s) -> %s" % (i, len(dims), i, dims, T(r, c), T(), out))
+            outs.append(("%%r%d_%d" % (i, len(dims)), out))
+    rt = ", ".join(t for _, t in outs)
+    return ("module {\n  func.func @main(%s) -> (%s) {\n%s\n    return %s : %s\n  }\n}\n"
+            % (", ".join("%%arg%d: %s" % kv for kv in enumerate(types)), rt, "\n".join(lines), ", ".join(o for o, _ in outs), rt))
+
+
+# a product whose tile takes all of the LDS; more differing sums than the LDS has room for one after the other; reductions of one
+# workgroup of 1024 threads beside others
+BESIDE = [(((512, 1024), (1024, 1000), (768, 1024)), "bf16", (2304, 2048, 2048)), (((64, 520), (65, 1000)), "f32", (512, 512, 256)),
+          (tuple((512, 528 + 16 * i) for i in range(24)), "bf16", None), (((8, 1000), (100, 1032), (1000, 1024), (7, 33)), "f32", None)]
+
+
+@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+@pytest.mark.parametrize("shapes,dt,product", BESIDE)
+def test_joined_kernels_fit_the_local_memory(tmp_path, monkeypatch, shapes, dt, product):
+    monkeypatch.setenv("RX_DUMP_CODE_OBJECT", str(tmp_path / "code"))
+    report = rx.compile_offline(sums_beside(shapes, dt, product))
+    notes = subprocess.run([READELF, "--notes", str(tmp_path / "code")], check=True, capture_output=True, text=True).stdout
+    static = {m.group(2): int(m.group(1)) for m in re.finditer(r"\.group_segment_fixed_size: (\d+).*?\.symbol: +(\w+)\.kd", notes, re.S)}
+    joined = [l.split() for l in report.splitlines() if "kind=" in l and "_joined" in l]
+    assert joined
+    for l in joined:
+        lds = int(next(w for w in l if w.startswith("lds="))[4:])
+        assert lds + static[l[1]] <= 160 * 1024 and (static[l[1]] == 0 if "gemm" in l[2] else lds == 0), l
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shapes,dt,product", BESIDE)
+def test_sums_beside_a_product(rx, client, shapes, dt, product):
+    text = sums_beside(shapes, dt, product)
+    rng = np.random.default_rng(len(shapes))
+    dims = ([(product[0], product[2]), (product[2], product[1])] if product else []) + list(shapes)
+    x = [rng.integers(-1, 2, size=d).astype(np.float64) for d in dims]      # whole numbers: sums and products are exact in every accumulator
+    got, exe = gpu_run(rx, client, text, [I.tensor(v, dt) for v in x])
+    assert any("_joined" in l["kernel"] for l in exe.launches())
+    want = ([x[0] @ x[1]] if product else []) + [s for v in x[2 if product else 0:] for s in (v.sum(axis=0), v.sum())]
+    for g, w in zip(got, want):
+        assert np.array_equal(np.asarray(g.a), np.asarray(I.tensor(w, dt).a))
