@@ -1799,7 +1799,11 @@ struct Planner {
       bool open = false, product = false, maps = false;
       unsigned others = 0;   // workgroups beside a product
       unsigned block = 0;
+      size_t params = 0;
     };
+    // The joined kernel takes every part's pointers, and tries its parts one after the other: 64 parts, as in
+    // merge_parameter_maps, and 2 KB of pointers.
+    constexpr size_t MAX_PARTS = 64, MAX_PARAMS = 256;
     const size_t n = plan.launches.size();
     std::vector<Group> groups;
     std::vector<size_t> group_of(n, 0);
@@ -1844,10 +1848,11 @@ struct Planner {
           bool placed = false;
           for (size_t q = lo; q < groups.size() && !placed; ++q) {
             Group& G = groups[q];
-            if (!G.open || (product && (G.product || G.maps || G.others > 128 || G.block > L.block[0])) || (part && G.product && (L.kind == "map" || G.others + wgs > 128 || L.block[0] > G.block)) ||
+            if (!G.open || G.members.size() >= MAX_PARTS || G.params + L.args.size() > MAX_PARAMS || (product && (G.product || G.maps || G.others > 128 || G.block > L.block[0])) || (part && G.product && (L.kind == "map" || G.others + wgs > 128 || L.block[0] > G.block)) ||
                 (part && !G.product && (G.others + wgs > 2048)))
               continue;
             G.members.push_back(j);
+            G.params += L.args.size();
             if (product) { G.product = true; G.block = L.block[0]; }
             else { G.others += wgs; G.block = std::max(G.block, L.block[0]); G.maps = G.maps || L.kind == "map"; }
             group_of[j] = q;
@@ -1856,6 +1861,7 @@ struct Planner {
           if (placed) continue;
           Group G;
           G.members = {j};
+          G.params = L.args.size();
           G.open = true;
           G.product = product;
           G.maps = L.kind == "map";

@@ -116,3 +116,26 @@ def test_sums_beside_a_product(rx, client, shapes, dt, product):
     want = ([x[0] @ x[1]] if product else []) + [s for v in x[2 if product else 0:] for s in (v.sum(axis=0), v.sum())]
     for g, w in zip(got, want):
         assert np.array_equal(np.asarray(g.a), np.asarray(I.tensor(w, dt).a))
+
+
+def many_sums(n):
+    """Sums of n short vectors of differing lengths."""
+    args = ["%%a%d: tensor<%dxf32>" % (i, 3 + i) for i in range(n)]
+    lines = ["    %%r%d = stablehlo.reduce(%%a%d init: %%z) applies stablehlo.add across dimensions = [0] : (tensor<%dxf32>, tensor<f32>) -> tensor<f32>" % (i, i, 3 + i) for i in range(n)]
+    rt = ", ".join(["tensor<f32>"] * n)
+    return ("module {\n  func.func @main(%s) -> (%s) {\n    %%z = stablehlo.constant dense<0.0> : tensor<f32>\n%s\n    return %s : %s\n  }\n}\n"
+            % (", ".join(args), rt, "\n".join(lines), ", ".join("%%r%d" % i for i in range(n)), rt))
+
+
+def test_a_joined_kernel_has_a_bounded_number_of_parts():
+    report = rx.compile_offline(many_sums(130), True)
+    assert kinds(report) == ["reduce"] * 3, report[:2000]
+    for m in re.finditer(r"void \w+_joined\((.*?)\) \{\n", report):
+        assert m.group(1).count(", ") < 256
+
+
+@pytest.mark.gpu
+def test_many_sums(rx, client):
+    args = [I.tensor(np.arange(3 + i, dtype=np.float64) - i, "f32") for i in range(130)]      # exact
+    got, _ = gpu_run(rx, client, many_sums(130), args)
+    assert [float(np.asarray(g.a)) for g in got] == [float(np.asarray(a.a, dtype=np.float64).sum()) for a in args]
