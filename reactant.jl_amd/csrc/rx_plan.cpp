@@ -1721,10 +1721,9 @@ struct Planner {
       if (F.kind != "reduce_final" || F.grid[0] != 1 || F.grid[1] != 1 || F.block[0] != (unsigned)kBlock || F.args.size() < 2) continue;
       if (M.kind != "map" || M.grid[1] != 1 || M.grid[2] != 1 || M.grid[0] < 1 || M.grid[0] > 2048 || M.block[0] != (unsigned)kBlock || M.lds_bytes != 0) continue;
       const int out = F.args.back();
-      const BufferDesc &S = plan.buffers[F.args[0]], &O = plan.buffers[out];
-      if (S.kind != BufferDesc::Scratch || O.kind != BufferDesc::Temp || O.ty.numel() != 1 || O.is_result) continue;
-      const int64_t partials = S.bytes / (O.ty.dt == DT::F64 || info(O.ty.dt).size == 8 ? 8 : 4);
-      if (partials < 64 || partials > 512) continue;
+      const BufferDesc& O = plan.buffers[out];
+      if (plan.buffers[F.args[0]].kind != BufferDesc::Scratch || O.kind != BufferDesc::Temp || O.ty.numel() != 1 || O.is_result) continue;
+      if (F.partials < 64 || F.partials > 512) continue;
       if (std::count(M.args.begin(), M.args.end(), out) != 1 || M.args.back() == out) continue;
       // nothing that the reduction's end reads is written by the map
       bool clear = true;
@@ -4619,6 +4618,7 @@ struct Planner {
     L2.grid[0] = 1;
     L2.block[0] = kBlock;
     L2.shared_bytes = shared2;
+    L2.partials = G;
     L2.args.push_back(sc);
     for (int i : in2) L2.args.push_back(buffer_for(i));
     L2.args.push_back(buffer_for(tail));

@@ -25,6 +25,7 @@ struct Launch {
   unsigned block[3] = {1, 1, 1};
   unsigned lds_bytes = 0;      // dynamic
   unsigned shared_bytes = 0;   // static, of the arrays that Planner::declare_shared declares
+  int partials = 0;            // of a full reduction, which this launch combines
   std::vector<int> args;       // buffer ids, in kernel parameter order
   int n_outputs = 1;           // trailing args written by the kernel
   double algo_bytes = 0;       // compulsory HBM traffic: distinct inputs once + outputs once

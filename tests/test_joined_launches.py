@@ -64,6 +64,20 @@ def test_two_quantizations(rx, client, a, b, dt):
         assert np.all(np.abs(g - r) <= {"bf16": 2.0 ** -8, "f32": 2.0 ** -23}[dt] * np.abs(r))      # a division, rounded: at most one unit in the last place
 
 
+@pytest.mark.parametrize("dt,n,tail,folded", [("f32", 512 * 2048, "f64", True), ("f32", 1024 * 4096, "f16", False), ("f64", 32 * 2048, "f32", False), ("f64", 64 * 2048, "f32", True), ("f32", 32 * 4096, "f64", False)])
+def test_partials_are_counted_whatever_the_type_of_the_end(dt, n, tail, folded):
+    """x - s and y - s for s = sin(tanh(exp(sqrt(max(x))))) in a type of another width than its reduction: folded from 64 to 512 partials"""
+    t, u, s, r, w = "tensor<%dx%s>" % (n, dt), "tensor<%dx%s>" % (n, tail), "tensor<%s>" % dt, "tensor<%s>" % tail, "tensor<77x%s>" % tail
+    report = rx.compile_offline(
+        "module {\n  func.func @main(%%a: %s, %%b: %s) -> (%s, %s) {\n    %%z = stablehlo.constant dense<0.0> : %s\n"
+        "    %%0 = stablehlo.reduce(%%a init: %%z) applies stablehlo.maximum across dimensions = [0] : (%s, %s) -> %s\n    %%1 = stablehlo.sqrt %%0 : %s\n"
+        "    %%2 = stablehlo.exponential %%1 : %s\n    %%t = stablehlo.tanh %%2 : %s\n    %%3 = stablehlo.sine %%t : %s\n    %%4 = stablehlo.convert %%3 : (%s) -> %s\n"
+        "    %%5 = stablehlo.broadcast_in_dim %%4, dims = [] : (%s) -> %s\n    %%6 = stablehlo.convert %%a : (%s) -> %s\n    %%7 = stablehlo.subtract %%6, %%5 : %s\n"
+        "    %%8 = stablehlo.broadcast_in_dim %%4, dims = [] : (%s) -> %s\n    %%9 = stablehlo.subtract %%b, %%8 : %s\n    return %%7, %%9 : %s, %s\n  }\n}\n"
+        % (t, w, u, w, s, t, s, s, s, s, s, s, s, r, r, u, t, u, u, r, w, w, u, w))
+    assert kinds(report)[:2] == (["reduce", "map"] if folded else ["reduce", "reduce_final"]), report[:2000]
+
+
 def sums_beside(shapes, dt, product=None):
     """Column sums and a full sum of independent tensors, and a matrix product of others, in one module."""
     T = lambda *d: "tensor<%s%s>" % ("".join("%dx" % v for v in d), dt)   # noqa: E731
