@@ -4626,17 +4626,47 @@ struct Planner {
     plan.launches.push_back(L2);
   }
 
-  // generic reduction: one thread per output element, sequential loops over reduced dims
-  void emit_reduce_columns(int root, Emitter& em, const std::vector<int>& kept, int red, int64_t nout, int VEC, int NC, int NG, int PER, int CX, int CY, const std::string& body,
+  // The longest columns that emit_reduce_columns is given: by what its kernel computes for an element.  Up to 1024 rows a thread
+  // adds 16 of them, as a thread of the two-launch form does, so that the second launch is spared whatever an element costs.  Longer
+  // columns leave that form more threads, which only elements of little arithmetic do not need.  Two launches -> one, us per call
+  // (columns of 1 and 4 KB rows; with workgroups of 256, and of 1024 threads from 1025 rows on):
+  //   sums alone: 1024 rows f32 8.9 -> 6.2, bf16 8.8 -> 6.2; 4096 f32 8.9 -> 6.4 and 8.8, bf16 9.0 -> 6.3 and 11.2 -> 8.8 (256 threads: 9.2);
+  //   twelve products: 1000 rows bf16 10.9 -> 6.4, 4096 rows f32 9.2 -> 6.4 and 9.2, f64 9.0 -> 6.3, bf16 9.8 -> 8.9 and 13.7 -> 12.4
+  //     (256 threads: 15 and 18; four products 9.0 -> 11.4 and 12.1 -> 21.3);
+  //   tanh: 1024 rows f32 12.9 -> 12.2, f64 14.4 -> 13.1; 2000 rows 15.1 -> 25.7, 1024 threads 15.6, 4096 15.4 -> 47.8 and 29.8;
+  //   four divisions: 1000 rows bf16 19.1 -> 14.9, f32 12.6 -> 9.8, but 1024 rows 9.1 -> 9.7.
+  // Beside a product (join_launches) the sums take compute units that it leaves idle, in workgroups no larger than its: training
+  // steps in bf16 over 1646 rows, 56.9 -> 52.1 us (1024 threads: 61.3), over 3320 rows 100 -> 75 (96).
+  int64_t column_rows(int operand, bool beside) const {
+    int64_t light = 0, heavy = 0;
+    if (!mat[operand])
+      for (int x : cone_nodes(operand)) {
+        const Node& n = g.nodes[x];
+        if (mat[x] || !is_arith(n.k)) continue;
+        static const std::set<std::string> few = {"abs", "negate", "sign", "floor", "ceil", "not", "is_finite"}, many = {"divide", "remainder", "power", "atan2"};
+        (n.k == OpK::Gelu || (n.k == OpK::Unary && !few.count(n.op)) || (n.k == OpK::Binary && many.count(n.op)) ? heavy : light)++;
+      }
+    if (heavy > 0) return std::min<int64_t>(1024, 3072 / heavy);
+    return beside && light > 2 ? 2048 : 4096;
+  }
+  // Column sums in one launch (emit_reduce_generic chooses): a workgroup takes CX vectors of outputs, its threads every CY-th row
+  // of them, in batches of up to eight whose loads are under way together.
+  void emit_reduce_columns(int root, Emitter& em, const std::vector<int>& kept, int red, int64_t nout, int VEC, int CX, int CY, const std::string& body,
                  const std::string& val, const std::string& ibody, const std::string& initv) {
     const Node& rn = g.nodes[root];
     const Node& inn = g.nodes[rn.in[0]];
     const DT dt = rn.ty.dt;
     const std::string ACC = acc_ctype(dt), it = em.idx_t();
     const int64_t len = inn.ty.dims[red], nvec = nout / VEC;
+    const int BLK = CX * CY, NC = CX * VEC;                         // threads, outputs
+    const int NG = std::min(BLK / NC, CY > 64 ? 16 : CY), PER = CY / NG;   // groups of threads' sums that are added first, sums in a group
+    // whole rounds of the threads over the rows, in batches of four to eight that leave no round over where there are such
+    const int64_t rounds = len / CY;
+    int64_t B = std::min<int64_t>(rounds, 8);
+    for (int64_t b = B; b >= 4; --b) if (rounds % b == 0) { B = b; break; }
     std::ostringstream o;
     o << "// reduce (columns): " << describe(rn.in[0]) << " -> " << rn.ty.str() << "\n";
-    o << signature("@K@_reduce_generic", em.inputs, {{info(dt).stype, "out0"}}) << " {\n";
+    o << signature("@K@_reduce_generic", em.inputs, {{info(dt).stype, "out0"}}, BLK) << " {\n";
     unsigned shared = 0;
     o << declare_shared({{ACC, acc_size(dt), "part", {CY, NC}}, {ACC, acc_size(dt), "sums", {NG, NC}}}, &shared);
     o << "  const int cx = threadIdx.x % " << CX << ", cy = threadIdx.x / " << CX << ";\n";
@@ -4647,12 +4677,16 @@ struct Planner {
       o << "    rr /= " << inn.ty.dims[kept[k]] << ";\n";
     }
     o << "    " << ACC << " accv[" << VEC << "];\n#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) accv[l] = " << red_identity(rn.red, dt) << ";\n";
-    o << "#pragma unroll 8\n    for (" << it << " r0 = cy; r0 < " << len << "; r0 += " << CY << ") {\n#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) {\n";
+    o << "    auto add = [&](const " << it << " r0) __attribute__((always_inline)) {\n#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) {\n";
     o << "      const " << it << " o" << kept.size() - 1 << " = o" << kept.size() - 1 << "b + l;\n" << body;
-    o << "      accv[l] = " << red_apply(rn.red, dt, "accv[l]", "(" + ACC + ")" + val) << ";\n    }\n    }\n";
+    o << "      accv[l] = " << red_apply(rn.red, dt, "accv[l]", "(" + ACC + ")" + val) << ";\n    }\n    };\n";
+    if (rounds >= B && B > 0)
+      o << "#pragma unroll 1\n    for (int b = 0; b < " << rounds / B << "; ++b) {\n#pragma unroll\n      for (int u = 0; u < " << B << "; ++u) add((b * " << B << " + u) * " << CY << " + cy);\n    }\n";
+    if (B > 0 && rounds % B) o << "#pragma unroll\n    for (int u = " << rounds / B * B << "; u < " << rounds << "; ++u) add(u * " << CY << " + cy);\n";
+    if (len % CY) o << "    if (cy < " << len % CY << ") add(" << rounds * CY << " + cy);\n";
     o << "#pragma unroll\n    for (int l = 0; l < " << VEC << "; ++l) part[cy][cx * " << VEC << " + l] = accv[l];\n  }\n  __syncthreads();\n";
     o << "  const int c = threadIdx.x % " << NC << ", q = threadIdx.x / " << NC << ";\n";
-    o << "  {\n    " << ACC << " a = part[q * " << PER << "][c];\n#pragma unroll\n    for (int y = 1; y < " << PER << "; ++y) a = "
+    o << "  if (q < " << NG << ") {\n    " << ACC << " a = part[q * " << PER << "][c];\n#pragma unroll\n    for (int y = 1; y < " << PER << "; ++y) a = "
       << red_apply(rn.red, dt, "a", "part[q * " + std::to_string(PER) + " + y][c]") << ";\n    sums[q][c] = a;\n  }\n  __syncthreads();\n";
     o << "  const " << it << " oid = (" << it << ")blockIdx.x * " << NC << " + c;\n";
     o << "  if (threadIdx.x >= " << NC << " || oid >= " << nout << ") return;\n";
@@ -4664,7 +4698,7 @@ struct Planner {
     L.kernel = named("@K@_reduce_generic", finalize(o.str()));
     L.kind = "reduce_generic";
     L.grid[0] = (unsigned)((nvec + CX - 1) / CX);
-    L.block[0] = kBlock;
+    L.block[0] = BLK;
     L.shared_bytes = shared;
     for (int i : em.inputs) L.args.push_back(buffer_for(i));
     L.args.push_back(buffer_for(root));
@@ -4672,6 +4706,7 @@ struct Planner {
     L.desc = describe(rn.in[0]) + " reduce";
     plan.launches.push_back(L);
   }
+  // generic reduction: one thread per output element, sequential loops over reduced dims
   void emit_reduce_generic(int root) {
     const Node& rn = g.nodes[root];
     const Node& inn = g.nodes[rn.in[0]];
@@ -4780,14 +4815,14 @@ struct Planner {
     const int64_t chunk = two_pass ? (inn.ty.dims[red[ks]] + split - 1) / split : 0;
     if (two_pass) split = (inn.ty.dims[red[ks]] + chunk - 1) / chunk;
     // One launch where the second one would cost more than it spares: a workgroup takes CX vectors of outputs, its threads
-    // every CY-th row of them (64 bytes of a row and 64 rows at a time), and adds the threads' sums through LDS in a fixed
-    // order.  A chain of additions is no longer than that of the chunks (a chunk, the partials of a wavefront, four of those).
-    // Kernels, us, two launches -> one: 1024 x 2048 bf16 4.3 + 4.0 -> 4.0, 1024 x 1000 4.8 + 4.4 -> 4.8, 4096 x 2048 7.4 + 4.2 -> 7.4; f32 1024^2 4.6 + 4.6 -> 5.0, 4096 x 960 4.6 + 5.8 -> 7.2; f64 1024^2 4.4 + 4.1 -> 4.1.
-    constexpr int CX = 4, CY = kBlock / CX;
-    const bool columns = two_pass && RB == 1 && VEC > 1 && red.size() == 1 && opt.column_reduce && red_len <= 4096 && inn.ty.numel() * esz <= (int64_t)16 << 20;
+    // every CY-th row of them (64 bytes of a row and 64 or 256 rows at a time), and adds the threads' sums through LDS in a
+    // fixed order.  A chain of additions is no longer than that of the chunks (a chunk, the partials of a wavefront, four of
+    // those): at most 64 rows, the sums of two to sixteen threads, 8 to 32 of those.
+    const bool beside = std::any_of(g.nodes.begin(), g.nodes.end(), [](const Node& x) { return x.k == OpK::DotGeneral; });
+    const int CX = 4, CY = (red_len > 1024 && !beside ? 1024 : kBlock) / CX;
+    const bool columns = two_pass && RB == 1 && VEC > 1 && red.size() == 1 && opt.column_reduce && red_len <= column_rows(rn.in[0], beside) && inn.ty.numel() * esz <= (int64_t)16 << 20;
     if (columns) {
-      const int NC = CX * VEC, NG = kBlock / NC, PER = CY / NG;   // outputs of a workgroup, groups of threads that add them, rows of sums per group
-      emit_reduce_columns(root, eu, kept, red[0], nout, VEC, NC, NG, PER, CX, CY, body, val, ibody, initv);
+      emit_reduce_columns(root, eu, kept, red[0], nout, VEC, CX, CY, body, val, ibody, initv);
       return;
     }
     std::ostringstream o;
