@@ -266,7 +266,7 @@ rx::PlanOptions plan_options() {
   if (const char* e = getenv("RX_COLUMN_REDUCE")) o.column_reduce = atoi(e) != 0;
   if (const char* e = getenv("RX_FOLD_FINALS")) o.fold_finals = atoi(e) != 0;
   if (const char* e = getenv("RX_JOIN_LAUNCHES")) o.join_launches = atoi(e) != 0;
-  if (const char* e = getenv("RX_CONV_SPLIT")) o.split_convs = atoi(e) != 0;
+  if (const char* e = getenv("RX_CONV_SPLIT")) o.split_convs = atoi(e) != 0 ? rx::kSplitShared : rx::kSplitNever;
   if (const char* e = getenv("RX_IN_PLACE")) o.in_place_updates = atoi(e) != 0;
   if (const char* e = getenv("RX_CHAIN_STEPS")) o.chain_steps = atoi(e);
   if (const char* e = getenv("RX_CHAIN_TILE")) { int v[3] = {0, 0, 0}; if (sscanf(e, "%d,%d,%d", &v[0], &v[1], &v[2]) >= 1) { o.chain_tile[0] = v[0]; o.chain_tile[1] = v[1]; o.chain_tile[2] = v[2]; } }
@@ -854,10 +854,14 @@ namespace {
 // Split filters are temporaries: a module that RxExecuteNoAlloc holds without them is planned without them.
 rx::Plan plan_module(const char* text, size_t len, rx::PlanOptions opt) {
   rx::Plan p = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
+  if (p.split_filters == 1) {   // the launch that splits filters is this one's alone
+    opt.split_convs = rx::kSplitAlone;
+    p = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
+  }
   const char* force = getenv("RX_CONV_SPLIT");
   if (p.split_filters > 0 && !(force && atoi(force) == 2) && p.temporary_bytes() > (int64_t)RX_NOALLOC_SCRATCH_BYTES) {
-    opt.split_convs = false;
-    rx::Plan plain = rx::make_plan(rx::parse_module(text, len, false), opt);
+    opt.split_convs = rx::kSplitNever;
+    rx::Plan plain = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
     if (plain.temporary_bytes() <= (int64_t)RX_NOALLOC_SCRATCH_BYTES) return plain;
   }
   return p;

@@ -645,7 +645,8 @@ ConvSplitChoice choose_conv_split(int64_t B, int64_t C, int64_t H, int64_t W, in
   return best;
 }
 
-bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl, int64_t sh, int64_t sw, int64_t dh, int64_t dw) {
+bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl, int64_t sh, int64_t sw, int64_t dh, int64_t dw,
+                     bool alone) {
   if (getenv("RX_CONV_DIRECT") && atoi(getenv("RX_CONV_DIRECT")) == 0) return false;
   const char* force = getenv("RX_CONV_SPLIT");   // 0: never; 2: wherever the kernel covers the case
   if (force && atoi(force) == 0) return false;
@@ -658,7 +659,17 @@ bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int6
   // VGG-11): 8 images of 14 x 14, 512 -> 512: 112 -> 54 + 14; 4 of 28 x 28, 256 -> 256: 53 -> 29 + 11; 8 of 56 x 56, 64 -> 128:
   // 43 -> 23 + 9; 2 of 32 x 32, 64 -> 128: 11.3 -> 6.3 + 6.7; against the product: 4 of 14 x 14, 512 -> 512: 60 -> 34 + 15; one:
   // 21 -> 18 + 14; 8 x 8: 15 -> 14 + 13; 2 of 10 x 10, 160 -> 160: 15 -> 7 + 8.  The product's estimate is a quarter too high.
-  return c.us < (d.ok ? d.us : 0.8 * product);
+  double share = 1.0;
+  if (alone) {
+    // 126 convolutions alone in their modules, 1 to 16 images of 5 x 5 to 64 x 64, 32 to 512 channels: below these shares of the
+    // estimates none took longer than before (0.14 to 1.00 of it), above them they took 0.7 to 1.5 of it.  The f32 kernel's
+    // estimate is low where its last group of 64 features is not whole, and for 25 taps.  us per call, before -> split: 4 of
+    // 41 x 36, 64 -> 192, stride 2: 12 -> 16; 4 of 18 x 44, 64 -> 384, 1 x 1: 6.7 -> 10; 16 of 50 x 27, 32 -> 128: 26 -> 30.
+    const int64_t taps = KH * KW;
+    if (d.ok) share = O % 64 != 0 || taps > 9 ? 1.0 : taps == 1 ? 0.7 : 0.82;
+    else if (taps > 1) share = 0.68;
+  }
+  return c.us < share * (d.ok ? d.us : 0.8 * product);
 }
 
 }  // namespace rx

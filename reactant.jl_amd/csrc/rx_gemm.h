@@ -78,7 +78,7 @@ struct ConvSplitChoice {
 };
 ConvSplitChoice choose_conv_split(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO,
                                   int64_t sh, int64_t sw, int64_t dh, int64_t dw);
-// Is that kernel the faster one?  `pl`: zero columns before the image.
-bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl, int64_t sh, int64_t sw, int64_t dh, int64_t dw);
+// Is that kernel the faster one?  `pl`: zero columns before the image; `alone`: no other filter shares the splitting launch.
+bool conv_split_pays(int64_t B, int64_t C, int64_t H, int64_t W, int64_t O, int64_t KH, int64_t KW, int64_t HO, int64_t WO, int64_t pl, int64_t sh, int64_t sw, int64_t dh, int64_t dw, bool alone);
 
 }  // namespace rx

@@ -109,8 +109,11 @@ struct Graph {
   }
 };
 
+// f32 convolutions on split operands: never; where the launch that splits their filters is shared with others; where it is one's alone
+enum SplitConvs { kSplitNever, kSplitShared, kSplitAlone };
+
 // Parse a module; functions called from @main are inlined.  Throws rx::Error.  `split_convs`: PlanOptions::split_convs.
-Graph parse_module(const char* text, size_t len, bool split_convs = true);
+Graph parse_module(const char* text, size_t len, SplitConvs split_convs = kSplitShared);
 
 // Constant payload helpers
 double splat_as_double(const Node& n);

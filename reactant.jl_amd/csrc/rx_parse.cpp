@@ -1065,7 +1065,7 @@ void fill_constant(Node& n, const std::string& payload_in, const std::function<v
 struct Builder {
   P& p;
   Graph g;
-  bool split_convs = true;
+  SplitConvs split_convs = kSplitShared;
   explicit Builder(P& pp) : p(pp) {}
   [[noreturn]] static void fail(const std::string& m) { throw Error("StableHLO import: " + m); }
 
@@ -1949,7 +1949,7 @@ struct Builder {
       const int64_t eh = xct.dims[2] + pad[0] + pad[1] - ((KH - 1) * rd[0] + 1), ew = xct.dims[3] + pad[2] + pad[3] - ((KW - 1) * rd[1] + 1);
       const int64_t HO = eh >= 0 ? eh / st[0] + 1 : 0, WO = ew >= 0 ? ew / st[1] + 1 : 0;
       if (HO >= 1 && WO >= 1 && (choose_conv(B, C, xct.dims[2], xct.dims[3], O, KH, KW, HO, WO, pad[2], st[0], st[1], rd[0], rd[1]).ok ||
-                                 (split_convs && xct.dt == DT::F32 && conv_split_pays(B, C, xct.dims[2], xct.dims[3], O, KH, KW, HO, WO, pad[2], st[0], st[1], rd[0], rd[1])))) {
+                                 (split_convs && xct.dt == DT::F32 && conv_split_pays(B, C, xct.dims[2], xct.dims[3], O, KH, KW, HO, WO, pad[2], st[0], st[1], rd[0], rd[1], split_convs == kSplitAlone)))) {
         std::vector<int64_t> want(r);
         want[cd[2].d0] = B; want[cd[2].d1] = O; want[cd[2].sp[0]] = HO; want[cd[2].sp[1]] = WO;
         if (want != out.dims) fail("convolution: result shape mismatch");
@@ -2632,7 +2632,7 @@ struct Builder {
 
 }  // namespace
 
-Graph parse_module(const char* text, size_t len, bool split_convs) {
+Graph parse_module(const char* text, size_t len, SplitConvs split_convs) {
   P p(text, len);
   p.parse();
   const RawFunc* mainf = nullptr;

@@ -4164,7 +4164,7 @@ struct Planner {
     ConvChoice cc;
     ConvSplitChoice cx;
     if (!shifted && opt.split_convs && conv_split_pays(xt.dims[0], xt.dims[1], xt.dims[2], xt.dims[3], wt.dims[0], wt.dims[2], wt.dims[3], cn.ty.dims[2], cn.ty.dims[3],
-                                                       cn.a0[2], cn.a1[0], cn.a1[1], cn.a2[0], cn.a2[1]))
+                                                       cn.a0[2], cn.a1[0], cn.a1[1], cn.a2[0], cn.a2[1], opt.split_convs == kSplitAlone))
       cx = choose_conv_split(xt.dims[0], xt.dims[1], xt.dims[2], xt.dims[3], wt.dims[0], wt.dims[2], wt.dims[3], cn.ty.dims[2], cn.ty.dims[3], cn.a1[0], cn.a1[1],
                              cn.a2[0], cn.a2[1]);
     if (!shifted && !cx.ok) {

@@ -68,7 +68,7 @@ struct PlanOptions {
   bool join_launches = true;    // small launches that do not depend on one another run as one
   bool nhwc_regions = true;     // the same for regions with several readers per value (residual additions): transposed once on the way in and out where needed
   double nhwc_region_ratio = 1.5;   // a region is rebuilt when the transposes that disappear move this many times the bytes of those that are added (two residual blocks: 3 against 2 tensors, 0.129 -> 0.115 ms)
-  bool split_convs = true;      // f32 convolutions of many channels on the bf16 matrix cores, operands split in three
+  SplitConvs split_convs = kSplitShared;   // f32 convolutions of many channels on the bf16 matrix cores, operands split in three
   bool pad_into_pools = true;   // zero padding of a pooled value (windows that do not overlap) moves onto the pooling's operand: no padding map
   bool epilogue_init = true;    // a bias added to a product on the streaming skeletons becomes the accumulators' first values
   bool row_fusion = true;       // fuse row reductions with their elementwise consumers

@@ -77,3 +77,24 @@ def test_plans(monkeypatch):
     assert kinds(conv(8, 512, 512, 14)) == ["filter_split", "conv"]
     monkeypatch.setenv("RX_CONV_SPLIT", "0")
     assert kinds(conv(8, 64, 128, 56)) == ["conv"]
+
+
+@pytest.mark.parametrize("xs,ws,stride,alone", [([4, 64, 41, 36], [192, 64, 3, 3], 2, False), ([4, 64, 18, 44], [384, 64, 1, 1], 1, False), ([16, 32, 50, 27], [128, 32, 3, 3], 1, False),
+                                                ([2, 64, 28, 26], [72, 64, 5, 5], 2, True), ([4, 64, 36, 27], [128, 64, 1, 1], 1, True)])
+def test_a_convolution_alone_pays_for_the_splitting_launch(xs, ws, stride, alone):
+    """Several convolutions share the launch that splits their filters: those stay on split operands."""
+    rx = load_pkg()
+    pad = ws[2] // 2
+    text, _ = NN.convolution(xs, ws, "f32", strides=[stride, stride], padding=[[pad, pad], [pad, pad]])
+    assert ("filter_split" in rx.compile_offline(text)) == alone
+    # the same operation twice, on other operands
+    op = next(l for l in text.splitlines() if "stablehlo.convolution" in l)
+    name, rest = op.split("=", 1)
+    head, tail = text[text.index("@main(") + 6:].split(")", 1)
+    xt, wt = [a.split(":", 1)[1].strip() for a in head.split("%")[1:]]
+    out = tail[tail.index("->") + 2:tail.index("{")].strip()
+    two = rest.replace("%arg0", "%arg2").replace("%arg1", "%arg3")
+    assert two != rest
+    text = ("module {\n  func.func @main(%%arg0: %s, %%arg1: %s, %%arg2: %s, %%arg3: %s) -> (%s, %s) {\n%s\n    %%second =%s\n    return %s, %%second : %s, %s\n  }\n}\n"
+            % (xt.rstrip(","), wt, xt.rstrip(","), wt, out, out, op, two, name.strip(), out, out))
+    assert "filter_split" in rx.compile_offline(text)
