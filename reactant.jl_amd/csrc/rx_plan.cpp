@@ -4417,7 +4417,8 @@ struct Planner {
   // one: f32 4099 elements 8.2 and 3.9, 8192 8.2 and 4.0, 32768 8.1 and 6.9, 65536 8.1 and 12; f64 4096 8.3 and 3.9, 8192 8.4
   // and 5.4, 16384 7.9 and 9.1.  A thread adds at most eight elements, as it does in the two-launch form.  Several
   // transcendental functions per element: fewer elements, and so for f64 functions of many instructions (us per call, two
-  // launches and one: tanh of 4096 elements 8.7 and 6.3, 8192 8.9 and 10.8; power 8.6 and 7.3, 8.5 and 12.7; log_plus_one 8.7 and 6.0, 8.7 and 9.1).
+  // launches and one: tanh of 4096 elements 8.7 and 6.3, 8192 8.9 and 10.8; power 8.6 and 7.3, 8.5 and 12.7; log_plus_one 8.7 and 6.0, 8.7 and 9.1; lgamma of 2048 elements 8.5
+  // and 13.7, erf_inv 9.5 and 20.2: those up to 1024, one element a thread).
   // `tail`: the reduction itself, or the elementwise root that is its only reader: evaluated by the thread that stores.
   void emit_reduce_full(int root, int tail) {
     const Node& rn = g.nodes[root];
@@ -4431,15 +4432,16 @@ struct Planner {
     const int64_t nv = inn.ty.numel() / vec;
     const int U = 4;
     int64_t slow_ops = 0;
-    bool dear = false;
+    int64_t dear = 0;
     for (int x : cone_nodes(rn.in[0])) {
       const Node& c = g.nodes[x];
-      slow_ops += c.k == OpK::Unary || c.k == OpK::Gelu || c.op == "power" || c.op == "atan2";
+      const bool special = c.k == OpK::Unary && (c.op == "lgamma" || c.op == "digamma" || c.op == "erf_inv");
+      slow_ops += special ? 2 : c.k == OpK::Unary || c.k == OpK::Gelu || c.op == "power" || c.op == "atan2";
       static const std::set<std::string> cheap = {"sine", "cosine", "tan", "exponential", "exponential_minus_one", "log", "logistic", "sqrt", "rsqrt", "cbrt", "abs", "negate", "sign", "floor", "ceil",
                                                   "round_nearest_even", "round_nearest_afz", "is_finite"};
-      dear = dear || (c.ty.dt == DT::F64 && (c.k == OpK::Gelu || (c.k == OpK::Unary && !cheap.count(c.op)) || c.op == "power"));
+      if (c.ty.dt == DT::F64 && (c.k == OpK::Gelu || (c.k == OpK::Unary && !cheap.count(c.op)) || c.op == "power")) dear += special ? 4 : 1;
     }
-    const bool one = n > 0 && inn.ty.numel() * std::max<int64_t>(1, slow_ops) <= opt.one_workgroup_reduce && !(dear && inn.ty.numel() > opt.one_workgroup_reduce / 2);
+    const bool one = n > 0 && inn.ty.numel() * std::max<int64_t>(1, slow_ops) <= opt.one_workgroup_reduce && inn.ty.numel() * dear <= opt.one_workgroup_reduce / 2;
     const int BLK = one ? 1024 : kBlock;
     int64_t tiles = (nv + (int64_t)kBlock * U - 1) / ((int64_t)kBlock * U);
     const int G = one ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(tiles, 2048));

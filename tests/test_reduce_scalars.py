@@ -70,9 +70,9 @@ def test_reductions_of_some_dimensions(rx, client, shape, dim, dt):
     assert np.array_equal(np.asarray(got[0].a), np.asarray(oracle_run(text, args, hifi=True)[0].a))
 
 
-@pytest.mark.parametrize("op,n,dt,launches", [("tanh", 4096, "f64", 1), ("tanh", 4097, "f64", 2), ("log_plus_one", 8192, "f64", 2), ("sine", 8192, "f64", 1), ("tanh", 8192, "f32", 1)])
+@pytest.mark.parametrize("op,n,dt,launches", [("tanh", 4096, "f64", 1), ("tanh", 4097, "f64", 2), ("log_plus_one", 8192, "f64", 2), ("sine", 8192, "f64", 1), ("tanh", 8192, "f32", 1), ("lgamma", 1024, "f64", 1), ("lgamma", 1025, "f64", 2), ("digamma", 4097, "f32", 2)])
 def test_one_workgroup_or_two_launches(op, n, dt, launches):
-    text = ("module {\n  func.func @main(%a: T) -> S {\n    %z = stablehlo.constant dense<0.0> : S\n    %m = stablehlo.OP %a : T\n"
-            "    %r = stablehlo.reduce(%m init: %z) applies stablehlo.add across dimensions = [0] : (T, S) -> S\n    return %r : S\n  }\n}\n").replace("OP", op)
+    text = ("module {\n  func.func @main(%a: T) -> S {\n    %z = stablehlo.constant dense<0.0> : S\n    %m = OP\n"
+            "    %r = stablehlo.reduce(%m init: %z) applies stablehlo.add across dimensions = [0] : (T, S) -> S\n    return %r : S\n  }\n}\n").replace("OP", "chlo.%s %%a : T -> T" % op if op in ("lgamma", "digamma") else "stablehlo.%s %%a : T" % op)
     report = rx.compile_offline(text.replace("T", "tensor<%dx%s>" % (n, dt)).replace("S", "tensor<%s>" % dt))
     assert report.count("kind=") == launches, report
