@@ -3278,8 +3278,8 @@ struct Planner {
   // unit one workgroup; larger arrays (but for those further down) stay maps, which move them from L2 with less arithmetic (116 x 116 x 70 f64: the best
   // chain of those tiles 87 us for 10 steps, maps 100; 171 x 100 x 29: 48 and 45; 206 x 106 x 106: 196 and 230).  Fitted to 51 (f64) and 26 (f32)
   // timings of 8 to 10 advection-diffusion steps on 36 x 36 x 26 to 165 x 100 x 29 points, tiles of 6 x 6 x 12 to 10 x 10 x 32 and
-  // 2 to 4 steps (9 and 8 % rms): rounds are of a workgroup over its cells, MB what all of them stage.  A map per step takes
-  // 4.4 us.  10 steps, us, tiles of 8 x 8 x 16 and two steps (f32: four) before -> as chosen: 67 x 53 x 39 f64 32.2 -> 26.2,
+  // 2 to 4 steps (9 and 8 % rms): rounds are of a workgroup over its cells, MB what all of them stage.  A map per step
+  // is counted as 4.4 us (rows of odd length: below).  10 steps, us, tiles of 8 x 8 x 16 and two steps (f32: four) before -> as chosen: 67 x 53 x 39 f64 32.2 -> 26.2,
   // f32 20 -> 17.5; 36 x 36 x 26 f64 28.7 -> 17.7.
   // (Runs of up to three steps are left as they are, and so are steps that update several arrays in turns.)
   // how many further arrays (0: the choice above is not for these steps)
@@ -3306,7 +3306,10 @@ struct Planner {
     const size_t cap = 5;
     double cost[6];
     int64_t tile[6][3] = {};
-    cost[1] = 4.4;
+    // Maps over rows of odd length, whose threads take one element each, are faster (3.2 us per step up to 570 000 cells, f64 3.4
+    // to 4.4), and are left only for a chain that the estimate has well ahead of them: 4 to 16 steps, maps -> the chain that
+    // 4.4 us chose, us: f32 111 x 74 x 60 51 -> 61, 93 x 115 x 65 17.9 -> 20.0, 115 x 88 x 56 55 -> 61, f64 71 x 88 x 45 17.2 -> 22.0.
+    cost[1] = D[2] % 2 == 0 ? 4.4 : es == 8 ? 3.3 : 2.9;
     for (size_t k = 2; k <= cap; ++k) {
       cost[k] = 1e30;
       for (int64_t a : {4, 5, 6, 8, 10})
