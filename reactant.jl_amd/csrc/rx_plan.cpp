@@ -3493,7 +3493,7 @@ struct Planner {
         }
         cur[writes[i]] = x;
       }
-      if (!ok) continue;
+      if (!ok || lds_bytes + 2 * margin * es > 160 * 1024) continue;   // (a chosen tile is bounded without the cells around it)
 
       std::ostringstream o;
       const std::string kname = "@K@_chain";
