@@ -1708,11 +1708,12 @@ struct Planner {
     src << text;
   }
 
-  // The second launch of a full reduction of 64 to 512 partials (fewer: the launches that the planner's tests of the benchmark
-  // programs state, not the time) runs in the map that reads its result (an absmax and the
+  // The second launch of a full reduction of 64 to 512 partials runs in the map that reads its result (an absmax and the
   // quantization): every workgroup of the map adds the partials in the same order, the first one also stores the
   // result for other readers.  A launch less for about a microsecond in a map of up to 2048 workgroups: e4m3 layers of 200 x 4096 x
-  // 6144 23.4 -> 22.4 us, 500 x 8192 x 4096 51.4 -> 50.0, 2000 x 1024 x 4096 32.5 -> 31.3.
+  // 6144 23.4 -> 22.4 us, 500 x 8192 x 4096 51.4 -> 50.0, 2000 x 1024 x 4096 32.5 -> 31.3; x / max |x| of 128 x 4096 f32 11.4 -> 8.7 per
+  // call.  Below 64 partials it gains as much (16 x 4096, 16 partials: 11.3 -> 8.2); the bound is there for the launches that
+  // the planner's tests of the benchmark programs state.
   void fold_finals() {
     if (!opt.fold_finals) return;
     std::set<std::string> gone;
