@@ -155,7 +155,8 @@ void RxExecuteProfiled(RxExecutable *exec, int num_args, RxBuffer **op_args, RxD
 int RxExecutableTakeTimings(RxExecutable *exec, double *launch_ms_sum);
 /* No counterpart in the reference.  For callers that cannot allocate device memory while they run
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the launch
- * list of `exec`, like XLAExecuteSharded, but the caller passes the result buffers too (existing
+ * list of `exec` (or of a second plan of the same module that needs less memory, compiled with it), like
+ * XLAExecuteSharded, but the caller passes the result buffers too (existing
  * buffers of the executable's result types, distinct from the arguments and from each other; they
  * are overwritten), and every temporary of the plan (partial results of the two-pass reductions,
  * tensors handed from one kernel to the next) lives in a static device array of

@@ -213,10 +213,16 @@ struct RxExecutable {
   std::vector<Mem> consts;          // per plan buffer (only Const kinds are set)
   std::string report;
   std::string text;                 // the module as compiled: a rebuild after a failed wait starts from it
+  std::unique_ptr<RxExecutable> small;   // the module in a plan whose temporaries fit RxExecuteNoAlloc, where `plan`'s do not
   bool waits = false;               // some kernel of the plan waits for other workgroups of its launch (has a fault-word argument)
   std::mutex mu;
   // event lists of executions profiled without blocking (RxExecuteProfiled), oldest first
   std::vector<std::vector<hipEvent_t>> pending_events;
+  void unload() {                   // (no kernel of the module is queued any more)
+    if (module) { (void)hipModuleUnload(module); module = nullptr; }
+    if (small) small->unload();
+    small.reset();
+  }
 };
 
 namespace {
@@ -851,18 +857,26 @@ RX_EXPORT void PjRtBufferFree(RxBuffer* b) {
 }
 
 namespace {
-// Split filters are temporaries: a module that RxExecuteNoAlloc holds without them is planned without them.
+// The plan of a module.  Filters split in three and the partial results of column sums are temporaries: a module that
+// RxExecuteNoAlloc holds without them is planned without them.
 rx::Plan plan_module(const char* text, size_t len, rx::PlanOptions opt) {
-  rx::Plan p = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
+  auto planned = [&]() { return rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt); };
+  auto fits = [](const rx::Plan& p) { return p.temporary_bytes() <= (int64_t)RX_NOALLOC_SCRATCH_BYTES; };
+  rx::Plan p = planned();
   if (p.split_filters == 1) {   // the launch that splits filters is this one's alone
     opt.split_convs = rx::kSplitAlone;
-    p = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
+    p = planned();
   }
+  if (fits(p)) return p;
   const char* force = getenv("RX_CONV_SPLIT");
-  if (p.split_filters > 0 && !(force && atoi(force) == 2) && p.temporary_bytes() > (int64_t)RX_NOALLOC_SCRATCH_BYTES) {
-    opt.split_convs = rx::kSplitNever;
-    rx::Plan plain = rx::make_plan(rx::parse_module(text, len, opt.split_convs), opt);
-    if (plain.temporary_bytes() <= (int64_t)RX_NOALLOC_SCRATCH_BYTES) return plain;
+  const bool split = p.split_filters > 0 && !(force && atoi(force) == 2);
+  const rx::SplitConvs with = opt.split_convs;
+  for (int k = 1; k < 4; ++k) {   // without split filters, without chunks of columns, without either
+    if (((k & 1) && !split) || ((k & 2) && !p.chunked_columns)) continue;
+    opt.split_convs = k & 1 ? rx::kSplitNever : with;
+    opt.column_sums_whole = (k & 2) != 0;
+    rx::Plan q = planned();
+    if (fits(q)) return q;
   }
   return p;
 }
@@ -929,6 +943,17 @@ void load_plan(RxExecutable* ex, rx::PlanOptions opt) {
     if (!B.data.empty()) HIP_CHECK(hipMemcpyAsync(ex->consts[b]->ptr, B.data.data(), B.data.size(), hipMemcpyHostToDevice, d->stream));
   }
   HIP_CHECK(hipStreamSynchronize(d->stream));   // pageable host data: wait before the plan may move
+  // Steps that run as maps keep more arrays than their chain, with the same results: RxExecuteNoAlloc runs the chain where
+  // that is what its memory holds.
+  if (!opt.chains_first && ex->plan.unchained_steps && ex->plan.temporary_bytes() > (int64_t)RX_NOALLOC_SCRATCH_BYTES) {
+    opt.chains_first = true;
+    if (plan_module(ex->text.data(), ex->text.size(), opt).temporary_bytes() > (int64_t)RX_NOALLOC_SCRATCH_BYTES) return;
+    ex->small.reset(new RxExecutable);
+    ex->small->client = ex->client;
+    ex->small->device = d;
+    ex->small->text = ex->text;
+    load_plan(ex->small.get(), opt);
+  }
 }
 
 // After a wait between workgroups has expired on the device (check_fault), an executable whose kernels wait is rebuilt
@@ -937,7 +962,7 @@ void rebuild_without_waits(RxExecutable* ex) {
   if (!ex->waits || !ex->device->waits_failed) return;
   HIP_CHECK(hipSetDevice(ex->device->ordinal));
   HIP_CHECK(hipStreamSynchronize(ex->device->stream));   // kernels of the old module may still be queued
-  if (ex->module) { (void)hipModuleUnload(ex->module); ex->module = nullptr; }
+  ex->unload();
   for (auto& evs : ex->pending_events)   // timings of the old plan's launches
     for (auto& e : evs) (void)hipEventDestroy(e);
   ex->pending_events.clear();
@@ -969,7 +994,7 @@ RX_EXPORT void ExecutableFree(RxExecutable* ex) {
   if (ex->module) {
     (void)hipSetDevice(ex->device->ordinal);
     (void)hipStreamSynchronize(ex->device->stream);
-    (void)hipModuleUnload(ex->module);
+    ex->unload();
   }
   for (auto& evs : ex->pending_events)
     for (auto& e : evs) (void)hipEventDestroy(e);
@@ -1069,6 +1094,7 @@ RX_EXPORT int RxExecuteNoAlloc(RxExecutable* ex, int num_args, RxBuffer** args, 
     check_exec(ex);
     RxDevice* dev = ex->device;
     std::lock_guard<std::mutex> lock(ex->mu);
+    if (ex->small) ex = ex->small.get();   // (under the same lock)
     if (ex->waits && dev->waits_failed)
       throw Error("FAILED_PRECONDITION: a wait between workgroups expired on this device earlier; this executable has to be rebuilt in the form "
                   "that does not wait, which allocates: execute it once through XLAExecuteSharded");

@@ -3310,7 +3310,7 @@ struct Planner {
     // Maps over rows of odd length, whose threads take one element each, are faster (3.2 us per step up to 570 000 cells, f64 3.4
     // to 4.4), and are left only for a chain that the estimate has well ahead of them: 4 to 16 steps, maps -> the chain that
     // 4.4 us chose, us: f32 111 x 74 x 60 51 -> 61, 93 x 115 x 65 17.9 -> 20.0, 115 x 88 x 56 55 -> 61, f64 71 x 88 x 45 17.2 -> 22.0.
-    cost[1] = D[2] % 2 == 0 ? 4.4 : es == 8 ? 3.3 : 2.9;
+    cost[1] = D[2] % 2 == 0 || opt.chains_first ? 4.4 : es == 8 ? 3.3 : 2.9;
     for (size_t k = 2; k <= cap; ++k) {
       cost[k] = 1e30;
       for (int64_t a : {4, 5, 6, 8, 10})
@@ -3390,6 +3390,7 @@ struct Planner {
     const bool chosen = others > 0;
     if (chosen) {
       longest = (size_t)choose_chain3(steps.size(), D.data(), es, others, T);
+      plan.unchained_steps = plan.unchained_steps || (D[2] % 2 != 0 && !opt.chains_first);
       if (longest < 2) return 0;
     }
     for (size_t k = longest; k >= 2; --k) {
@@ -4834,7 +4835,9 @@ struct Planner {
     // those): at most 64 rows, the sums of two to sixteen threads, 8 to 32 of those.
     const bool beside = std::any_of(g.nodes.begin(), g.nodes.end(), [](const Node& x) { return x.k == OpK::DotGeneral; });
     const int CX = 4, CY = (red_len > 1024 && !beside ? 1024 : kBlock) / CX;
-    const bool columns = two_pass && RB == 1 && VEC > 1 && red.size() == 1 && opt.column_reduce && red_len <= column_rows(rn.in[0], beside) && inn.ty.numel() * esz <= (int64_t)16 << 20;
+    const bool can = two_pass && RB == 1 && VEC > 1 && red.size() == 1 && opt.column_reduce && red_len <= 4096 && inn.ty.numel() * esz <= (int64_t)16 << 20;
+    const bool columns = can && (opt.column_sums_whole || red_len <= column_rows(rn.in[0], beside));
+    plan.chunked_columns = plan.chunked_columns || (can && !columns);
     if (columns) {
       emit_reduce_columns(root, eu, kept, red[0], nout, VEC, CX, CY, body, val, ibody, initv);
       return;

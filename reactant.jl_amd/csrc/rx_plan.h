@@ -47,6 +47,8 @@ struct Plan {
   double hlo_operand_bytes[2] = {0, 0};
   std::string report() const;          // text summary for debugging
   int split_filters = 0;               // temporaries that hold a filter split in three
+  bool chunked_columns = false;        // column sums that would take no temporaries in one launch take two
+  bool unchained_steps = false;        // steps whose chain would keep fewer arrays run as maps
   int64_t temporary_bytes() const;     // what its temporaries take when each has memory of its own (RxExecuteNoAlloc)
 };
 
@@ -65,6 +67,8 @@ struct PlanOptions {
   bool merge_parameter_maps = true;  // plain maps that read only the module's arguments run first, several of them as one launch
   bool fold_finals = true;      // the end of a full reduction runs in the map that reads its result
   bool column_reduce = true;    // column sums of matrices of up to 16 MB in one launch
+  bool column_sums_whole = false;  // ... of up to 4096 rows, whatever their elements cost
+  bool chains_first = false;    // rank-3 steps over rows of odd length as over others: chains where their estimate is below 4.4 us per step
   bool join_launches = true;    // small launches that do not depend on one another run as one
   bool nhwc_regions = true;     // the same for regions with several readers per value (residual additions): transposed once on the way in and out where needed
   double nhwc_region_ratio = 1.5;   // a region is rebuilt when the transposes that disappear move this many times the bytes of those that are added (two residual blocks: 3 against 2 tensors, 0.129 -> 0.115 ms)

@@ -34,6 +34,16 @@ def test_launches(rows, dt, ops, product, launches, block):
     assert block is None or " part[%d][" % (block // 4) in report, report[:2000]     # threads' sums, four vectors of outputs side by side
 
 
+@pytest.mark.parametrize("n,launches", [(2, 2), (3, 1)])
+def test_partial_results_stay_within_what_a_call_without_allocations_holds(n, launches):
+    """1.9 MB of partial results per sum, 4 MiB for all"""
+    t, o = "tensor<4096x2000xbf16>", "tensor<2000xbf16>"
+    lines = ["%%m%d = stablehlo.tanh %%a%d : %s\n    %%r%d = stablehlo.reduce(%%m%d init: %%z) applies stablehlo.add across dimensions = [0] : (%s, tensor<bf16>) -> %s" % (i, i, t, i, i, t, o) for i in range(n)]
+    text = ("module {\n  func.func @main(%s) -> (%s) {\n    %%z = stablehlo.constant dense<0.0> : tensor<bf16>\n    %s\n    return %s : %s\n  }\n}\n"
+            % (", ".join("%%a%d: %s" % (i, t) for i in range(n)), ", ".join([o] * n), "\n    ".join(lines), ", ".join("%%r%d" % i for i in range(n)), ", ".join([o] * n)))
+    assert ("combine partials" in rx.compile_offline(text)) == (launches == 2)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", ["f32", "f64", "bf16", "i32"])
 @pytest.mark.parametrize("rows", [65, 127, 640, 1021, 1024, 1025, 1279, 1280, 3333, 4095, 4096])
